@@ -90,6 +90,38 @@ struct Flow {
 };
 constexpr unsigned kFlowSpinLimit = 1u << 23;  // polls per wait (seconds)
 
+// The bits of T, for relaxed agent-scope atomic accesses: such a load reads
+// past the caches of this XCD, such a store writes through them.
+template <typename T> struct BitsOf;
+template <> struct BitsOf<double> { using type = unsigned long long; };
+template <> struct BitsOf<float> { using type = unsigned int; };
+template <typename T>
+__device__ __forceinline__ T load_agent(const T* p) {
+  using B = typename BitsOf<T>::type;
+  return __builtin_bit_cast(
+      T, __hip_atomic_load(reinterpret_cast<const B*>(p), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT));
+}
+template <typename T>
+__device__ __forceinline__ void store_agent(T* p, T v) {
+  using B = typename BitsOf<T>::type;
+  __hip_atomic_store(reinterpret_cast<B*>(p), __builtin_bit_cast(B, v),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// lane l's value, to every lane (v_readlane: a few cycles, where a
+// ds_bpermute shuffle takes an LDS round trip)
+__device__ __forceinline__ double read_lane(double v, int l) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, l);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), l);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ float read_lane(float v, int l) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_readlane(__builtin_bit_cast(unsigned, v), l));
+}
+
 // The row this workgroup factors (dataflow) or blockIdx.x's row (levels).
 template <bool kFlow>
 __device__ __forceinline__ int flow_row(const int* level_rows, int nrows,
@@ -111,11 +143,54 @@ __device__ __forceinline__ int flow_row(const int* level_rows, int nrows,
 // Wait until the pivot rows piv[0..target] are final.  s_rdy[par] holds the
 // length of the prefix of piv known to be final; wavefront 0 extends it
 // 64 flags per load (one ballot), sleeping between polls while the next
-// pivot row is not done, then takes the agent-scope acquire that makes the
-// pivot rows' values visible, and publishes the new prefix in the other
-// slot, s_rdy[par ^ 1]: every thread reads s_rdy[par] to decide whether to
-// wait, so it must not change until all have passed the barrier.
+// pivot row is not done, and publishes the new prefix in the other slot,
+// s_rdy[par ^ 1]: every thread reads s_rdy[par] to decide whether to wait,
+// so it must not change until all have passed the barrier.
 // Uniform: every thread of the workgroup calls it with the same target.
+// kFence: the wait ends with an agent-scope acquire (it invalidates this
+// XCD's L2); without it the caller reads the pivot rows under the rules
+// below.
+//
+// Pivot rows without cache maintenance.  The rows are exchanged between the
+// XCDs, whose L2 caches are not coherent with each other.  An agent-scope
+// release and acquire pair per row writes back and invalidates the L2, so
+// nothing stays cached: the pattern and the U rows, which hundreds of rows
+// re-read, come from memory each time.  Instead
+//   - a row's final D and U values are written with agent-scope stores
+//     (through the L2), and its flag is set once every wavefront has waited
+//     for its stores (flow_publish);
+//   - a row is read only once its flag is set, so no L2 or L1 can hold an
+//     older copy of a line inside the row, except the owner's own XCD, whose
+//     caches its stores have passed through;
+//   - a line at either end of a row is shared with the next row and may have
+//     been cached earlier, by a reader or the owner of that neighbour: the
+//     blocks that touch the first or last kEdgeBytes of a row are read with
+//     agent-scope loads (edge_block).
+// Cached lines of final rows stay valid, so the L2 serves the re-reads.
+constexpr int kEdgeBytes = 256;  // two 128-byte lines
+// blocks of a row, from either end, that touch its first or last kEdgeBytes
+template <typename T>
+constexpr int kEdgeBlocks = (kEdgeBytes + 36 * (int)sizeof(T) - 1) /
+                            (36 * (int)sizeof(T));
+// block t of the nu blocks of a U part lies at an end of its row (the
+// diagonal block comes before block 0)
+template <typename T>
+__device__ __forceinline__ bool edge_block(int t, int nu) {
+  return t >= nu - kEdgeBlocks<T> || t < kEdgeBlocks<T> - 1;
+}
+template <typename T, bool kFlow>
+__device__ __forceinline__ T load_pivot(const T* p, bool edge) {
+  return kFlow && edge ? load_agent(p) : *p;
+}
+// a row's final value: written through for the rows that wait for it
+template <typename T, bool kFlow>
+__device__ __forceinline__ void store_final(T* p, T v) {
+  if (kFlow)
+    store_agent(p, v);
+  else
+    *p = v;
+}
+template <bool kFence>
 __device__ __forceinline__ void flow_wait(const int* piv, int npiv,
                                           int target, int* s_rdy, int& par,
                                           const Flow& f) {
@@ -153,21 +228,62 @@ __device__ __forceinline__ void flow_wait(const int* piv, int npiv,
       for (int z = 0; z < nap; z++) __builtin_amdgcn_s_sleep(1);
       nap = nap * 2 > 8 ? 8 : nap * 2;
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (kFence)
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    else
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     if (lane == 0) s_rdy[par ^ 1] = rdy;
   }
   __syncthreads();
   par ^= 1;
 }
 
-// Publish row i as final: every wavefront's stores of the row are released
-// at agent scope before the flag is set.
+// Publish row i as final, once every wavefront's stores of the row have
+// completed: released at agent scope (kFence), or written through by
+// store_final and waited for.
+template <bool kFence>
 __device__ __forceinline__ void flow_publish(int i, const Flow& f) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  if (kFence)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  else
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (threadIdx.x == 0)
-    __hip_atomic_store(f.done + i, f.epoch, __ATOMIC_RELEASE,
-                       __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) {
+    if (kFence)
+      __hip_atomic_store(f.done + i, f.epoch, __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    else
+      __hip_atomic_store(f.done + i, f.epoch, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// LU of a 6 x 6 diagonal block without pivoting by wavefront 0 (all 64 lanes
+// call it): lane r < 6 holds row r in d.  Each step's multipliers are formed
+// by the lanes at once, so five divisions are on the chain instead of
+// fifteen.
+template <typename T>
+__device__ __forceinline__ void factor_diag(T (&d)[6], int lane, int i,
+                                            int* pivot) {
+  for (int c = 0; c < 6; c++) {
+    T u[6];
+#pragma unroll
+    for (int m = 0; m < 6; m++) u[m] = read_lane(d[m], c);
+    T piv = u[0], dc = d[0];
+#pragma unroll
+    for (int m = 1; m < 6; m++) {
+      piv = m == c ? u[m] : piv;
+      dc = m == c ? d[m] : dc;
+    }
+    if (piv == T(0)) {
+      if (lane == 0) atomicMin(pivot, i);
+      break;
+    }
+    const T l = dc / piv;
+#pragma unroll
+    for (int m = 0; m < 6; m++)
+      if (lane > c && m >= c) d[m] = m == c ? l : d[m] - l * u[m];
+  }
 }
 
 // One 256-thread workgroup per row of the current level.  The row's column
@@ -209,7 +325,7 @@ __global__ void __launch_bounds__(kIluThreads)
   // dataflow: pivot row scol[kl] is waited for before it is staged (kl) or
   // used (L_ik reads U_kk staged from it; the update reads U_kj)
   auto wait_for = [&](int kl) {
-    if (kFlow) flow_wait(scol, di - r0, kl, s_rdy, par, f);
+    if (kFlow) flow_wait<true>(scol, di - r0, kl, s_rdy, par, f);
   };
   // everything about pivot row k (its U part, U_kk, the positions of its
   // columns in row i) is final before this row starts, so it is staged for
@@ -362,7 +478,7 @@ __global__ void __launch_bounds__(kIluThreads)
 #pragma unroll
     for (int r = 0; r < 6; r++) A[6 * r + c] = x[r];
   }
-  if (kFlow) flow_publish(i, f);
+  if (kFlow) flow_publish<true>(i, f);
 }
 
 // Rows too long for LDS, with the pivots applied in batches.  The values of
@@ -439,7 +555,7 @@ __global__ void __launch_bounds__(kIluThreads)
     int np = min(nbatch, dl - kb);
     if (kFlow) {
       // the batch: the pivots from kb on whose rows are known to be final
-      flow_wait(scol, dl, kb, s_rdy, par, f);
+      flow_wait<false>(scol, dl, kb, s_rdy, par, f);
       np = min(np, s_rdy[par] - kb);
     }
     if (tid < np) {
@@ -450,7 +566,8 @@ __global__ void __launch_bounds__(kIluThreads)
     }
     for (int e = tid; e < 36 * np; e += nth) {
       const int p = e / 36, q = e % 36;
-      const T u = vals[36 * (size_t)diag[scol[kb + p]] + q];
+      const T u = load_pivot<T, kFlow>(
+          vals + 36 * (size_t)diag[scol[kb + p]] + q, true);
       s_ukk[p][q] = u;
       if (q % 7 == 0) s_udi[p][q / 7] = T(1) / u;
       s_ab[p][q] = vals[36 * (size_t)(r0 + kb + p) + q];
@@ -472,8 +589,9 @@ __global__ void __launch_bounds__(kIluThreads)
       if (q <= p) continue;
       const int v = hit[p * maxlen + kb + q];
       if (v)
-        s_uq[batch_pair(p, q)][m] =
-            vals[36 * (size_t)(s_u0[p] + v - 1) + m];
+        s_uq[batch_pair(p, q)][m] = load_pivot<T, kFlow>(
+            vals + 36 * (size_t)(s_u0[p] + v - 1) + m,
+            edge_block<T>(v - 1, s_nu[p]));
     }
     __syncthreads();
     if (tid < 64) {
@@ -547,8 +665,11 @@ __global__ void __launch_bounds__(kIluThreads)
           const int q = q0 + qq;
           const T* U =
               vals + 36 * (size_t)(tt[q] >= 0 ? s_u0[q] + tt[q] : 0) + c;
+          const bool edge = edge_block<T>(tt[q], s_nu[q]);
 #pragma unroll
-          for (int m = 0; m < 6; m++) u[qq][m] = tt[q] >= 0 ? U[6 * m] : T(0);
+          for (int m = 0; m < 6; m++)
+            u[qq][m] = tt[q] >= 0 ? load_pivot<T, kFlow>(U + 6 * m, edge)
+                                  : T(0);
         }
 #pragma unroll
         for (int qq = 0; qq < 4 && q0 + qq < kIluBatch; qq++) {
@@ -579,17 +700,18 @@ __global__ void __launch_bounds__(kIluThreads)
   __syncthreads();
   // factor the diagonal block (no pivoting)
   T* D = vals + 36 * (size_t)(r0 + dl);
-  if (tid == 0) {
-    for (int c = 0; c < 6; c++) {
-      const T piv = D[6 * c + c];
-      if (piv == T(0)) {
-        atomicMin(pivot, i);
-        break;
-      }
-      for (int r = c + 1; r < 6; r++) {
-        const T l = D[6 * r + c] / piv;
-        D[6 * r + c] = l;
-        for (int m = c + 1; m < 6; m++) D[6 * r + m] -= l * D[6 * c + m];
+  T* Dl = s_ab[0];
+  if (tid < 64) {
+    const int r = tid < 6 ? tid : 5;
+    T d[6];
+#pragma unroll
+    for (int m = 0; m < 6; m++) d[m] = D[6 * r + m];
+    factor_diag(d, tid, i, pivot);
+    if (tid < 6) {
+#pragma unroll
+      for (int m = 0; m < 6; m++) {
+        Dl[6 * r + m] = d[m];
+        store_final<T, kFlow>(D + 6 * r + m, d[m]);
       }
     }
   }
@@ -604,13 +726,13 @@ __global__ void __launch_bounds__(kIluThreads)
     for (int r = 0; r < 6; r++) {
       T s = A[6 * r + c];
 #pragma unroll
-      for (int m = 0; m < r; m++) s -= D[6 * r + m] * x[m];
+      for (int m = 0; m < r; m++) s -= Dl[6 * r + m] * x[m];
       x[r] = s;
     }
 #pragma unroll
-    for (int r = 0; r < 6; r++) A[6 * r + c] = x[r];
+    for (int r = 0; r < 6; r++) store_final<T, kFlow>(A + 6 * r + c, x[r]);
   }
-  if (kFlow) flow_publish(i, f);
+  if (kFlow) flow_publish<false>(i, f);
 }
 
 // The same factorisation with row i held in LDS for the whole row: L_ik is
@@ -675,7 +797,7 @@ __global__ void __launch_bounds__(kThreads)
   // dataflow: the values of pivot row scol[kl] are read one (U_kj) or two
   // (U_kk) pivots ahead, so iteration kl waits for pivot kl + 2
   auto wait_for = [&](int kl) {
-    if (kFlow) flow_wait(scol, dl, min(kl, dl - 1), s_rdy, par, f);
+    if (kFlow) flow_wait<false>(scol, dl, min(kl, dl - 1), s_rdy, par, f);
   };
   const int ts = tid - 6, ns = nth - 6;  // staging threads (tid >= 6)
   // position of column j among scol[lo..nb), or -1
@@ -705,8 +827,10 @@ __global__ void __launch_bounds__(kThreads)
       const bool ok = w < 6 * nu;
       const T* U =
           vals + 36 * (size_t)(u0 + (ok ? w / 6 : 0)) + (ok ? w % 6 : 0);
+      const bool edge = edge_block<T>(w / 6, nu);
 #pragma unroll
-      for (int m = 0; m < 6; m++) dst[sp][m] = ok ? U[6 * m] : T(0);
+      for (int m = 0; m < 6; m++)
+        dst[sp][m] = ok ? load_pivot<T, kFlow>(U + 6 * m, edge) : T(0);
     }
   };
   auto load_cols = [&](int kl) {
@@ -718,7 +842,8 @@ __global__ void __launch_bounds__(kThreads)
       pc[q] = (ts >= 0 && t < nu) ? cols[u0 + t] : -1;
     }
     pd = (ts >= 0 && ts < 36 && kl < dl)
-             ? vals[36 * (size_t)diag[scol[kl]] + ts]
+             ? load_pivot<T, kFlow>(vals + 36 * (size_t)diag[scol[kl]] + ts,
+                                    true)
              : T(0);
   };
   // positions and U_kk of pivot kl into buffer buf from the registers
@@ -742,7 +867,8 @@ __global__ void __launch_bounds__(kThreads)
     const int k = scol[0];
     const int u0 = ubs[0], nu = ubs[1] - u0;
     if (tid < 36) {
-      const T u = vals[36 * (size_t)diag[k] + tid];
+      const T u =
+          load_pivot<T, kFlow>(vals + 36 * (size_t)diag[k] + tid, true);
       udg[0][tid] = u;
       if (tid % 7 == 0) udi[0][tid / 7] = T(1) / u;
     }
@@ -800,9 +926,10 @@ __global__ void __launch_bounds__(kThreads)
       const int pl = pos[cur][w / 6], c = w % 6;
       if (pl < 0) continue;
       const T* U = vals + 36 * (size_t)(u0 + w / 6) + c;
+      const bool edge = edge_block<T>(w / 6, nu);
       T um[6];
 #pragma unroll
-      for (int m = 0; m < 6; m++) um[m] = U[6 * m];
+      for (int m = 0; m < 6; m++) um[m] = load_pivot<T, kFlow>(U + 6 * m, edge);
 #pragma unroll
       for (int r = 0; r < 6; r++) {
         T v = 0;
@@ -819,18 +946,15 @@ __global__ void __launch_bounds__(kThreads)
   }
   // factor the diagonal block (no pivoting)
   T* D = row + 36 * dl;
-  if (tid == 0) {
-    for (int c = 0; c < 6; c++) {
-      const T piv = D[6 * c + c];
-      if (piv == T(0)) {
-        atomicMin(pivot, i);
-        break;
-      }
-      for (int r = c + 1; r < 6; r++) {
-        const T l = D[6 * r + c] / piv;
-        D[6 * r + c] = l;
-        for (int m = c + 1; m < 6; m++) D[6 * r + m] -= l * D[6 * c + m];
-      }
+  if (tid < 64) {
+    const int r = tid < 6 ? tid : 5;
+    T d[6];
+#pragma unroll
+    for (int m = 0; m < 6; m++) d[m] = D[6 * r + m];
+    factor_diag(d, tid, i, pivot);
+    if (tid < 6) {
+#pragma unroll
+      for (int m = 0; m < 6; m++) D[6 * r + m] = d[m];
     }
   }
   __syncthreads();
@@ -851,8 +975,9 @@ __global__ void __launch_bounds__(kThreads)
     for (int r = 0; r < 6; r++) A[6 * r + c] = x[r];
   }
   __syncthreads();
-  for (int e = tid; e < 36 * nb; e += nth) vals[36 * (size_t)r0 + e] = row[e];
-  if (kFlow) flow_publish(i, f);
+  for (int e = tid; e < 36 * nb; e += nth)
+    store_final<T, kFlow>(vals + 36 * (size_t)r0 + e, row[e]);
+  if (kFlow) flow_publish<false>(i, f);
 }
 
 // Six lanes per row (lane = scalar row r), ten rows per wave.
@@ -991,19 +1116,6 @@ __device__ __forceinline__ void store_value(T* p, T v) {
   using B = typename Sentinel<T>::Bits;
   __hip_atomic_store(reinterpret_cast<B*>(p), __builtin_bit_cast(B, v),
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// lane l's value, to every lane (v_readlane: a few cycles, where a
-// ds_bpermute shuffle takes an LDS round trip)
-__device__ __forceinline__ double read_lane(double v, int l) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, l);
-  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), l);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-__device__ __forceinline__ float read_lane(float v, int l) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_readlane(__builtin_bit_cast(unsigned, v), l));
 }
 
 template <typename T>
