@@ -227,7 +227,9 @@ size_t ProblemPlan::device_bytes(bool caching) const {
   // one chunk per row), row descriptors, pivot, counter, flags, done
   add((n + 1) * I); add(nm * I); add(n * I); add(n * I); add(n * I);
   add((n + 1) * I); add(4 * n * I); add(4 * n * I); add((n + 1) * I);
-  add(I); add(8); add(2 * I); add(n * I);
+  add(I); add(ilu_counter_bytes()); add(2 * I); add(n * I);
+  // row groups of the two sweeps (at most)
+  add(ilu_group_bytes(n)); add(ilu_group_bytes(n));
   // values and vectors
   add(36 * nk * D); add(36 * nm * D);
   for (int i = 0; i < 5; i++) add(N * D);

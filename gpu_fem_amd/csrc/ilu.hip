@@ -18,7 +18,9 @@
 //     previous level.  GPUFEM_ILU_SCHEDULE=level runs one launch per level
 //     instead.  The arithmetic of a row is the same either way, so the two
 //     schedules give bitwise-identical factors.
-//   sweeps: one persistent launch per sweep, synchronised through the data:
+//   sweeps: over groups of up to eight rows of a chain (trsv_group_kernel,
+//     below) or, for patterns without such chains, over rows.  One
+//     persistent launch per sweep, synchronised through the data:
 //     the output vector is pre-filled with a signalling-NaN sentinel, each
 //     entry is written once with a relaxed agent-scope atomic store, and a
 //     row polls the entries it needs with relaxed agent-scope atomic loads
@@ -50,22 +52,27 @@ struct gf_ilu_s {
   std::vector<int> lmaxlen;                // longest row of each L level
   // sync-free sweep state
   int *lchunk = nullptr, *uchunk = nullptr; // chunk offsets (see below)
-  int4 *lmeta = nullptr, *umeta = nullptr;  // {row, k0, k1, crit} per
+  int4 *lmeta = nullptr, *umeta = nullptr;  // {row, k0, k1, 0} per
                                             // position in hand-out order
   int nlchunk = 0, nuchunk = 0;
   bool lchains = false, uchains = false;  // chunks are chains in row order
   unsigned long long* counter = nullptr;   // chunk dispenser (monotonic)
   int* err = nullptr;  // set when a bounded wait expires: [0] sweeps,
                       // [1] factorisation
-  unsigned long long base = 0;             // counter value at sweep start
+  unsigned long long base = 0;   // value of counter 0 (factorisation, groups)
+  unsigned long long wbase = 0;  // of the counters after it (other sweeps)
   int grid = 0;                            // workgroups per sweep launch
   bool level_sweeps = false;
   // dataflow factorisation: done[i] == epoch once row i is final
   int* done = nullptr;
   int epoch = 0;
-  // dependency level of every chunk (host; batched sweeps merge the chunk
-  // lists of several systems level by level)
-  std::vector<int> lchunk_level, uchunk_level;
+  // sweeps over row groups (trsv_group_kernel; none: nlgroup == 0)
+  int *lgroup = nullptr, *ugroup = nullptr;  // group records
+  int nlgroup = 0, nugroup = 0, ggrid = 0;
+  // dependency level of every group, or of every chunk where there are no
+  // groups (host; batched sweeps merge the items of several systems level by
+  // level)
+  std::vector<int> llevel, ulevel;
 };
 
 namespace gf {
@@ -1046,13 +1053,8 @@ constexpr int kSweepThreads = 256;        // 4 wavefronts per workgroup
 #define GPUFEM_SWEEP_MINWAVES 1
 #endif
 // Waiting on the latest-level dependency alone before gathering the others
-// (GPUFEM_SWEEP_CRIT=1) cuts polling traffic but adds a round trip per row:
-// measured 4.70 vs 3.54 ms a sweep pair on the 400x400 plate (AMD, ILU(12))
-// and 5.53 vs 3.47 ms on the 87x87 plate, and more wavefronts per CU did not
-// recover it (5.07-5.41 ms at 6-16), so it is off.
-#ifndef GPUFEM_SWEEP_CRIT
-#define GPUFEM_SWEEP_CRIT 0
-#endif
+// cuts polling traffic but adds a round trip per row: 4.70 vs 3.54 ms a sweep
+// pair on the 400x400 plate (AMD, ILU(12)).
 // longest sleep between polls, x 64 cycles: L+U pair on the 400x400 plate
 // (ILU(16), 4 batches) 16 -> 4.14 ms, 8 -> 4.09, 4 -> 4.06, 2 -> 4.06,
 // 1 -> 4.07; with 12 batches 8 -> 3.29, 2 -> 3.26; ILU(96), entries of a
@@ -1077,7 +1079,7 @@ constexpr int kSweepThreads = 256;        // 4 wavefronts per workgroup
 #define GPUFEM_SWEEP_WAVES_PER_CU 4
 #endif
 constexpr int kSweepIter = GPUFEM_SWEEP_ITER;  // block batches in registers
-constexpr int kSlots = 10;                // blocks per batch (6 lanes each)
+constexpr int kCounterStride = 32;        // 256 bytes between the counters
 constexpr int kGather = 64;               // dependency blocks per pass
 // blocks next to the diagonal taken as a row's last pass: ILU(96) plate,
 // L+U pair 5.99 ms without, 5.90 / 5.82 / 5.84 / 5.87 / 5.89 ms with 4 / 6 /
@@ -1193,21 +1195,33 @@ __global__ void __launch_bounds__(kSweepThreads, GPUFEM_SWEEP_MINWAVES)
 #pragma unroll
   for (int c = 0; c < 6; c++) cx[c] = T(0);
   auto cached = [&](int j) { return kUseCache && cid == j; };
+  // Wavefront c of a workgroup draws the chunks c, c + kCounters, ... from
+  // counter c: atomics on one address take 12 ns each, 1.8 ms a sweep with a
+  // ticket per row of the 400x400 plate.  Every workgroup has a wavefront of
+  // each class, so the lowest unfinished chunk is always held, or next in
+  // line for a wavefront that holds no unfinished chunk.
+  constexpr int kCounters = kBatched ? 1 : kSweepThreads / 64;
+  const int cls = kBatched ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  counter += kCounterStride * cls;
+  const int ntk = (nchunks + kCounters - 1) / kCounters;
   unsigned long long tk = 0;
   if (lane == 0) tk = atomicAdd(counter, 1ull);
   tk = __shfl(tk, 0, 64);
   long long kc = (long long)(tk - base);
-  while (kc < nchunks) {
+  for (; kc < ntk; kc = (long long)(tk - base)) {
     // take the next chunk now: the counter round trip overlaps this chunk
     unsigned long long tn = 0;
     if (lane == 0) tn = atomicAdd(counter, 1ull);
-    int lc = (int)kc;
+    int lc = (int)kc * kCounters + cls;
+    if (lc >= nchunks) {
+      tk = __shfl(tn, 0, 64);
+      continue;
+    }
     if constexpr (kBatched) {
       const int2 mc = merged[kc];
       lc = mc.y;
       if (*slots[mc.x].go != 1) {  // this system takes no step now
-        tn = __shfl(tn, 0, 64);
-        kc = (long long)(tn - base);
+        tk = __shfl(tn, 0, 64);
         continue;
       }
       if (mc.x != cur_slot) {
@@ -1232,7 +1246,6 @@ __global__ void __launch_bounds__(kSweepThreads, GPUFEM_SWEEP_MINWAVES)
       if (pb + kRows + grp < p1) mnext = meta[pb + kRows + grp];
       const int i = m.x, k0 = live ? m.y : 0, k1 = live ? m.z : 0;
       const int di = kLower ? m.z : m.y - 1;
-      const int crit = live ? m.w : -1;
       T s = (live && gl < 6) ? b[6 * (size_t)i + gl] : T(0);
       if (kLower && fill_next && live && gl < 6)
         reinterpret_cast<B*>(fill_next)[6 * (size_t)i + gl] =
@@ -1256,28 +1269,6 @@ __global__ void __launch_bounds__(kSweepThreads, GPUFEM_SWEEP_MINWAVES)
       // are read (lane q: blocks q, q+G, ...) and the dependencies' entries
       // are loaded at once, polled until no sentinel is left, and parked in
       // LDS; then lanes (t, r) accumulate A[q][r][:] . x[col_q][:].
-#if GPUFEM_SWEEP_CRIT
-      // wait for the critical dependency alone (one load per row group per
-      // poll) before the row's dependencies are gathered: a wavefront that
-      // is levels ahead then adds little polling traffic
-      {
-        const int cj = (crit >= 0 && !cached(crit)) ? crit : -1;
-        B v = cj >= 0 ? load_bits(x + 6 * (size_t)cj) : B(0);
-        unsigned spins = 0;
-        int nap = 1;
-        while (__any(v == Sentinel<T>::value)) {
-          if (++spins > kSpinLimit) {
-            if (lane == 0)
-              __hip_atomic_store(err, 1, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-            break;
-          }
-          for (int z = 0; z < nap; z++) __builtin_amdgcn_s_sleep(1);
-          nap = nap * 2 > GPUFEM_SWEEP_BACKOFF ? GPUFEM_SWEEP_BACKOFF : nap * 2;
-          if (v == Sentinel<T>::value) v = load_bits(x + 6 * (size_t)cj);
-        }
-      }
-#endif
       T acc = T(0);
       const int nb = k1 - k0;
       // The row's latest dependency is usually its nearest row: the last
@@ -1442,12 +1433,515 @@ __global__ void __launch_bounds__(kSweepThreads, GPUFEM_SWEEP_MINWAVES)
         for (int c = 0; c < 6; c++) cx[c] = read_lane(s, c);
       }
     }
-    tn = __shfl(tn, 0, 64);
-    kc = (long long)(tn - base);
+    tk = __shfl(tn, 0, 64);
   }
 }
 
+// ---- sweeps over row groups ----
+// A level of a few rows costs a row's whole latency, from a dependency's
+// store to the row's own (1.2 us on an idle device, 1.6-2.1 us under load).
+// Most of the rows of the narrow levels are chains: row i's first U column
+// is its parent row, which depends on it.  Up to kGroupRows rows of such a
+// chain form a group, solved by one workgroup: wavefront p sums the external
+// dependencies (rows outside the group) of row p as trsv_syncfree_kernel
+// does, and the last wavefront then solves the rows one after another in
+// registers, lane 6p + a holding scalar row a of row p, so that a dependency
+// inside a group costs six v_readlane/fma steps (0.1 us) instead of a round
+// trip through memory.  Each row's entries are stored as soon as the row is
+// solved.  Fewer rows than wavefronts: each row gets several.
+// What bounds it now: 2.5-3 us a group level (0.9 us from the last store to
+// its being seen, 0.5 us for the pass, 0.4 us to the solver, 0.7-1 us the
+// chain), and in the wide levels the 5-9 us latency of a record at two
+// workgroups a CU.  L+U pair, row by row -> groups: 400x400 plate AMD +
+// ILU(96) (1,372 row levels, 181 group levels) FP64 5.15 -> 2.15 ms, FP32
+// 4.88 -> 1.95 ms; 101x101 ILU(64) FP64 1.77 -> 0.50 ms; 45x45 ILU(64)
+// 0.79 -> 0.23 ms; complete LU of a 24,390-node wingbox (3,876 -> 489
+// levels) 10.5 -> 2.65 ms.
+//
+// Group record (kGroupInts ints, rows in solve order): [0] rows n,
+// [8 + p] row, [16 + p], [24 + p] its dependency blocks [k0, k1) (internal
+// ones included: their columns are skipped), [32 + 8 p + q] block index of
+// (row p, row q) for q < p, of the diagonal block for q == p, -1 for none.
+constexpr int kGroupRows = 8;
+constexpr int kGroupInts = 96;
+constexpr int kGroupThreads = 64 * kGroupRows;
+constexpr int kGroupNear = 16;  // blocks next to the diagonal, last pass
+// Groups are used for patterns with at least kGroupRatio row levels per group
+// level: a group level costs 2.5-3 us, a row level 1.2-1.6 us.  FP64 pair row
+// by row / in groups on a 256x256 plate: natural ILU(0) (ratio 1.4) 1.88 /
+// 2.44 ms, AMD ILU(0) (0.2) 0.41 / 0.60 ms, AMD ILU(3) (5.6) 0.75 / 0.58 ms,
+// RCM ILU(3) (5.0) 5.9 / 2.3 ms; RCM ILU(3) of a wingbox (1.6) 7.1 / 6.0 ms.
+constexpr double kGroupRatio = 1.5;
+// records of a sweep at most (a pattern that would need more is swept row by
+// row), for the accounting of device memory
+inline size_t group_records_max(size_t n) { return n / 4 + 64; }
+// kBatched: the groups of several systems, merged[q] = {system, group}; the
+// arrays of a system are in its slot.
+template <typename T, bool kLower, bool kBatched = false>
+__global__ void __launch_bounds__(kGroupThreads, 4)
+    trsv_group_kernel(const int* __restrict__ groups, int ngroups,
+                      const int* __restrict__ cols_, const T* __restrict__ lu_,
+                      const T* b_, T* x_, T* fill_next_,
+                      unsigned long long* counter, unsigned long long base,
+                      int* err,
+                      const SweepSlot<T>* __restrict__ slots = nullptr,
+                      const int2* __restrict__ merged = nullptr) {
+  using B = typename Sentinel<T>::Bits;
+  const int* __restrict__ cols = cols_;
+  const T* __restrict__ lu = lu_;
+  const T* b = b_;
+  T* x = x_;
+  T* fill_next = fill_next_;
+  // batches of ten blocks whose values a pass holds in registers, blocks of a
+  // pass, dependency entries per lane.  Two workgroups a CU take at most 128
+  // registers: 400x400 plate, FP64 pair 2.15 ms with 2 batches, 2.19 ms with
+  // 3 (which spill), 2.25 / 2.31 ms with 4 / 6 and one workgroup a CU.
+  constexpr int kIter = sizeof(T) == 8 ? 2 : 4;
+  constexpr int kPass = 10 * kIter;
+  constexpr int kE = (6 * kPass + 63) / 64;
+  __shared__ T xs_all[kGroupRows][kPass][6];
+  __shared__ T ext[kGroupRows][60];    // external sums of a wavefront's slots
+  __shared__ T coef[6 * kGroupRows][6 * kGroupRows];  // [column][scalar row]
+  __shared__ T diag[6 * kGroupRows];   // U: diagonal entries
+  // group count for which a wavefront has written its coefficients, its sums
+  __shared__ int staged[kGroupRows], arrived[kGroupRows];
+  __shared__ int s_ticket;
+  const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
+  const int t = lane / 6, r = lane % 6;
+  const bool act = lane < 60;
+  if (threadIdx.x < kGroupRows)
+    staged[threadIdx.x] = arrived[threadIdx.x] = 0;
+  // A workgroup holds the ticket of its next group while it works on one,
+  // and every wavefront has the next record in two registers by then (lane l:
+  // ints l and 64 + l), so that neither round trip is waited for.
+  auto ticket = [&]() {  // thread 0: a group, or -1 once there is none left
+    const long long q = (long long)(atomicAdd(counter, 1ull) - base);
+    return q >= 0 && q < ngroups ? (int)q : -1;
+  };
+  int ra = 0, rb = 0, next_sys = 0;
+  auto load_record = [&](int g) {
+    const int* rec;
+    if constexpr (kBatched) {
+      const int2 mg = merged[g];
+      next_sys = mg.x;
+      rec = (kLower ? slots[mg.x].lgroup : slots[mg.x].ugroup) +
+            (size_t)kGroupInts * mg.y;
+    } else {
+      rec = groups + (size_t)kGroupInts * g;
+    }
+    ra = rec[lane];
+    rb = lane < kGroupInts - 64 ? rec[64 + lane] : -1;
+  };
+  int tk = -1;  // thread 0: the ticket after the one in s_ticket
+  if (threadIdx.x == 0) {
+    s_ticket = ticket();
+    if (s_ticket >= 0) tk = ticket();
+  }
+  __syncthreads();
+  int g = s_ticket;
+  if (g >= 0) load_record(g);
+  __syncthreads();
+  for (int seq = 1; g >= 0; seq++) {
+    const int rec0 = ra, rec1 = rb, sys = next_sys;
+    if (threadIdx.x == 0) s_ticket = tk;
+    __syncthreads();
+    g = s_ticket;  // the next group
+    if (g >= 0) {
+      if (threadIdx.x == 0) tk = ticket();
+      load_record(g);
+    }
+    // rows of the group; none where this system takes no step now
+    int n = __builtin_amdgcn_readlane(rec0, 0);
+    if constexpr (kBatched) {
+      const SweepSlot<T>& S = slots[sys];
+      if (*S.go != 1) n = 0;
+      cols = S.cols;
+      lu = S.lu;
+      b = kLower ? S.b : S.tmp;
+      x = kLower ? S.tmp : S.x;
+      fill_next = kLower ? S.x : nullptr;
+    }
+    if (n > 0) {
+      const int p = w % n, part = w / n;
+      const int nparts = (kGroupRows - p + n - 1) / n;
+      int mem[kGroupRows];  // the group's rows: internal dependencies
+#pragma unroll
+      for (int q = 0; q < kGroupRows; q++)
+        mem[q] = q < n ? __builtin_amdgcn_readlane(rec0, 8 + q) : -1;
+      const int k0 = __builtin_amdgcn_readlane(rec0, 16 + p);
+      const int k1 = __builtin_amdgcn_readlane(rec0, 24 + p);
+      const bool solver = w == kGroupRows - 1;
+      // the solver's lane 6 p + a is scalar row a of the group's row p
+      const int sp = lane / 6, sa = lane % 6;
+      const bool live = solver && lane < 6 * n;
+      int srow = 0;
+      T s = T(0);
+      if (solver) {
+        srow = __shfl(rec0, live ? 8 + sp : 8, 64);
+        if (live) s = b[6 * (size_t)srow + sa];
+        if (kLower && fill_next && live)
+          reinterpret_cast<B*>(fill_next)[6 * (size_t)srow + sa] =
+              Sentinel<T>::value;
+      }
+      // coefficients of row p for the solver: the internal blocks (p, q),
+      // q < p, and the strict triangle of the diagonal block, one LDS row per
+      // scalar column
+      if (part == 0) {
+        T v[5];
+        int at[5];
+#pragma unroll
+        for (int z = 0; z < 5; z++) {
+          const int e = 64 * z + lane, q = e / 36;
+          const int i = 32 + 8 * p + (q < 8 ? q : 7);
+          const int b0 = __shfl(rec0, i & 63, 64),
+                    b1 = __shfl(rec1, i & 63, 64);
+          const int bi = q <= p ? (i < 64 ? b0 : b1) : -1;
+          v[z] = bi >= 0 ? lu[36 * (size_t)bi + e % 36] : T(0);
+          at[z] = q;
+        }
+#pragma unroll
+        for (int z = 0; z < 5; z++) {
+          const int q = at[z], rc = (64 * z + lane) % 36, a = rc / 6,
+                    c = rc % 6;
+          if (q >= kGroupRows) continue;
+          if (q == p && a == c) diag[6 * p + a] = v[z];
+          if (q == p && (kLower ? c >= a : c <= a)) v[z] = T(0);
+          coef[6 * q + c][6 * p + a] = v[z];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0)
+          __hip_atomic_store(&staged[w], seq, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      // the solver forms its reciprocal diagonal before the waits
+      const int lc = lane < 6 * kGroupRows ? lane : 0;
+      T dinv = T(1);
+      if (solver) {
+        // every row's coefficients (wavefronts 0 .. n - 1)
+        for (;;) {
+          const int v = lane < n
+                            ? __hip_atomic_load(&staged[lane], __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP)
+                            : seq;
+          if (!__any(v != seq)) break;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        if (!kLower && live) dinv = T(1) / diag[lc];
+        asm volatile("" : "+v"(dinv), "+v"(s));
+      }
+      T(&xs)[kPass][6] = xs_all[w];
+      T acc = T(0);
+      const int nb = k1 - k0;
+      // passes as in trsv_syncfree_kernel: the blocks next to the diagonal
+      // last (part 0), the others in passes of kPass dealt out over the parts,
+      // U rows taking theirs last to first
+      const bool split = nb > kPass;
+      const int nfar = split ? nb - kGroupNear : nb;
+      const int nfp = (nfar + kPass - 1) / kPass;
+      const int npass = nfp + (split ? 1 : 0);
+      for (int pi = part; pi < npass; pi += nparts) {
+        int g0b, ng;
+        const int j = kLower ? pi : nfp - 1 - pi;
+        if (pi == nfp) {
+          g0b = kLower ? k1 - kGroupNear : k0;
+          ng = kGroupNear;
+        } else {
+          const int fb = kLower ? k0 : k0 + (split ? kGroupNear : 0);
+          const int fe = kLower ? (split ? k1 - kGroupNear : k1) : k1;
+          g0b = fb + j * kPass;
+          ng = max(0, min(kPass, fe - g0b));
+        }
+        T a[kIter][6];
+#pragma unroll
+        for (int it = 0; it < kIter; it++) {
+          const int q = 10 * it + t;
+          const bool ok = act && q < ng;
+          const T* ap = lu + 36 * (size_t)(ok ? g0b + q : 0) + 6 * r;
+#pragma unroll
+          for (int c = 0; c < 6; c++) a[it][c] = ok ? ap[c] : T(0);
+        }
+        int jj[kE];
+        B xb[kE];
+#pragma unroll
+        for (int k = 0; k < kE; k++) {
+          const int q = (lane + 64 * k) / 6;
+          int j2 = q < ng ? cols[g0b + q] : -1;
+#pragma unroll
+          for (int u = 0; u < kGroupRows; u++) j2 = j2 == mem[u] ? -1 : j2;
+          jj[k] = j2;
+        }
+#pragma unroll
+        for (int k = 0; k < kE; k++)
+          xb[k] = jj[k] >= 0
+                      ? load_bits(x + 6 * (size_t)jj[k] + (lane + 64 * k) % 6)
+                      : B(0);
+        unsigned spins = 0;
+        int nap = 1;
+        for (;;) {
+          bool pending = false;
+#pragma unroll
+          for (int k = 0; k < kE; k++)
+            pending |= xb[k] == Sentinel<T>::value;
+          if (!__any(pending)) break;
+          if (++spins > kSpinLimit) {
+            if (lane == 0)
+              __hip_atomic_store(err, 1, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int k = 0; k < kE; k++)
+              if (xb[k] == Sentinel<T>::value) xb[k] = B(0);
+            break;
+          }
+          for (int z = 0; z < nap; z++) __builtin_amdgcn_s_sleep(1);
+          nap = nap * 2 > GPUFEM_SWEEP_BACKOFF ? GPUFEM_SWEEP_BACKOFF : nap * 2;
+#pragma unroll
+          for (int k = 0; k < kE; k++)
+            if (xb[k] == Sentinel<T>::value)
+              xb[k] = load_bits(x + 6 * (size_t)jj[k] + (lane + 64 * k) % 6);
+        }
+#pragma unroll
+        for (int k = 0; k < kE; k++) {
+          const int q = (lane + 64 * k) / 6;
+          if (q < ng) xs[q][(lane + 64 * k) % 6] = __builtin_bit_cast(T, xb[k]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int it = 0; it < kIter; it++) {
+          const int q = 10 * it + t;
+          if (act && q < ng) {
+#pragma unroll
+            for (int c = 0; c < 6; c++) acc += a[it][c] * xs[q][c];
+          }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+      // the ten slots' sums go to the solver
+      if (act) ext[w][lane] = acc;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      if (lane == 0)
+        __hip_atomic_store(&arrived[w], seq, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (solver) {
+        T cf[2][6];  // coefficients of this row's columns and the next row's
+#pragma unroll
+        for (int m = 0; m < 6; m++) cf[0][m] = coef[m][lc];
+        // the wavefronts p, p + n, ... sum row p: their sums are added in that
+        // order, once all of them have arrived, and subtracted when row p's turn
+        // comes (the result does not depend on the order of arrival)
+        unsigned mine = 0;
+        for (int u = sp; u < kGroupRows; u += n) mine |= 1u << u;
+        bool taken = !live;
+        T es = T(0);  // external sum of this lane's row
+        unsigned arr = 0;  // wavefronts seen to have arrived
+#pragma unroll
+        for (int q = 0; q < kGroupRows; q++) {
+          if (q < n) {
+            unsigned need = 0;
+            for (int u = q; u < kGroupRows; u += n) need |= 1u << u;
+            while ((arr & need) != need) {
+              const int v = lane < kGroupRows
+                                ? __hip_atomic_load(&arrived[lane],
+                                                    __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_WORKGROUP)
+                                : 0;
+              const unsigned now = (unsigned)__ballot(v == seq);
+              if (now == arr) continue;
+              arr = now;
+              __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+              if (!taken && (arr & mine) == mine) {
+                taken = true;
+                for (int u = sp; u < kGroupRows; u += n) {
+                  T e[10];
+#pragma unroll
+                  for (int z = 0; z < 10; z++) e[z] = ext[u][6 * z + sa];
+#pragma unroll
+                  for (int z = 0; z < 10; z++) es += e[z];
+                }
+              }
+            }
+            if (q + 1 < kGroupRows)
+#pragma unroll
+              for (int m = 0; m < 6; m++)
+                cf[(q + 1) & 1][m] = coef[6 * (q + 1) + m][lc];
+            s -= sp == q ? es : T(0);
+            // L: unit diagonal.  U: x = s / diagonal (a lane's s is final once
+            // its own step is reached)
+#pragma unroll
+            for (int z = 0; z < 6; z++) {
+              const int m = kLower ? z : 5 - z;
+              const T y = read_lane(kLower ? s : s * dinv, 6 * q + m);
+              s -= cf[q & 1][m] * y;
+            }
+            if (sp == q && live)
+              store_value(x + 6 * (size_t)srow + sa, kLower ? s : s * dinv);
+          }
+        }
+      }
+    }
+    __syncthreads();  // s_ticket and the LDS buffers are rewritten next
+  }
+}
+
+// Row groups of a pattern (host).  A row joins the group of the child whose
+// first U column it is (the child latest in level order, when it has
+// several), as long as the group stays free of cycles: no row outside the
+// group with an index below the joining row may depend on a member, or be a
+// dependency of a member in the U sweep.  Then ordering the groups by their
+// last row is a valid order of both sweeps.
+struct SweepGroup {
+  int n = 0;            // rows
+  int row[kGroupRows];  // ascending
+};
+struct SweepGroups {
+  std::vector<SweepGroup> g;
+  std::vector<int> gid;    // group of a row
+  std::vector<int> llev;   // group level of the lower sweep
+  std::vector<int> order;  // groups by last row
+};
+void sweep_groups(int n, const int* rowp, const int* cols, const int* diag,
+                  const std::vector<int>& lptr, const std::vector<int>& lrows,
+                  SweepGroups& sg) {
+  std::vector<int> best(n, -1), lev(n);
+  for (size_t l = 0; l + 1 < lptr.size(); l++)
+    for (int q = lptr[l]; q < lptr[l + 1]; q++) lev[lrows[q]] = (int)l;
+  for (int i = 0; i < n; i++) {
+    if (diag[i] + 1 >= rowp[i + 1]) continue;
+    const int j = cols[diag[i] + 1];
+    if (best[j] < 0 || lev[i] >= lev[best[j]]) best[j] = i;
+  }
+  std::vector<int>& gid = sg.gid;
+  gid.assign(n, -1);
+  sg.g.clear();
+  sg.g.reserve(n / 2 + 1);
+  sg.llev.clear();
+  std::vector<char> closed;  // a row outside depends on a member
+  for (int i = 0; i < n; i++) {
+    int g = -1;
+    const int c = best[i];
+    if (c >= 0) {
+      g = gid[c];
+      const SweepGroup& m = sg.g[g];
+      bool ok = m.n < kGroupRows && m.row[m.n - 1] == c && !closed[g];
+      for (int q = 0; ok && q < m.n; q++)
+        for (int k = diag[m.row[q]] + 1;
+             ok && k < rowp[m.row[q] + 1] && cols[k] < i; k++)
+          ok = gid[cols[k]] == g;
+      if (!ok) g = -1;
+    }
+    if (g < 0) {
+      g = (int)sg.g.size();
+      sg.g.emplace_back();
+      sg.llev.push_back(0);
+      closed.push_back(0);
+    }
+    gid[i] = g;
+    // the groups this row depends on take no more rows, so their levels are
+    // final
+    int l = sg.llev[g];
+    for (int k = rowp[i]; k < diag[i]; k++) {
+      const int h = gid[cols[k]];
+      if (h == g) continue;
+      closed[h] = 1;
+      l = std::max(l, sg.llev[h] + 1);
+    }
+    sg.llev[g] = l;
+    sg.g[g].row[sg.g[g].n++] = i;
+  }
+  sg.order.clear();
+  for (int i = 0; i < n; i++) {
+    const SweepGroup& m = sg.g[gid[i]];
+    if (m.row[m.n - 1] == i) sg.order.push_back(gid[i]);
+  }
+}
+
+// Group records of one sweep, in hand-out order (by group level).
+// level: the group level of each record; returns the number of levels.
+int group_records(const int* rowp, const int* cols, const int* diag,
+                  const SweepGroups& sg, bool lower, std::vector<int>& out,
+                  std::vector<int>& level) {
+  const int ng = (int)sg.g.size();
+  std::vector<int> lev(ng, 0);
+  int nlev = 0;
+  for (int q = 0; q < ng; q++) {
+    const int g = sg.order[lower ? q : ng - 1 - q];
+    const SweepGroup& m = sg.g[g];
+    int l = lower ? sg.llev[g] : 0;
+    if (!lower)
+      for (int z = 0; z < m.n; z++)
+        for (int k = diag[m.row[z]] + 1; k < rowp[m.row[z] + 1]; k++) {
+          const int h = sg.gid[cols[k]];
+          if (h != g) l = std::max(l, lev[h] + 1);
+        }
+    lev[g] = l;
+    nlev = std::max(nlev, l + 1);
+  }
+  std::vector<int> ptr(nlev + 1, 0);
+  for (int g = 0; g < ng; g++) ptr[lev[g] + 1]++;
+  for (int l = 0; l < nlev; l++) ptr[l + 1] += ptr[l];
+  std::vector<int> order(ng);
+  for (int q = 0; q < ng; q++) {
+    const int g = sg.order[lower ? q : ng - 1 - q];
+    order[ptr[lev[g]]++] = g;  // ptr[l] moves to the end of level l
+  }
+  // Groups of one level share a record as long as it holds their rows: the
+  // largest group left, then the largest that still fit.
+  out.clear();
+  out.reserve((size_t)kGroupInts * (ng / 2 + 1));
+  level.clear();
+  std::vector<int> bySize[kGroupRows + 1];
+  for (int l = 0, q0 = 0; l < nlev; q0 = ptr[l++]) {
+    for (int q = ptr[l] - 1; q >= q0; q--)
+      bySize[sg.g[order[q]].n].push_back(order[q]);
+    for (;;) {
+      int used = 0, *rec = nullptr;
+      for (int sz = kGroupRows; sz > 0;) {
+        if (sz > kGroupRows - used || bySize[sz].empty()) {
+          sz--;
+          continue;
+        }
+        const SweepGroup& m = sg.g[bySize[sz].back()];
+        bySize[sz].pop_back();
+        if (!used) {
+          out.resize(out.size() + kGroupInts, -1);
+          rec = out.data() + out.size() - kGroupInts;
+          level.push_back(l);
+        }
+        for (int z = 0; z < sz; z++) {
+          const int i = m.row[lower ? z : sz - 1 - z], p = used + z;
+          const int k0 = lower ? rowp[i] : diag[i] + 1;
+          const int k1 = lower ? diag[i] : rowp[i + 1];
+          rec[8 + p] = i;
+          rec[16 + p] = k0;
+          rec[24 + p] = k1;
+          rec[32 + 8 * p + p] = diag[i];
+          for (int q = used; q < p; q++) {
+            const int* c = std::lower_bound(cols + k0, cols + k1, rec[8 + q]);
+            if (c < cols + k1 && *c == rec[8 + q])
+              rec[32 + 8 * p + q] = (int)(c - cols);
+          }
+        }
+        used += sz;
+        rec[0] = used;
+      }
+      if (!used) break;
+    }
+  }
+  return nlev;
+}
+
 }  // namespace
+
+size_t ilu_counter_bytes() {
+  return sizeof(unsigned long long) * kCounterStride *
+         (1 + kSweepThreads / 64);
+}
+size_t ilu_group_bytes(size_t n) {
+  return sizeof(int) * kGroupInts * group_records_max(n);
+}
 }  // namespace gf
 
 extern "C" {
@@ -1534,11 +2028,32 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
   }
   h->lchains = use_chains;
   h->uchains = use_chains;
+  h->level_sweeps = tenv && std::string(tenv) == "level";
+  // row groups, by the rule at kGroupRatio
+  std::vector<int> lgr, ugr;
+  if (!use_chains && !h->level_sweeps) {
+    gf::SweepGroups sg;
+    gf::sweep_groups(n, rowp, cols, diag.data(), h->lptr, lrows, sg);
+    const int gl = gf::group_records(rowp, cols, diag.data(), sg, true, lgr,
+                                     h->llevel);
+    const int gu =
+        gf::group_records(rowp, cols, diag.data(), sg, false, ugr, h->ulevel);
+    const size_t most = gf::kGroupInts * gf::group_records_max(n);
+    if (lgr.size() <= most && ugr.size() <= most &&
+        gf::kGroupRatio * std::max(gl, gu) <=
+            (double)std::max(h->lptr.size(), h->uptr.size()) - 1) {
+      h->nlgroup = (int)(lgr.size() / gf::kGroupInts);
+      h->nugroup = (int)(ugr.size() / gf::kGroupInts);
+    } else {
+      lgr.clear();
+      ugr.clear();
+    }
+  }
   if (h->lchains) lch = lcn; else chunks(h->lptr, lch);
   if (h->uchains) uch = ucn; else chunks(h->uptr, uch);
   h->nlchunk = (int)lch.size() - 1;
   h->nuchunk = (int)uch.size() - 1;
-  if (!use_chains) {
+  if (!use_chains && !h->nlgroup) {
     auto levels_of = [](const std::vector<int>& ch, const std::vector<int>& lp,
                         std::vector<int>& out) {
       out.resize(ch.size() - 1);
@@ -1548,45 +2063,18 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
         out[c] = (int)l;
       }
     };
-    levels_of(lch, h->lptr, h->lchunk_level);
-    levels_of(uch, h->uptr, h->uchunk_level);
+    levels_of(lch, h->lptr, h->llevel);
+    levels_of(uch, h->uptr, h->ulevel);
   }
-  // row descriptors in hand-out order: one 16-byte load per row
-  // {row, first block, end block, critical dependency}: the diagonal block
-  // is the end (L) or one before the first (U); the critical dependency is
-  // the row's dependency of the highest level, latest in hand-out order
-  // (-1 for none), which is usually the last one to be solved
+  // row descriptors in hand-out order, one 16-byte load per row: {row, first
+  // block, end block, 0}; the diagonal block is the end (L) or one before the
+  // first (U)
   std::vector<int4> lm(n), um(n);
-  {
-    std::vector<int> lev(n), ord(n);
-    auto crit_of = [&](const std::vector<int>& lp, const std::vector<int>& rows,
-                       bool lower, std::vector<int>& out) {
-      for (size_t l = 0; l + 1 < lp.size(); l++)
-        for (int q = lp[l]; q < lp[l + 1]; q++) lev[rows[q]] = (int)l;
-      for (int q = 0; q < n; q++) ord[use_chains ? (lower ? q : n - 1 - q) : rows[q]] = q;
-      out.assign(n, -1);
-      for (int i = 0; i < n; i++) {
-        const int k0 = lower ? rowp[i] : diag[i] + 1;
-        const int k1 = lower ? diag[i] : rowp[i + 1];
-        int best = -1;
-        for (int k = k0; k < k1; k++) {
-          const int j = cols[k];
-          if (best < 0 || lev[j] > lev[best] ||
-              (lev[j] == lev[best] && ord[j] > ord[best]))
-            best = j;
-        }
-        out[i] = best;
-      }
-    };
-    std::vector<int> lcrit, ucrit;
-    crit_of(h->lptr, lrows, true, lcrit);
-    crit_of(h->uptr, urows, false, ucrit);
-    for (int p = 0; p < n; p++) {
-      const int li = use_chains ? p : lrows[p];
-      lm[p] = make_int4(li, rowp[li], diag[li], lcrit[li]);
-      const int ui = use_chains ? n - 1 - p : urows[p];
-      um[p] = make_int4(ui, diag[ui] + 1, rowp[ui + 1], ucrit[ui]);
-    }
+  for (int p = 0; p < n; p++) {
+    const int li = use_chains ? p : lrows[p];
+    lm[p] = make_int4(li, rowp[li], diag[li], 0);
+    const int ui = use_chains ? n - 1 - p : urows[p];
+    um[p] = make_int4(ui, diag[ui] + 1, rowp[ui + 1], 0);
   }
   auto up = [&](int** dst, const int* src, size_t cnt) -> int {
     GF_TRY(gf::dmalloc(ctx, (void**)dst, sizeof(int) * (cnt ? cnt : 1)));
@@ -1595,7 +2083,9 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
     return GF_OK;
   };
   int st = GF_OK;
-  if ((st = up(&h->rowp, rowp, n + 1)) || (st = up(&h->cols, cols, rowp[n])) ||
+  if ((st = up(&h->lgroup, lgr.data(), lgr.size())) ||
+      (st = up(&h->ugroup, ugr.data(), ugr.size())) ||
+      (st = up(&h->rowp, rowp, n + 1)) || (st = up(&h->cols, cols, rowp[n])) ||
       (st = up(&h->diag, diag.data(), n)) ||
       (st = up(&h->lrows, lrows.data(), n)) ||
       (st = up(&h->urows, urows.data(), n)) ||
@@ -1604,12 +2094,12 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
       (st = up((int**)&h->umeta, (const int*)um.data(), 4 * (size_t)n)) ||
       (st = up(&h->uchunk, uch.data(), uch.size())) ||
       (st = gf::dmalloc(ctx, (void**)&h->pivot, sizeof(int))) ||
-      (st = gf::dmalloc(ctx, (void**)&h->counter, sizeof(unsigned long long))) ||
+      (st = gf::dmalloc(ctx, (void**)&h->counter, gf::ilu_counter_bytes())) ||
       (st = gf::dmalloc(ctx, (void**)&h->err, 2 * sizeof(int))) ||
       (st = gf::dmalloc(ctx, (void**)&h->done, sizeof(int) * (size_t)n)) ||
       (st = gf::check_hip(ctx, hipMemsetAsync(h->done, 0, sizeof(int) * (size_t)n,
                                               ctx->stream), "memset")) ||
-      (st = gf::check_hip(ctx, hipMemsetAsync(h->counter, 0, sizeof(unsigned long long),
+      (st = gf::check_hip(ctx, hipMemsetAsync(h->counter, 0, gf::ilu_counter_bytes(),
                                               ctx->stream), "memset")) ||
       (st = gf::check_hip(ctx, hipMemsetAsync(h->err, 0, 2 * sizeof(int), ctx->stream),
                           "memset"))) {
@@ -1627,8 +2117,15 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
         1, std::min({std::max(h->nlchunk, h->nuchunk), target_waves,
                      std::max(64, 8 * mean_w)}));
     h->grid = (waves + 3) / 4;
-    const char* env = getenv("GPUFEM_TRSV");
-    h->level_sweeps = env && std::string(env) == "level";
+    // Workgroups of a group sweep: two a CU where each has dozens of
+    // records to take (400x400 plate 2.15 against 2.25 ms a pair), one
+    // otherwise (wingbox of 24,390 nodes 2.65 against 2.82 ms), fewer for a
+    // small system, which would only wait in them (45x45 plate: 0.25 ms with
+    // 64, 128 or 256) and take the device from other streams.
+    const int nrec = std::max(h->nlgroup, h->nugroup);
+    const int cus = std::max(1, ctx->num_cus);
+    h->ggrid = std::min({nrec, nrec >= 32 * cus ? 2 * cus : cus,
+                         std::max(64, nrec / 6)});
   }
   st = gf::check_hip(ctx, hipStreamSynchronize(ctx->stream), "ilu upload");
   if (st) {
@@ -1650,6 +2147,8 @@ int gf_ilu_destroy(gf_ilu h) {
   gf::dfree(h->ctx, h->lchunk);
   gf::dfree(h->ctx, h->lmeta);
   gf::dfree(h->ctx, h->umeta);
+  gf::dfree(h->ctx, h->lgroup);
+  gf::dfree(h->ctx, h->ugroup);
   gf::dfree(h->ctx, h->uchunk);
   gf::dfree(h->ctx, h->counter);
   gf::dfree(h->ctx, h->err);
@@ -1708,8 +2207,10 @@ int ilu_view(gf_ilu h, IluView* v) {
   v->lchunk = h->lchunk;
   v->uchunk = h->uchunk;
   v->cols = h->cols;
-  v->lchunk_level = &h->lchunk_level;
-  v->uchunk_level = &h->uchunk_level;
+  v->lgroup = h->nlgroup ? h->lgroup : nullptr;
+  v->ugroup = h->nlgroup ? h->ugroup : nullptr;
+  v->llevel = &h->llevel;
+  v->ulevel = &h->ulevel;
   v->grid = h->grid;
   return GF_OK;
 }
@@ -1718,35 +2219,45 @@ __global__ void reset_counters_kernel(unsigned long long* c, int n) {
   if ((int)threadIdx.x < n) c[threadIdx.x] = 0ull;
 }
 
-// One L and one U sync-free sweep over several systems: each chunk list is
-// the systems' chunks merged level by level (see IluView).  counters[0..1]
-// are zeroed first by a kernel (no memset: the launches may be captured in
-// a graph), so the tickets start at 0 in every replay.
+// One L and one U sweep over several systems (see SweepItems): the chunks of
+// the systems without row groups, then the groups of the others.  The
+// counters are zeroed first by a kernel (no memset: the launches may be
+// captured in a graph), so the tickets start at 0 in every replay.
 template <typename T>
 int launch_batch_sweeps(hipStream_t s, const SweepSlot<T>* slots,
-                        const int2* lmerged, int nl, const int2* umerged,
-                        int nu, int grid, unsigned long long* counters,
-                        int* err) {
+                        const SweepItems& it, int grid, int ggrid,
+                        unsigned long long* counters, int* err) {
   hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counters,
-                     2);
-  hipLaunchKernelGGL((trsv_syncfree_kernel<T, true, 1, true>), dim3(grid),
-                     dim3(kSweepThreads), 0, s, (const int4*)nullptr,
-                     (const int*)nullptr, (const int*)nullptr, nl,
-                     (const T*)nullptr, (const T*)nullptr, (T*)nullptr,
-                     (T*)nullptr, counters, 0ull, err, slots, lmerged);
-  hipLaunchKernelGGL((trsv_syncfree_kernel<T, false, 1, true>), dim3(grid),
-                     dim3(kSweepThreads), 0, s, (const int4*)nullptr,
-                     (const int*)nullptr, (const int*)nullptr, nu,
-                     (const T*)nullptr, (const T*)nullptr, (T*)nullptr,
-                     (T*)nullptr, counters + 1, 0ull, err, slots, umerged);
+                     kBatchCounters);
+  auto sweep = [&](auto lower) {
+    constexpr bool kLower = decltype(lower)::value;
+    const int2* items = kLower ? it.l : it.u;
+    const int nc = kLower ? it.lc : it.uc, ng = kLower ? it.lg : it.ug;
+    unsigned long long* c = counters + (kLower ? 0 : 2);
+    if (nc > 0)
+      hipLaunchKernelGGL((trsv_syncfree_kernel<T, kLower, 1, true>),
+                         dim3(grid), dim3(kSweepThreads), 0, s,
+                         (const int4*)nullptr, (const int*)nullptr,
+                         (const int*)nullptr, nc, (const T*)nullptr,
+                         (const T*)nullptr, (T*)nullptr, (T*)nullptr, c, 0ull,
+                         err, slots, items);
+    if (ng > 0)
+      hipLaunchKernelGGL((trsv_group_kernel<T, kLower, true>),
+                         dim3(std::min(ggrid, ng)), dim3(kGroupThreads), 0, s,
+                         (const int*)nullptr, ng, (const int*)nullptr,
+                         (const T*)nullptr, (const T*)nullptr, (T*)nullptr,
+                         (T*)nullptr, c + 1, 0ull, err, slots, items + nc);
+  };
+  sweep(std::true_type{});
+  sweep(std::false_type{});
   return hipGetLastError() == hipSuccess ? GF_OK : GF_ERR_DEVICE;
 }
 template int launch_batch_sweeps<double>(hipStream_t, const SweepSlot<double>*,
-                                         const int2*, int, const int2*, int,
-                                         int, unsigned long long*, int*);
+                                         const SweepItems&, int, int,
+                                         unsigned long long*, int*);
 template int launch_batch_sweeps<float>(hipStream_t, const SweepSlot<float>*,
-                                        const int2*, int, const int2*, int,
-                                        int, unsigned long long*, int*);
+                                        const SweepItems&, int, int,
+                                        unsigned long long*, int*);
 }  // namespace gf
 
 namespace {
@@ -1981,23 +2492,38 @@ int ilu_apply(gf_ilu h, const T* lu, const T* b, T* tmp, T* x) {
     return GF_ERR_INVALID;
   gf_context ctx = h->ctx;
   if (!h->level_sweeps) {
-    const unsigned long long waves = 4ull * h->grid;
     const size_t N = 6 * (size_t)h->n;
     hipLaunchKernelGGL(gf::fill_sentinel_kernel<T>, dim3(gf::div_up(N, 256)),
                        dim3(256), 0, ctx->stream, N, tmp);
+    if (h->nlgroup) {
+      hipLaunchKernelGGL((gf::trsv_group_kernel<T, true>), dim3(h->ggrid),
+                         dim3(gf::kGroupThreads), 0, ctx->stream, h->lgroup,
+                         h->nlgroup, h->cols, lu, b, tmp, x, h->counter,
+                         h->base, h->err);
+      h->base += (unsigned long long)(h->nlgroup + h->ggrid);
+      hipLaunchKernelGGL((gf::trsv_group_kernel<T, false>), dim3(h->ggrid),
+                         dim3(gf::kGroupThreads), 0, ctx->stream, h->ugroup,
+                         h->nugroup, h->cols, lu, tmp, x, (T*)nullptr,
+                         h->counter, h->base, h->err);
+      h->base += (unsigned long long)(h->nugroup + h->ggrid);
+      return gf::check_launch(ctx, "trsv_group_kernel");
+    }
     // one row per wavefront: two rows of a level per wavefront
     // (trsv_syncfree_kernel<T, L, 2>) measured slower, 4.8 vs 3.5 ms a pair
     // on the 400x400 plate
+    unsigned long long* const ctr = h->counter + gf::kCounterStride;
     hipLaunchKernelGGL((gf::trsv_syncfree_kernel<T, true, 1>), dim3(h->grid),
                        dim3(gf::kSweepThreads), 0, ctx->stream, h->lmeta,
-                       h->cols, h->lchunk, h->nlchunk, lu, b, tmp, x,
-                       h->counter, h->base, h->err);
-    h->base += (unsigned long long)h->nlchunk + waves;
+                       h->cols, h->lchunk, h->nlchunk, lu, b, tmp, x, ctr,
+                       h->wbase, h->err);
+    h->wbase += gf::div_up(h->nlchunk, gf::kSweepThreads / 64) +
+                (unsigned long long)h->grid;
     hipLaunchKernelGGL((gf::trsv_syncfree_kernel<T, false, 1>), dim3(h->grid),
                        dim3(gf::kSweepThreads), 0, ctx->stream, h->umeta,
                        h->cols, h->uchunk, h->nuchunk, lu, tmp, x, (T*)nullptr,
-                       h->counter, h->base, h->err);
-    h->base += (unsigned long long)h->nuchunk + waves;
+                       ctr, h->wbase, h->err);
+    h->wbase += gf::div_up(h->nuchunk, gf::kSweepThreads / 64) +
+                (unsigned long long)h->grid;
     return gf::check_launch(ctx, "trsv_syncfree_kernel");
   }
   const int nl = (int)h->lptr.size() - 1;

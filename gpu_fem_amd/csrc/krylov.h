@@ -87,6 +87,8 @@ struct SweepSlot {
   const int4* umeta;
   const int* lchunk;
   const int* uchunk;
+  const int* lgroup;  // group records (null: swept by chunks)
+  const int* ugroup;
   const int* cols;
   const T* lu;
   const T* b;
@@ -94,22 +96,35 @@ struct SweepSlot {
   T* x;
   const int* go;  // batched launches sweep the system only while *go == 1
 };
-// The device schedule of an ILU analysis (chunk mode only) and the
-// dependency level of each chunk.
+// The device schedule of an ILU analysis (row groups where it has them, else
+// chunks) and the dependency level of each item.
 struct IluView {
   int n = 0;
   const int4 *lmeta = nullptr, *umeta = nullptr;
   const int *lchunk = nullptr, *uchunk = nullptr, *cols = nullptr;
-  const std::vector<int>* lchunk_level = nullptr;
-  const std::vector<int>* uchunk_level = nullptr;
+  const int *lgroup = nullptr, *ugroup = nullptr;  // null: no row groups
+  const std::vector<int>* llevel = nullptr;  // of each group, or each chunk
+  const std::vector<int>* ulevel = nullptr;
   int grid = 0;
 };
+// Work items {system, chunk or group} of a batched sweep pair on the device:
+// nc chunks of the systems without row groups, then ng groups of the others,
+// each part merged level by level.
+struct SweepItems {
+  const int2 *l = nullptr, *u = nullptr;
+  int lc = 0, lg = 0, uc = 0, ug = 0;
+};
+// tickets counters of a batched sweep pair (device, unsigned long long each)
+constexpr int kBatchCounters = 4;
 int ilu_view(gf_ilu h, IluView* v);
+// device memory of an analysis: ticket counters; row groups of one sweep (at
+// most) of a pattern of n rows
+size_t ilu_counter_bytes();
+size_t ilu_group_bytes(size_t n);
 template <typename T>
 int launch_batch_sweeps(hipStream_t s, const SweepSlot<T>* slots,
-                        const int2* lmerged, int nl, const int2* umerged,
-                        int nu, int grid, unsigned long long* counters,
-                        int* err);
+                        const SweepItems& items, int grid, int ggrid,
+                        unsigned long long* counters, int* err);
 // bit pattern the sweeps take for "not yet written"
 unsigned long long sweep_sentinel_bits(bool fp64);
 

@@ -1144,7 +1144,7 @@ struct Solve {
   // solo sweep of the cycle end: a one-entry table and its chunk lists
   void* d_solo = nullptr;
   int2 *d_sl = nullptr, *d_su = nullptr;
-  int nsl = 0, nsu = 0;
+  SweepItems solo;
   int* d_one = nullptr;
   bool finished = false;
   int status = GF_ERR_NO_CONVERGENCE;
@@ -1170,7 +1170,8 @@ class BatchEngine {
   long long *d_voff = nullptr, *d_roff = nullptr;
   int2 *d_lm = nullptr, *d_um = nullptr;
   size_t lm_cap = 0, um_cap = 0;
-  int nl = 0, nu = 0, grid = 1, maxm = 1;
+  SweepItems items;
+  int grid = 1, maxm = 1;
   long long ntot = 0, nrows = 0;
   unsigned long long* d_counters = nullptr;
   int* d_err = nullptr;
@@ -1207,6 +1208,8 @@ SweepSlot<T> sweep_entry(const Solve* v, const int* go) {
   e.umeta = v->iv.umeta;
   e.lchunk = v->iv.lchunk;
   e.uchunk = v->iv.uchunk;
+  e.lgroup = v->iv.lgroup;
+  e.ugroup = v->iv.ugroup;
   e.cols = v->iv.cols;
   gf_problem p = v->p;
   if (sizeof(T) == 8) {
@@ -1277,15 +1280,16 @@ int BatchEngine::rebuild() {
     maxm = std::max(maxm, v->m);
     gsum += std::max(1, v->iv.grid);
   }
-  // chunk lists merged level by level
-  auto merge = [&](bool lower, std::vector<int2>& out) {
-    out.clear();
+  // items merged level by level: the chunks of the systems without row
+  // groups, then the groups of the others
+  auto merge = [&](bool lower, bool groups, std::vector<int2>& out) {
     std::vector<size_t> cur(ns, 0);
     for (int lev = 0;; lev++) {
       bool any = false;
       for (int i = 0; i < ns; i++) {
+        if ((act[i]->iv.lgroup != nullptr) != groups) continue;
         const std::vector<int>& cl =
-            lower ? *act[i]->iv.lchunk_level : *act[i]->iv.uchunk_level;
+            lower ? *act[i]->iv.llevel : *act[i]->iv.ulevel;
         while (cur[i] < cl.size() && cl[cur[i]] == lev) {
           out.push_back(make_int2(i, (int)cur[i]));
           cur[i]++;
@@ -1295,10 +1299,14 @@ int BatchEngine::rebuild() {
       if (!any) break;
     }
   };
-  merge(true, lm);
-  merge(false, um);
-  nl = (int)lm.size();
-  nu = (int)um.size();
+  merge(true, false, lm);
+  items.lc = (int)lm.size();
+  merge(true, true, lm);
+  items.lg = (int)lm.size() - items.lc;
+  merge(false, false, um);
+  items.uc = (int)um.size();
+  merge(false, true, um);
+  items.ug = (int)um.size() - items.uc;
   ntot = voff[ns];
   nrows = roff[ns];
   grid = std::max(1, std::min(gsum, std::max(1, waves_per_cu * ctx->num_cus / 4)));
@@ -1311,6 +1319,8 @@ int BatchEngine::rebuild() {
   };
   GF_TRY(ensure(&d_lm, lm_cap, lm.size()));
   GF_TRY(ensure(&d_um, um_cap, um.size()));
+  items.l = d_lm;
+  items.u = d_um;
   std::vector<unsigned char> sw;
   if (fp64())
     fill_tables<double>(sw);
@@ -1374,7 +1384,7 @@ int BatchEngine::issue_steps() {
       hipLaunchKernelGGL(batch_gather<double>, g1, dim3(256), 0, s, ns, ntot,
                          d_voff, d_kry, d_state, sent);
       GF_TRY(launch_batch_sweeps<double>(
-          s, (const SweepSlot<double>*)d_sweep, d_lm, nl, d_um, nu, grid,
+          s, (const SweepSlot<double>*)d_sweep, items, grid, ctx->num_cus,
           d_counters, d_err));
       hipLaunchKernelGGL(batch_spmv<double>, g1r, dim3(256), 0, s, ns, nrows,
                          d_roff, d_kry, d_state);
@@ -1382,7 +1392,7 @@ int BatchEngine::issue_steps() {
       hipLaunchKernelGGL(batch_gather<float>, g1, dim3(256), 0, s, ns, ntot,
                          d_voff, d_kry, d_state, sent);
       GF_TRY(launch_batch_sweeps<float>(
-          s, (const SweepSlot<float>*)d_sweep, d_lm, nl, d_um, nu, grid,
+          s, (const SweepSlot<float>*)d_sweep, items, grid, ctx->num_cus,
           d_counters, d_err));
       hipLaunchKernelGGL(batch_spmv<float>, g1r, dim3(256), 0, s, ns, nrows,
                          d_roff, d_kry, d_state);
@@ -1435,19 +1445,23 @@ int BatchEngine::start(Solve* v) {
   else
     *reinterpret_cast<SweepSlot<float>*>(v->h_solo.data()) =
         sweep_entry<float>(v, v->d_one);
-  v->nsl = (int)v->iv.lchunk_level->size();
-  v->nsu = (int)v->iv.uchunk_level->size();
-  v->h_sl.resize(v->nsl);
-  v->h_su.resize(v->nsu);
-  for (int c = 0; c < v->nsl; c++) v->h_sl[c] = make_int2(0, c);
-  for (int c = 0; c < v->nsu; c++) v->h_su[c] = make_int2(0, c);
-  GF_TRY(dmalloc(ctx, (void**)&v->d_sl, sizeof(int2) * std::max(1, v->nsl)));
-  GF_TRY(dmalloc(ctx, (void**)&v->d_su, sizeof(int2) * std::max(1, v->nsu)));
+  const int nsl = (int)v->iv.llevel->size(), nsu = (int)v->iv.ulevel->size();
+  v->h_sl.resize(nsl);
+  v->h_su.resize(nsu);
+  for (int c = 0; c < nsl; c++) v->h_sl[c] = make_int2(0, c);
+  for (int c = 0; c < nsu; c++) v->h_su[c] = make_int2(0, c);
+  GF_TRY(dmalloc(ctx, (void**)&v->d_sl, sizeof(int2) * std::max(1, nsl)));
+  GF_TRY(dmalloc(ctx, (void**)&v->d_su, sizeof(int2) * std::max(1, nsu)));
+  v->solo = SweepItems{};
+  v->solo.l = v->d_sl;
+  v->solo.u = v->d_su;
+  (v->iv.lgroup ? v->solo.lg : v->solo.lc) = nsl;
+  (v->iv.lgroup ? v->solo.ug : v->solo.uc) = nsu;
   GF_HIP(ctx, hipMemcpyAsync(v->d_solo, v->h_solo.data(), v->h_solo.size(),
                              hipMemcpyHostToDevice, s));
-  GF_HIP(ctx, hipMemcpyAsync(v->d_sl, v->h_sl.data(), sizeof(int2) * v->nsl,
+  GF_HIP(ctx, hipMemcpyAsync(v->d_sl, v->h_sl.data(), sizeof(int2) * nsl,
                              hipMemcpyHostToDevice, s));
-  GF_HIP(ctx, hipMemcpyAsync(v->d_su, v->h_su.data(), sizeof(int2) * v->nsu,
+  GF_HIP(ctx, hipMemcpyAsync(v->d_su, v->h_su.data(), sizeof(int2) * nsu,
                              hipMemcpyHostToDevice, s));
   KrylovWork& W = p->kw;
   hipLaunchKernelGGL(multi_dot_partial, dim3(kDotBlocks, 1), dim3(kDotThreads),
@@ -1557,18 +1571,16 @@ int BatchEngine::cycle_end(Solve* v) {
     hipLaunchKernelGGL(gather_one<double>, grid1(v->N), dim3(256), 0, s, v->N,
                        W.tmp, p->work64, p->work64b, sent);
     GF_TRY(launch_batch_sweeps<double>(s, (const SweepSlot<double>*)v->d_solo,
-                                       v->d_sl, v->nsl, v->d_su, v->nsu,
-                                       std::max(1, v->iv.grid), d_counters,
-                                       d_err));
+                                       v->solo, std::max(1, v->iv.grid),
+                                       ctx->num_cus, d_counters, d_err));
     hipLaunchKernelGGL(axpy_from<double>, grid1(v->N), dim3(256), 0, s, v->N,
                        (const double*)p->kw.z, p->sol);
   } else {
     hipLaunchKernelGGL(gather_one<float>, grid1(v->N), dim3(256), 0, s, v->N,
                        W.tmp, p->t32a, p->t32b, sent);
     GF_TRY(launch_batch_sweeps<float>(s, (const SweepSlot<float>*)v->d_solo,
-                                      v->d_sl, v->nsl, v->d_su, v->nsu,
-                                      std::max(1, v->iv.grid), d_counters,
-                                      d_err));
+                                      v->solo, std::max(1, v->iv.grid),
+                                      ctx->num_cus, d_counters, d_err));
     hipLaunchKernelGGL(axpy_from<float>, grid1(v->N), dim3(256), 0, s, v->N,
                        (const float*)p->t32c, p->sol);
   }
@@ -1772,7 +1784,8 @@ int batch_engine_create(int device, int precision, int max_slots,
   if (!st) st = dmalloc(c, (void**)&e->d_state, sizeof(SlotState) * max_slots);
   if (!st) st = dmalloc(c, (void**)&e->d_voff, sizeof(long long) * (max_slots + 1));
   if (!st) st = dmalloc(c, (void**)&e->d_roff, sizeof(long long) * (max_slots + 1));
-  if (!st) st = dmalloc(c, (void**)&e->d_counters, 2 * sizeof(unsigned long long));
+  if (!st) st = dmalloc(c, (void**)&e->d_counters,
+                        kBatchCounters * sizeof(unsigned long long));
   if (!st) st = dmalloc(c, (void**)&e->d_err, sizeof(int));
   if (!st)
     st = check_hip(c, hipHostMalloc((void**)&e->h_state,
