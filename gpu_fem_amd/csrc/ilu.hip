@@ -745,11 +745,12 @@ __global__ void __launch_bounds__(kIluThreads)
 // The same factorisation with row i held in LDS for the whole row: L_ik is
 // formed from, and the updates A_ij -= L_ik U_kj are applied to, the LDS
 // copy, so the only global accesses inside the pivot loop are reads of the
-// final rows k.  Those are pipelined one pivot ahead: the U-part bounds of
-// every pivot row are read into LDS once; while pivot k is processed, the
-// column indices and U_kk of pivot k+2 and each thread's U_kj columns of
-// pivot k+1 are loaded into registers, and the positions of pivot k+1's
-// columns in row i are searched.  The row is written back once at the end.
+// final rows k.  Those are pipelined: the U-part bounds of every pivot row
+// are read into LDS once; while pivot k is processed, the column indices of
+// pivot k+2 and, if it is final by then, U_kk and each thread's U_kj columns
+// of pivot k+1 are loaded into registers, and the positions of pivot k+1's
+// columns in row i are searched.  The row is written back once at the end,
+// D and U first.
 // Arithmetic is that of ilu_row_kernel, operation for operation.
 // Dynamic LDS: 36 * nb values, nb column indices, 2 * nl pivot bounds.
 #ifndef GPUFEM_ILU_PAIRS
@@ -801,11 +802,12 @@ __global__ void __launch_bounds__(kThreads)
   if (tid == 0) s_rdy[0] = 0;
   int par = 0;
   __syncthreads();
-  // dataflow: the values of pivot row scol[kl] are read one (U_kj) or two
-  // (U_kk) pivots ahead, so iteration kl waits for pivot kl + 2
+  // dataflow: pivot kl is waited for when its turn comes; its values are read
+  // one pivot ahead where it is known to be final by then
   auto wait_for = [&](int kl) {
-    if (kFlow) flow_wait<false>(scol, dl, min(kl, dl - 1), s_rdy, par, f);
+    if (kFlow) flow_wait<false>(scol, dl, kl, s_rdy, par, f);
   };
+  auto ready = [&](int kl) { return !kFlow || s_rdy[par] > kl; };
   const int ts = tid - 6, ns = nth - 6;  // staging threads (tid >= 6)
   // position of column j among scol[lo..nb), or -1
   auto find = [&](int j, int lo) {
@@ -820,8 +822,8 @@ __global__ void __launch_bounds__(kThreads)
     return (lo < nb && scol[lo] == j) ? lo : -1;
   };
   // registers: this thread's U_kj columns for the current and next pivot,
-  // and (staging threads) the column indices and U_kk entry of the pivot
-  // after next
+  // and (staging threads) the column indices of the pivot after next and the
+  // U_kk entry of the next
   T uv[kIluPairs][6], un[kIluPairs][6];
   int pc[kIluCols];
   T pd = T(0);
@@ -848,12 +850,8 @@ __global__ void __launch_bounds__(kThreads)
       const int t = ts + q * ns;
       pc[q] = (ts >= 0 && t < nu) ? cols[u0 + t] : -1;
     }
-    pd = (ts >= 0 && ts < 36 && kl < dl)
-             ? load_pivot<T, kFlow>(vals + 36 * (size_t)diag[scol[kl]] + ts,
-                                    true)
-             : T(0);
   };
-  // positions and U_kk of pivot kl into buffer buf from the registers
+  // positions of pivot kl into buffer buf from the registers
   auto stage_from_regs = [&](int kl, int buf) {
     const int u0 = ubs[2 * kl], nu = ubs[2 * kl + 1] - u0;
 #pragma unroll
@@ -863,32 +861,44 @@ __global__ void __launch_bounds__(kThreads)
     }
     for (int t = ts + kIluCols * ns; t < nu; t += ns)
       pos[buf][t] = find(cols[u0 + t], kl + 1);
-    if (ts < 36) {
+  };
+  // U_kk of pivot kl (threads 6 .. 41), into buffer buf
+  auto load_diag = [&](int kl) {
+    if (ts >= 0 && ts < 36)
+      pd = load_pivot<T, kFlow>(vals + 36 * (size_t)(ubs[2 * kl] - 1) + ts,
+                                true);
+  };
+  auto stage_diag = [&](int buf) {
+    if (ts >= 0 && ts < 36) {
       udg[buf][ts] = pd;
       if (ts % 7 == 0) udi[buf][ts / 7] = T(1) / pd;
     }
   };
   if (dl > 0) {
-    wait_for(1);
-    // pivot 0 staged directly by all threads
-    const int k = scol[0];
     const int u0 = ubs[0], nu = ubs[1] - u0;
-    if (tid < 36) {
-      const T u =
-          load_pivot<T, kFlow>(vals + 36 * (size_t)diag[k] + tid, true);
-      udg[0][tid] = u;
-      if (tid % 7 == 0) udi[0][tid / 7] = T(1) / u;
-    }
     for (int t = tid; t < nu; t += nth) pos[0][t] = find(cols[u0 + t], 1);
-    load_u(0, uv);
     load_cols(1);
   }
+  bool have = false;  // pivot kl's values are staged
   __syncthreads();
   for (int kl = 0; kl < dl; kl++) {
     const int cur = kl & 1;
     const int u0 = ubs[2 * kl], nu = ubs[2 * kl + 1] - u0;
-    if (kl + 1 < dl) wait_for(kl + 2);
-    load_u(kl + 1, un);
+    if (!have) {
+      wait_for(kl);
+      load_u(kl, uv);
+      load_diag(kl);
+      stage_diag(cur);
+      __syncthreads();
+    }
+    // the next pivot's values, if it is known to be final (waiting for it
+    // here would hold back this pivot: in a chain, the last two pivots of a
+    // row would be applied after the last one had become final)
+    const bool next = kl + 1 < dl && ready(kl + 1);
+    if (next) {
+      load_u(kl + 1, un);
+      load_diag(kl + 1);
+    }
     if (tid < 6) {
       const int r = tid;
       const T* Ukk = udg[cur];
@@ -945,11 +955,13 @@ __global__ void __launch_bounds__(kThreads)
         row[36 * pl + 6 * r + c] -= v;
       }
     }
+    if (next) stage_diag(cur ^ 1);
     __syncthreads();
 #pragma unroll
     for (int sp = 0; sp < kIluPairs; sp++)
 #pragma unroll
       for (int m = 0; m < 6; m++) uv[sp][m] = un[sp][m];
+    have = next;
   }
   // factor the diagonal block (no pivoting)
   T* D = row + 36 * dl;
@@ -982,9 +994,11 @@ __global__ void __launch_bounds__(kThreads)
     for (int r = 0; r < 6; r++) A[6 * r + c] = x[r];
   }
   __syncthreads();
-  for (int e = tid; e < 36 * nb; e += nth)
+  // the rows that wait read D and U only: L follows the flag
+  for (int e = 36 * dl + tid; e < 36 * nb; e += nth)
     store_final<T, kFlow>(vals + 36 * (size_t)r0 + e, row[e]);
   if (kFlow) flow_publish<false>(i, f);
+  for (int e = tid; e < 36 * dl; e += nth) vals[36 * (size_t)r0 + e] = row[e];
 }
 
 // Six lanes per row (lane = scalar row r), ten rows per wave.
