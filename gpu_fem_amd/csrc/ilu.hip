@@ -488,22 +488,25 @@ __global__ void __launch_bounds__(kIluThreads)
   if (kFlow) flow_publish<true>(i, f);
 }
 
-// Rows too long for LDS, with the pivots applied in batches.  The values of
-// row i stay in global memory.  A batch takes up to nbatch consecutive
-// pivots whose rows are final; wavefront 0 forms their L_ik in order, each
-// applied at once to the batch's own later L-part blocks (held in LDS), and
-// then one pass reads every (block, column) pair of the rest of the row that
-// a pivot of the batch updates once, subtracts the batch's contributions
-// L_ik U_kj in pivot order and writes it once: one read-modify-write of the
-// touched part of the row per batch instead of one per pivot, and each U_kj
-// column loaded once for its six rows.  The pass walks the pivots' U-part
-// lists (a pair is taken by the first pivot of the batch that updates it),
-// so a batch of one pivot costs what a pivot step of ilu_row_kernel does.
-// Every entry sees the operations of ilu_row_kernel in the same order, so
-// the factors agree bit for bit.
-// Dynamic LDS: the column indices of row i; per pivot of the batch, the
-// position in row i of each of its U-part columns (or -1) and, per position
-// of row i, 1 + the index in the pivot's U part (0: not updated).
+// Rows too long for LDS, with the pivots applied in runs.  The values of row
+// i stay in global memory.  A window of up to nbatch pivots is prepared ahead,
+// final or not: where the columns of their U parts lie in row i depends on
+// the pattern alone.  The pivots of the window that are final form a run:
+// wavefront 0 forms their L_ik in order, each applied at once to the run's
+// own later L-part blocks (held in LDS), and one pass reads every block of the
+// rest of the row that a pivot of the run updates once, subtracts the run's
+// contributions L_ik U_kj in pivot order and writes it once.  Every entry
+// sees the operations of ilu_row_kernel in the same order, so the factors
+// agree bit for bit.
+// A thread takes kBatchCols columns of a block: it loads whole rows of U_kj
+// in wide loads (one column per thread takes four times the load
+// instructions, each touching as many lines), the next pivot's while the
+// current one is applied, and shares each value of L_ik read from LDS among
+// them.
+// Dynamic LDS per position of row i: its column index, its place in the list
+// of the run's blocks, and per pivot of the window the index (+ 1) of the
+// position in the pivot's U part (0: not updated) and, as a list, the position
+// of each of its U-part columns (or -1).
 #ifndef GPUFEM_ILU_BATCH
 #define GPUFEM_ILU_BATCH 8
 #endif
@@ -513,37 +516,52 @@ constexpr int kIluPairSlots = kIluBatch * (kIluBatch - 1) / 2;
 __device__ __forceinline__ int batch_pair(int p, int q) {
   return p * (2 * kIluBatch - p - 1) / 2 + (q - p - 1);
 }
-// dynamic LDS bytes per position of the longest row, batch of nbatch
+// dynamic LDS bytes per position of the longest row, window of nbatch
 __host__ __device__ constexpr size_t batch_lds_per_pos(int nbatch) {
-  return sizeof(int) + 2 * sizeof(short) * (size_t)nbatch;
+  return sizeof(int) + sizeof(short) * (size_t)(2 * nbatch + 1);
 }
+// 400x400 plate, AMD + ILU(96), whole factorisation, columns per thread:
+// FP64 1 / 2 / 3 / 6: 96 / 89 / 122 / 126 ms (3 and 6 leave room for one
+// workgroup a CU), FP32 2 / 3 / 6: 78 / 78 / 101 ms; 256 or 1,024 threads
+// 102 or 109 ms FP64.  (One column per thread, batches that waited for all
+// their pivots' lists, and the row's pairs found by walking the U parts:
+// 111 ms FP64, 97 ms FP32.)
+constexpr int kBatchThreads = 512;
+template <typename T> constexpr int kBatchCols = sizeof(T) == 8 ? 2 : 3;
 template <typename T, bool kFlow>
-__global__ void __launch_bounds__(kIluThreads)
+__global__ void __launch_bounds__(kBatchThreads)
     ilu_row_batch_kernel(const int* __restrict__ level_rows, int nrows,
                          const int* __restrict__ rowp,
                          const int* __restrict__ cols,
                          const int* __restrict__ diag, T* vals, int* pivot,
                          Flow f, int nbatch, int maxlen) {
-  extern __shared__ __align__(16) int ilu_bdyn[];
-  __shared__ int s_u0[kIluBatch], s_nu[kIluBatch];
-  __shared__ T s_ukk[kIluBatch][36];
+  constexpr int C = kBatchCols<T>, S = 6 / C;
+  // blocks of a pivot's U part that load_pivot reads past the caches: its
+  // first kHead and last kTail ones go through LDS
+  constexpr int kTail = kEdgeBlocks<T>, kHead = kEdgeBlocks<T> - 1;
+  constexpr int kEdge = 1 + kTail + kHead;  // with the diagonal block
+  extern __shared__ __align__(16) unsigned char ilu_bdyn[];
+  __shared__ int s_u0[kIluBatch], s_nu[kIluBatch];  // per window slot
+  __shared__ __align__(16) T s_edge[kIluBatch][kEdge][36];
   __shared__ T s_udi[kIluBatch][6];  // 1 / diagonal of U_kk
-  __shared__ T s_lik[kIluBatch][36];
-  __shared__ T s_ab[kIluBatch][36];       // A_ik of the batch's pivots
-  __shared__ T s_uq[kIluPairSlots][36];   // U_kp,kq, p < q in the batch
-  __shared__ int s_row, s_rdy[2];
+  __shared__ __align__(16) T s_lik[kIluBatch][36];
+  __shared__ T s_ab[kIluBatch][36];       // A_ik of the run's pivots
+  __shared__ T s_uq[kIluPairSlots][36];   // U_kp,kq, p < q in the run
+  __shared__ int s_row, s_rdy[2], s_cnt;
   const int i = flow_row<kFlow>(level_rows, nrows, f, &s_row);
   if (i < 0) return;
-  const int tid = threadIdx.x, nth = blockDim.x;
+  const int tid = threadIdx.x, nth = kBatchThreads;
   const int r0 = rowp[i], r1 = rowp[i + 1], nb = r1 - r0, dl = diag[i] - r0;
-  int* scol = ilu_bdyn;
-  // hit[p * maxlen + pl] = 1 + index in U(k_p) of position pl, or 0
-  unsigned short* hit = reinterpret_cast<unsigned short*>(ilu_bdyn + maxlen);
-  // upos[p * maxlen + t] = position in row i of U(k_p)'s column t, or -1
+  int* scol = reinterpret_cast<int*>(ilu_bdyn);
+  // hit[s * maxlen + pl] = 1 + index in U(k) of position pl for the pivot k in
+  // slot s, or 0; upos[s * maxlen + t] = position of U(k)'s column t, or -1
+  unsigned short* hit = reinterpret_cast<unsigned short*>(scol + maxlen);
   short* upos = reinterpret_cast<short*>(hit + (size_t)nbatch * maxlen);
+  unsigned short* list =
+      reinterpret_cast<unsigned short*>(upos + (size_t)nbatch * maxlen);
   for (int t = tid; t < nb; t += nth) scol[t] = cols[r0 + t];
   for (int e = tid; e < nbatch * maxlen; e += nth) hit[e] = 0;
-  if (tid == 0) s_rdy[0] = 0;
+  if (tid == 0) s_rdy[0] = s_cnt = 0;
   int par = 0;
   __syncthreads();
   // position of column j among scol[lo..nb), or -1
@@ -558,51 +576,111 @@ __global__ void __launch_bounds__(kIluThreads)
     }
     return (lo < nb && scol[lo] == j) ? lo : -1;
   };
-  for (int kb = 0; kb < dl;) {
-    int np = min(nbatch, dl - kb);
-    if (kFlow) {
-      // the batch: the pivots from kb on whose rows are known to be final
-      flow_wait<false>(scol, dl, kb, s_rdy, par, f);
-      np = min(np, s_rdy[par] - kb);
-    }
-    if (tid < np) {
-      const int k = scol[kb + tid];
+  // pivots [k0, k1) of the row into their slots (pivot k: slot k % nbatch)
+  auto prepare = [&](int k0, int k1) {
+    if (tid < k1 - k0) {
+      const int k = scol[k0 + tid], s = (k0 + tid) % nbatch;
       const int u0 = diag[k] + 1;
-      s_u0[tid] = u0;
-      s_nu[tid] = rowp[k + 1] - u0;
-    }
-    for (int e = tid; e < 36 * np; e += nth) {
-      const int p = e / 36, q = e % 36;
-      const T u = load_pivot<T, kFlow>(
-          vals + 36 * (size_t)diag[scol[kb + p]] + q, true);
-      s_ukk[p][q] = u;
-      if (q % 7 == 0) s_udi[p][q / 7] = T(1) / u;
-      s_ab[p][q] = vals[36 * (size_t)(r0 + kb + p) + q];
+      s_u0[s] = u0;
+      s_nu[s] = rowp[k + 1] - u0;
     }
     __syncthreads();
-    int tot = 0;  // U-part columns of the batch's pivots
-    for (int p = 0; p < np; p++) {
-      const int u0 = s_u0[p], nu = s_nu[p];
+    for (int k = k0; k < k1; k++) {
+      const int s = k % nbatch, u0 = s_u0[s], nu = s_nu[s];
       for (int t = tid; t < nu; t += nth) {
-        const int pl = find(cols[u0 + t], kb + p + 1);
-        upos[p * maxlen + t] = (short)pl;
-        if (pl >= 0) hit[p * maxlen + pl] = (unsigned short)(t + 1);
+        const int pl = find(cols[u0 + t], k + 1);
+        upos[s * maxlen + t] = (short)pl;
+        if (pl >= 0) hit[s * maxlen + pl] = (unsigned short)(t + 1);
       }
-      tot += nu;
     }
     __syncthreads();
-    for (int e = tid; e < 36 * np * np; e += nth) {
-      const int pq = e / 36, m = e % 36, p = pq / np, q = pq % np;
-      if (q <= p) continue;
-      const int v = hit[p * maxlen + kb + q];
-      if (v)
-        s_uq[batch_pair(p, q)][m] = load_pivot<T, kFlow>(
-            vals + 36 * (size_t)(s_u0[p] + v - 1) + m,
-            edge_block<T>(v - 1, s_nu[p]));
+  };
+  int kb = 0, kw = min(nbatch, dl);  // the window: pivots [kb, kw)
+  if (dl > 0) prepare(0, kw);
+  while (kb < dl) {
+    int pe = kw;  // the run [kb, pe)
+    if (kFlow) {
+      flow_wait<false>(scol, dl, kb, s_rdy, par, f);
+      pe = min(pe, s_rdy[par]);
+    }
+    const int np = pe - kb, sb = kb % nbatch;
+    // slot of the run's pivot p
+    auto slot = [&](int p) { return sb + p >= nbatch ? sb + p - nbatch : sb + p; };
+    // U_kk and the edge blocks of the pivots' U parts, and A_ik
+    for (int e = tid; e < 36 * kEdge * np; e += nth) {
+      const int p = e / (36 * kEdge), b = e / 36 % kEdge, q = e % 36;
+      const int nu = s_nu[slot(p)], u0 = s_u0[slot(p)];
+      // block of the row part D U: the diagonal, the head, the tail
+      const int blk = b <= kHead ? b - 1 : nu - (kEdge - b);
+      if (b > 0 && (blk < 0 || blk >= nu)) continue;
+      const T u =
+          load_pivot<T, kFlow>(vals + 36 * (size_t)(u0 + blk) + q, true);
+      s_edge[p][b][q] = u;
+      if (b == 0) {
+        if (q % 7 == 0) s_udi[p][q / 7] = T(1) / u;
+        s_ab[p][q] = vals[36 * (size_t)(r0 + kb + p) + q];
+      }
+    }
+    // U_kp,kq for the pairs of the run
+    if (np > 1)
+      for (int e = tid; e < 36 * np * np; e += nth) {
+        const int pq = e / 36, m = e % 36, p = pq / np, q = pq % np;
+        if (q <= p) continue;
+        const int v = hit[slot(p) * maxlen + kb + q];
+        if (v)
+          s_uq[batch_pair(p, q)][m] = load_pivot<T, kFlow>(
+              vals + 36 * (size_t)(s_u0[slot(p)] + v - 1) + m,
+              edge_block<T>(v - 1, s_nu[slot(p)]));
+      }
+    // the blocks past the run's L part that a pivot of the run updates
+    for (int pl = pe + tid; pl < nb; pl += nth) {
+      unsigned any = 0;
+      for (int p = 0; p < np; p++) any |= hit[slot(p) * maxlen + pl];
+      if (any) list[atomicAdd(&s_cnt, 1)] = (unsigned short)pl;
     }
     __syncthreads();
+    const int items = S * s_cnt;
+    // this thread's item: its block of the row, its columns, its values
+    T a[6][C], u[6][C];
+    int pl = -1, c0 = 0;
+    T* A = nullptr;
+    auto load_u = [&](int p) {  // false: pivot p does not update the block
+      const int s = slot(p);
+      const int tt = pl >= 0 ? (int)hit[s * maxlen + pl] - 1 : -1;
+      if (tt < 0) return false;
+      const int nu = s_nu[s];
+      if (kFlow && edge_block<T>(tt, nu)) {
+        const T* U = s_edge[p][tt >= nu - kTail ? kEdge - (nu - tt) : 1 + tt];
+#pragma unroll
+        for (int m = 0; m < 6; m++)
+#pragma unroll
+          for (int c = 0; c < C; c++) u[m][c] = U[6 * m + c0 + c];
+      } else {
+        const T* U = vals + 36 * (size_t)(s_u0[s] + tt) + c0;
+#pragma unroll
+        for (int m = 0; m < 6; m++)
+#pragma unroll
+          for (int c = 0; c < C; c++) u[m][c] = U[6 * m + c];
+      }
+      return true;
+    };
+    bool on = false;
+    auto load_item = [&](int w) {
+      pl = -1;
+      if (w < items) {
+        pl = list[w / S];
+        c0 = C * (w % S);
+        A = vals + 36 * (size_t)(r0 + pl) + c0;
+#pragma unroll
+        for (int r = 0; r < 6; r++)
+#pragma unroll
+          for (int c = 0; c < C; c++) a[r][c] = A[6 * r + c];
+      }
+      on = load_u(0);
+    };
+    load_item(tid);
     if (tid < 64) {
-      // wavefront 0: L_ik of each pivot, each applied to the batch's later
+      // wavefront 0: L_ik of each pivot, each applied to the run's later
       // L-part blocks before the next is formed
       for (int p = 0; p < np; p++) {
         if (tid < 6) {
@@ -612,7 +690,7 @@ __global__ void __launch_bounds__(kIluThreads)
           for (int c = 0; c < 6; c++) {
             T v = s_ab[p][6 * r + c];
 #pragma unroll
-            for (int m = 0; m < c; m++) v -= x[m] * s_ukk[p][6 * m + c];
+            for (int m = 0; m < c; m++) v -= x[m] * s_edge[p][0][6 * m + c];
             x[c] = v * s_udi[p][c];
           }
 #pragma unroll
@@ -623,91 +701,87 @@ __global__ void __launch_bounds__(kIluThreads)
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        if (tid < 36) {
-          const int r = tid / 6, c = tid % 6;
-          for (int q = p + 1; q < np; q++) {
-            if (!hit[p * maxlen + kb + q]) continue;
-            const T* U = s_uq[batch_pair(p, q)];
-            T acc = 0;
+        for (int e = tid; e < 36 * (np - 1 - p); e += 64) {
+          const int q = p + 1 + e / 36, r = e % 36 / 6, c = e % 6;
+          if (!hit[slot(p) * maxlen + kb + q]) continue;
+          const T* U = s_uq[batch_pair(p, q)];
+          T acc = 0;
 #pragma unroll
-            for (int m = 0; m < 6; m++) acc += s_lik[p][6 * r + m] * U[6 * m + c];
-            s_ab[q][6 * r + c] = s_ab[q][6 * r + c] - acc;
-          }
+          for (int m = 0; m < 6; m++) acc += s_lik[p][6 * r + m] * U[6 * m + c];
+          s_ab[q][6 * r + c] = s_ab[q][6 * r + c] - acc;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
       }
     }
     __syncthreads();
+    if (tid == 0) s_cnt = 0;
     for (int e = tid; e < 36 * np; e += nth)
       vals[36 * (size_t)(r0 + kb + e / 36) + e % 36] = s_ab[e / 36][e % 36];
-    // the rest of the row: (block, column) pairs of the pivots' U-part
-    // lists, each taken by the first pivot of the batch that updates it
-    const int pl0 = kb + np;
-    for (int w = tid; w < 6 * tot; w += nth) {
-      // L_ik is re-read from LDS per pair (hoisted out of the loop it would
-      // take 36 registers per pivot)
-      __asm__ volatile("" ::: "memory");
-      int p = 0, rem = w;
-      while (rem >= 6 * s_nu[p]) rem -= 6 * s_nu[p++];
-      const int t = rem / 6, c = rem % 6;
-      const int pl = upos[p * maxlen + t];
-      if (pl < pl0) continue;  // not in the row (-1), or in the batch's L part
-      bool first = true;
-      for (int q = 0; q < p; q++) first = first && !hit[q * maxlen + pl];
-      if (!first) continue;
-      int tt[kIluBatch];
+    for (int w = tid; w < items; w += nth) {
+      if (w > tid) load_item(w);
+      for (int p = 0; p < np; p++) {
+        T uc[6][C];
+        const bool now = on;
 #pragma unroll
-      for (int q = 0; q < kIluBatch; q++)
-        tt[q] = (q >= p && q < np) ? (int)hit[q * maxlen + pl] - 1 : -1;
-      T* A = vals + 36 * (size_t)(r0 + pl) + c;
-      T a[6];
+        for (int m = 0; m < 6; m++)
 #pragma unroll
-      for (int r = 0; r < 6; r++) a[r] = A[6 * r];
-#pragma unroll
-      for (int q0 = 0; q0 < kIluBatch; q0 += 4) {
-        T u[4][6];
-#pragma unroll
-        for (int qq = 0; qq < 4 && q0 + qq < kIluBatch; qq++) {
-          const int q = q0 + qq;
-          const T* U =
-              vals + 36 * (size_t)(tt[q] >= 0 ? s_u0[q] + tt[q] : 0) + c;
-          const bool edge = edge_block<T>(tt[q], s_nu[q]);
-#pragma unroll
-          for (int m = 0; m < 6; m++)
-            u[qq][m] = tt[q] >= 0 ? load_pivot<T, kFlow>(U + 6 * m, edge)
-                                  : T(0);
-        }
-#pragma unroll
-        for (int qq = 0; qq < 4 && q0 + qq < kIluBatch; qq++) {
-          const int q = q0 + qq;
-          if (tt[q] < 0) continue;
+          for (int c = 0; c < C; c++) uc[m][c] = u[m][c];
+        if (p + 1 < np) on = load_u(p + 1);
+        if (now) {
 #pragma unroll
           for (int r = 0; r < 6; r++) {
-            T v = 0;
+            T l[6];
 #pragma unroll
-            for (int m = 0; m < 6; m++) v += s_lik[q][6 * r + m] * u[qq][m];
-            a[r] = a[r] - v;
+            for (int m = 0; m < 6; m++) l[m] = s_lik[p][6 * r + m];
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+              T v = 0;
+#pragma unroll
+              for (int m = 0; m < 6; m++) v += l[m] * uc[m][c];
+              a[r][c] = a[r][c] - v;
+            }
           }
         }
       }
 #pragma unroll
-      for (int r = 0; r < 6; r++) A[6 * r] = a[r];
+      for (int r = 0; r < 6; r++)
+#pragma unroll
+        for (int c = 0; c < C; c++) A[6 * r + c] = a[r][c];
     }
     __syncthreads();
-    // clear the batch's hits
-    for (int p = 0; p < np; p++)
-      for (int t = tid; t < s_nu[p]; t += nth) {
-        const int pl = upos[p * maxlen + t];
-        if (pl >= 0) hit[p * maxlen + pl] = 0;
+    // the run's slots are free: clear their hits, prepare the next pivots
+    for (int p = 0; p < np; p++) {
+      const int s = slot(p);
+      for (int t = tid; t < s_nu[s]; t += nth) {
+        const int q = upos[s * maxlen + t];
+        if (q >= 0) hit[s * maxlen + q] = 0;
       }
+    }
     __syncthreads();
-    kb += np;
+    kb = pe;
+    const int kn = min(kb + nbatch, dl);
+    if (kn > kw) prepare(kw, kn);
+    kw = kn;
   }
   __syncthreads();
-  // factor the diagonal block (no pivoting)
+  // factor the diagonal block (no pivoting); meanwhile the first pairs of the
+  // U part are loaded
   T* D = vals + 36 * (size_t)(r0 + dl);
   T* Dl = s_ab[0];
+  const int nr = nb - (dl + 1);
+  constexpr int K = 4;  // (block, column) pairs per thread in flight
+  T x[K][6];
+  auto load_u_part = [&](int w0) {
+#pragma unroll
+    for (int z = 0; z < K; z++) {
+      const int w = w0 + z * nth + tid;
+      const T* B = D + 36 * (size_t)(1 + (w < 6 * nr ? w / 6 : 0)) + w % 6;
+#pragma unroll
+      for (int r = 0; r < 6; r++) x[z][r] = w < 6 * nr ? B[6 * r] : T(0);
+    }
+  };
+  load_u_part(0);
   if (tid < 64) {
     const int r = tid < 6 ? tid : 5;
     T d[6];
@@ -724,20 +798,20 @@ __global__ void __launch_bounds__(kIluThreads)
   }
   __syncthreads();
   // U_ij = L_ii^-1 A_ij for the blocks right of the diagonal
-  const int nr = nb - (dl + 1);
-  for (int w = tid; w < 6 * nr; w += nth) {
-    const int t = w / 6, c = w % 6;
-    T* A = D + 36 * (size_t)(1 + t);
-    T x[6];
+  for (int w0 = 0; w0 < 6 * nr; w0 += K * nth) {
+    if (w0 > 0) load_u_part(w0);
 #pragma unroll
-    for (int r = 0; r < 6; r++) {
-      T s = A[6 * r + c];
+    for (int z = 0; z < K; z++) {
+      const int w = w0 + z * nth + tid;
+      if (w >= 6 * nr) continue;
 #pragma unroll
-      for (int m = 0; m < r; m++) s -= Dl[6 * r + m] * x[m];
-      x[r] = s;
+      for (int r = 1; r < 6; r++)
+#pragma unroll
+        for (int m = 0; m < r; m++) x[z][r] -= Dl[6 * r + m] * x[z][m];
+      T* B = D + 36 * (size_t)(1 + w / 6) + w % 6;
+#pragma unroll
+      for (int r = 0; r < 6; r++) store_final<T, kFlow>(B + 6 * r, x[z][r]);
     }
-#pragma unroll
-    for (int r = 0; r < 6; r++) store_final<T, kFlow>(A + 6 * r + c, x[r]);
   }
   if (kFlow) flow_publish<false>(i, f);
 }
@@ -2284,8 +2358,8 @@ int ilu_factor(gf_ilu h, T* vals, int* zero_pivot) {
                              hipMemcpyHostToDevice, ctx->stream));
   // rows whose values fit in LDS (dynamic LDS per level: its longest row)
   // are factored there; the other levels run ilu_row_kernel
-  static size_t lds_cap[2] = {0, 0};
-  static size_t batch_cap[2] = {0, 0};
+  static size_t lds_cap[2] = {0, 0}, lds_half[2] = {0, 0};
+  static size_t batch_cap[2] = {0, 0}, batch_cap2[2] = {0, 0};
   static std::once_flag once[2];
   const int ti = sizeof(T) == 8 ? 0 : 1;
   std::call_once(once[ti], [&] {
@@ -2338,7 +2412,11 @@ int ilu_factor(gf_ilu h, T* vals, int* zero_pivot) {
         bcap = 0;
       }
     batch_cap[ti] = bcap;
+    // dynamic LDS that lets two workgroups share a CU
+    const size_t stat = total - bcap;
+    batch_cap2[ti] = total / 2 > stat ? total / 2 - stat : 0;
     lds_cap[ti] = cap;
+    lds_half[ti] = cap > total / 2 ? cap - total / 2 : cap;
   });
   const int maxlen = h->max_row_len;
   const size_t gdyn = 3 * sizeof(int) * (size_t)maxlen;
@@ -2351,7 +2429,7 @@ int ilu_factor(gf_ilu h, T* vals, int* zero_pivot) {
   int nbatch = 0;
   {
     // two workgroups per CU where the LDS allows
-    const size_t cap2 = std::min(batch_cap[ti], (size_t)64 * 1024);
+    const size_t cap2 = std::min(batch_cap[ti], batch_cap2[ti]);
     for (int nbt = gf::kIluBatch; nbt >= 1 && !nbatch; nbt--)
       if (gf::batch_lds_per_pos(nbt) * maxlen <= cap2) nbatch = nbt;
     for (int nbt = gf::kIluBatch; nbt >= 1 && !nbatch; nbt--)
@@ -2367,12 +2445,12 @@ int ilu_factor(gf_ilu h, T* vals, int* zero_pivot) {
     if (nbatch > 0) {
       if (flow)
         hipLaunchKernelGGL((gf::ilu_row_batch_kernel<T, true>), dim3(cnt),
-                           dim3(gf::kIluThreads), bdyn, ctx->stream, rows,
+                           dim3(gf::kBatchThreads), bdyn, ctx->stream, rows,
                            cnt, h->rowp, h->cols, h->diag, vals, h->pivot, f,
                            nbatch, maxlen);
       else
         hipLaunchKernelGGL((gf::ilu_row_batch_kernel<T, false>), dim3(cnt),
-                           dim3(gf::kIluThreads), bdyn, ctx->stream, rows,
+                           dim3(gf::kBatchThreads), bdyn, ctx->stream, rows,
                            cnt, h->rowp, h->cols, h->diag, vals, h->pivot, f,
                            nbatch, maxlen);
     } else if (flow) {
@@ -2426,9 +2504,20 @@ int ilu_factor(gf_ilu h, T* vals, int* zero_pivot) {
                                  ctx->stream));
       h->epoch = 1;
     }
-    int first_global = 0;
-    while (first_global < nl && !no_lds && dyn_of(first_global) <= cap)
-      first_global++;
+    // A row that takes more than half of a CU's LDS has the CU to itself,
+    // where two workgroups of the global-memory kernel fit: such levels run
+    // there unless they are chains (fewer than 1.25 rows a level), where only
+    // a row's latency counts.  Half / all of the LDS: 400x400 plate ILU(96)
+    // FP32 65 / 75 ms, FP64 83 / 86 ms; 101x101 ILU(64) FP32 6.0 / 7.6 ms;
+    // complete LU of a wingbox of 24,390 nodes FP64 26.5 / 20.3 ms.
+    auto levels_within = [&](size_t lim) {
+      int l = 0;
+      while (l < nl && !no_lds && dyn_of(l) <= lim) l++;
+      return l;
+    };
+    int first_global = levels_within(std::min(cap, lds_half[ti]));
+    if (4 * (h->n - h->lptr[first_global]) < 5 * (nl - first_global))
+      first_global = levels_within(cap);
     // longest row up to each level: it bounds the U part of every pivot row
     // of the rows up to there
     std::vector<int> pmax(nl + 1, 0);
