@@ -521,14 +521,26 @@ __global__ void __launch_bounds__(64)
 // block of v_mfma_f64_4x4x4_4b_f64 (four independent 4x4x4 products per
 // instruction).  K_e = sum_q detXd_q B_q^T C B_q is one 24 x 24 x 36 product
 // with the 36 = 9 strains x 4 quadrature points stacked strain-major: k-block
-// s (4 wide) holds strain s at the four points.  Lane (i, q) of an element
-// (its A row i and k index q, see mfma_d_row) forms the columns j = i + 4J
-// (J = 0..5) of B_q in registers -- exactly the MFMA A operand
-// A[i][q] = B_q[s][4I + i] of tile row I and the B operand
-// D[q][j] = detXd_q (C B_q)[s][4J + j] of tile column J -- so B and D never
-// pass through LDS.  Only the 21 tiles on and above the diagonal of the
-// 6 x 6 tile grid are formed (K_e is symmetric): 9 x 21 MFMAs per four
-// elements, 24,192 flops per element.  K_e is then staged in LDS and
+// s (4 wide) holds strain s at the four points.  Tile (I, J) of the product
+// is taken over the nodes, K_e[6a + I][6b + J] for a, b = 0..3: the lane
+// (a, q) of an element (its A row a and k index q, see MfmaLane) forms the
+// six columns 6a + k of node a at point q in registers -- the MFMA A operand
+// A[a][q] = B_q[s][6a + I] and the B operand D[q][b] = detXd_q (C B_q)[s]
+// [6b + J] -- so B and D never pass through LDS, which DOF a column is of is
+// known at compile time, and the node's and the point's frames are formed in
+// the lane itself: only the node normals and drill vectors go through LDS.
+// With column 4J + i in the lane instead (DOF and node both of the lane), the
+// two kinds of columns diverge and index arrays at run time, and geometry
+// and column parts went through 20 KB of LDS a wavefront in four steps on 4,
+// 5 or 16 of 64 lanes: 400 x 400 plate, colour-ordered, 4 x 182 us; so
+// 85, 110, 140 and 145 us.  What bounds it: the first colour, all stores, the
+// chain of loads and frames at two wavefronts a SIMD (75 us without the
+// scatter; three do not fit 54 + 21 doubles); the later colours also the adds'
+// read-modify-writes of K (as plain stores 76 us; as loads and stores 157 to
+// 180).
+// Only the 21 tiles I <= J are formed (K_e is symmetric): 9 x 21 MFMAs per
+// four elements, 24,192 flops per element.  K_e is then staged in LDS (lane
+// (a, b) holds half of block (a, b) and half of (b, a)) and
 // written as whole 6 x 6 blocks, consecutive lanes on consecutive entries
 // of a block: plain stores (first element of the colour order to touch the
 // block) and FP64 adds without return.  In the colour-ordered launches no
@@ -536,51 +548,49 @@ __global__ void __launch_bounds__(64)
 // launch sequence and the sum is deterministic; the uncoloured entry point
 // adds in any order.
 constexpr int kMfmaElems = 4;  // elements per wavefront (MFMA blocks)
+// doubles from one 6 x 6 block to the next in LDS: with 36 the 16 blocks of an
+// element would start on 8 of the 32 pairs of banks
+constexpr int kBlkStride = 37;
 
-struct ElemMfma {
+struct ElemData {
   double X[12];
   double u[24];
   double data[4];
-  union {
-    struct {
-      mitc4::Geom g;
-      mitc4::BColumnPrep prep[24];  // quadrature-independent column parts
-    };
-    double Ke[24][25];  // padded rows
-  };
+  double fn[4][3], dv[4][3], dw[4][3];
+};
+union ElemMfma {
+  ElemData d;
+  double Ke[16 * kBlkStride];  // block 4a + b, row-major 6 x 6
 };
 
-// Lane layout of v_mfma_f64_4x4x4_4b_f64 on gfx950 (measured): the block of
-// lane L is (L / 4) % 4; its A operand is A[L % 4][L / 16], its B operand
-// B[L / 16][L % 4] and its result D[L / 16][L % 4].  With the index
-// l16 = L % 4 + 4 (L / 16) inside the block, a lane's A row, B column and
-// D column are l16 % 4 and its k index and D row l16 / 4.
-__device__ __forceinline__ int mfma_d_row(int l16) { return l16 >> 2; }
-__device__ __forceinline__ int mfma_d_col(int l16) { return l16 & 3; }
-
-// Row s of detXd C (stress of a2d/a2disotropicshellstress.h:13-51) applied
-// to the strain column e[0..8].
+// detXd C (stress of a2d/a2disotropicshellstress.h:13-51) applied to the
+// strain column e[0..8]; the weight of the point is in the moduli.
 struct StressRows {
-  double Q0, Q1, G, am, ab, ad, As;
-  __device__ __forceinline__ void init(const double d[4]) {
+  double m0, m1, mg, b0, b1, bg, d0, d1, dg, As;
+  __device__ __forceinline__ void init(const double d[4], double sc) {
     const double E = d[0], nu = d[1], t = d[2], to = d[3];
-    const double D = E / (1.0 - nu * nu);
-    Q0 = D;
-    Q1 = nu * D;
-    G = E / 2.0 / (1.0 + nu);
-    am = t;
-    ab = -t * t * to;
-    ad = t * t * t / 12.0 + t * t * t * to * to;
-    As = (5.0 / 6.0) * t * G;
+    const double Q0 = E / (1.0 - nu * nu), G = E / 2.0 / (1.0 + nu);
+    const double am = sc * t, ab = -sc * t * t * to;
+    const double ad = sc * (t * t * t / 12.0 + t * t * t * to * to);
+    m0 = am * Q0;
+    m1 = am * (nu * Q0);
+    mg = am * G;
+    b0 = ab * Q0;
+    b1 = ab * (nu * Q0);
+    bg = ab * G;
+    d0 = ad * Q0;
+    d1 = ad * (nu * Q0);
+    dg = ad * G;
+    As = sc * ((5.0 / 6.0) * t * G);
   }
   __device__ __forceinline__ double row(int s, const double e[9]) const {
     switch (s) {
-      case 0: return am * (Q0 * e[0] + Q1 * e[1]) + ab * (Q0 * e[3] + Q1 * e[4]);
-      case 1: return am * (Q1 * e[0] + Q0 * e[1]) + ab * (Q1 * e[3] + Q0 * e[4]);
-      case 2: return am * (G * e[2]) + ab * (G * e[5]);
-      case 3: return ab * (Q0 * e[0] + Q1 * e[1]) + ad * (Q0 * e[3] + Q1 * e[4]);
-      case 4: return ab * (Q1 * e[0] + Q0 * e[1]) + ad * (Q1 * e[3] + Q0 * e[4]);
-      case 5: return ab * (G * e[2]) + ad * (G * e[5]);
+      case 0: return m0 * e[0] + m1 * e[1] + b0 * e[3] + b1 * e[4];
+      case 1: return m1 * e[0] + m0 * e[1] + b1 * e[3] + b0 * e[4];
+      case 2: return mg * e[2] + bg * e[5];
+      case 3: return b0 * e[0] + b1 * e[1] + d0 * e[3] + d1 * e[4];
+      case 4: return b1 * e[0] + b0 * e[1] + d1 * e[3] + d0 * e[4];
+      case 5: return bg * e[2] + dg * e[5];
       case 6: return As * e[6];
       case 7: return As * e[7];
       default: return 10.0 * As * e[8];
@@ -591,6 +601,228 @@ struct StressRows {
 #ifndef GPUFEM_MFMA_MINWAVES
 #define GPUFEM_MFMA_MINWAVES 2
 #endif
+// A lane's place in the four-elements-per-wavefront layout.  Lane layout of
+// v_mfma_f64_4x4x4_4b_f64 on gfx950 (measured): the block of lane L is
+// (L / 4) % 4; its A operand is A[L % 4][L / 16], its B operand
+// B[L / 16][L % 4] and its result D[L / 16][L % 4].  So a lane forms the
+// columns of node a = L % 4 at point q = L / 16, and receives node block
+// (q, a) of the product.  Blocks past the last element take element 0's
+// data, and nothing of theirs is written.
+struct MfmaLane {
+  int grp, a, q, slot, e, node;
+  bool valid;
+  __device__ __forceinline__ MfmaLane(int nelems, const int* elem_list,
+                                      const int* conn) {
+    const int lane = threadIdx.x;
+    grp = (lane >> 2) & 3;
+    a = lane & 3;
+    q = lane >> 4;
+    slot = blockIdx.x * kMfmaElems + grp;
+    valid = slot < nelems;
+    e = !valid ? 0 : elem_list ? elem_list[slot] : slot;
+    node = conn[4 * (size_t)e + a];
+  }
+};
+
+// Sum over the four lanes of a quad (the nodes of an element at one point).
+template <int kCtrl>
+__device__ __forceinline__ double quad_perm(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, kCtrl, 0xf, 0xf, true);
+  const int hi =
+      __builtin_amdgcn_mov_dpp((int)(b >> 32), kCtrl, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double quad_sum(double v) {
+  v += quad_perm<0xb1>(v);         // lanes 1, 0, 3, 2
+  return v + quad_perm<0x4e>(v);   // lanes 2, 3, 0, 1
+}
+// Sum over the four points of an element (lanes 16 apart).
+__device__ __forceinline__ double point_sum(double v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// The lane's columns and what else the kernels need of its node and point.
+struct LaneColumns {
+  double B[6][9];
+  double nf[3];
+  mitc4::NodePoint np;
+  StressRows C;
+};
+__device__ __forceinline__ void mfma_columns(ElemData& s, const MfmaLane& L,
+                                             const double* xpts,
+                                             const double* vars,
+                                             const double* data,
+                                             LaneColumns& c) {
+  if (L.q < 3) s.X[3 * L.a + L.q] = xpts[3 * (size_t)L.node + L.q];
+  if (vars) {
+    s.u[6 * L.a + L.q] = vars[6 * (size_t)L.node + L.q];
+    if (L.q < 2) s.u[6 * L.a + 4 + L.q] = vars[6 * (size_t)L.node + 4 + L.q];
+  }
+  if (L.q == 3) s.data[L.a] = data[4 * (size_t)L.e + L.a];
+  __syncthreads();
+  double nd[3], dv[3], dw[3];
+  mitc4::node_frame(L.a, s.X, c.nf, nd, dv, dw);
+  if (L.q == 0) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      s.fn[L.a][k] = c.nf[k];
+      s.dv[L.a][k] = dv[k];
+      s.dw[L.a][k] = dw[k];
+    }
+  }
+  __syncthreads();
+  double A[9], Z[9], T[6];
+  c.C.init(s.data, mitc4::quad_frame(L.q, s.X, s.fn, A, Z, T));
+  c.np.init(L.a, L.q, A, Z);
+  mitc4::node_columns_q(L.a, L.q, s.X, s.fn, s.dv, s.dw, c.nf, nd, A, T, c.np,
+                        c.B);
+}
+
+// Upper tiles of K_e: acc[t] of lane (q, a) is K_e[6q + I][6a + J].
+__device__ __forceinline__ void mfma_product(const LaneColumns& c,
+                                             double (&acc)[21]) {
+#pragma unroll
+  for (int t = 0; t < 21; t++) acc[t] = 0.0;
+#pragma unroll
+  for (int st = 0; st < 9; st++) {
+    double d[6];
+#pragma unroll
+    for (int J = 0; J < 6; J++) d[J] = c.C.row(st, c.B[J]);
+    int t = 0;
+#pragma unroll
+    for (int I = 0; I < 6; I++)
+#pragma unroll
+      for (int J = I; J < 6; J++, t++)
+        acc[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(c.B[I][st], d[J], acc[t],
+                                                    0, 0, 0);
+  }
+}
+
+// K_e of the wavefront's elements: staged in LDS (over the element data) and
+// added to its blocks.
+template <bool kColored>
+__device__ __forceinline__ void mfma_scatter(ElemMfma* S, const MfmaLane& L,
+                                             const double (&acc)[21],
+                                             int nelems, int own_dst,
+                                             int* s_dst, double* kvals) {
+  __syncthreads();  // element data no longer read
+  {
+    s_dst[16 * L.grp + 4 * L.q + L.a] = own_dst;
+    double* k1 = &S[L.grp].Ke[kBlkStride * (4 * L.q + L.a)];
+    double* k2 = &S[L.grp].Ke[kBlkStride * (4 * L.a + L.q)];
+    int t = 0;
+#pragma unroll
+    for (int I = 0; I < 6; I++)
+#pragma unroll
+      for (int J = I; J < 6; J++, t++) {
+        k1[6 * I + J] = acc[t];
+        if (J != I) k2[6 * J + I] = acc[t];
+      }
+  }
+  __syncthreads();
+  // entry rc of block nb of the wavefront's 64, 64 entries further each time
+  const int nblk = 16 * min(kMfmaElems, nelems - (int)blockIdx.x * kMfmaElems);
+  const double* ke = &S[0].Ke[0];
+  int nb = threadIdx.x >= 36, rc = (int)threadIdx.x - 36 * nb;
+#pragma unroll 4
+  for (int it = 0; it < 36; it++) {
+    if (nb < nblk) {
+      const double v = ke[kBlkStride * nb + rc];
+      const int dst = s_dst[nb];
+      // colour-ordered: no other element of this launch touches the block,
+      // so the add without return is ordered by the launches alone (the same
+      // sum, bit for bit, as a read-add-write, without the read's latency)
+      if (kColored && dst < 0)
+        kvals[36 * (size_t)~dst + rc] = v;
+      else
+        unsafeAtomicAdd(&kvals[36 * (size_t)dst + rc], v);
+    }
+    nb += 1;
+    rc += 28;
+    if (rc >= 36) {
+      rc -= 36;
+      nb += 1;
+    }
+  }
+}
+
+// Where block 4q + a of the lane's element goes: its block of K,
+// complemented if the element is the first to touch it.
+template <bool kColored>
+__device__ __forceinline__ int mfma_dst(const MfmaLane& L,
+                                        const int* elem_ind_map, int mask) {
+  const int ab = 4 * L.q + L.a;
+  const int b = elem_ind_map[16 * (size_t)L.e + ab];
+  return kColored && ((mask >> ab) & 1) ? ~b : b;
+}
+
+// B u of the lane's point and its stress, detXd C (B u).
+__device__ __forceinline__ void point_strain(const ElemData& s,
+                                             const MfmaLane& L,
+                                             const LaneColumns& c,
+                                             double (&E)[9]) {
+#pragma unroll
+  for (int st = 0; st < 9; st++) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < 6; k++) v += c.B[k][st] * s.u[6 * L.a + k];
+    E[st] = quad_sum(v);
+  }
+}
+__device__ __forceinline__ void point_stress(const LaneColumns& c,
+                                             const double (&E)[9],
+                                             double (&St)[9]) {
+#pragma unroll
+  for (int st = 0; st < 9; st++) St[st] = c.C.row(st, E);
+}
+// Energy of the wavefront's elements.
+__device__ __forceinline__ void mfma_energy(const MfmaLane& L,
+                                            const double (&E)[9],
+                                            const double (&St)[9],
+                                            double* energy) {
+  double es = 0.0;
+#pragma unroll
+  for (int st = 0; st < 9; st++) es += E[st] * St[st];
+  es = wave_sum(L.valid && L.a == 0 ? 0.5 * es : 0.0);
+  if (threadIdx.x == 0) unsafeAtomicAdd(energy, es);
+}
+// R_e = sum_q B_q^T S_q into res: point q's lanes write DOFs q and 4 + q.
+template <bool kColored>
+__device__ __forceinline__ void mfma_residual(const MfmaLane& L,
+                                              const LaneColumns& c,
+                                              const double (&St)[9],
+                                              const int* perm, int mask,
+                                              double* res) {
+  double own[2] = {0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    double v = 0.0;
+#pragma unroll
+    for (int st = 0; st < 9; st++) v += c.B[k][st] * St[st];
+    v = point_sum(v);
+    if (k % 4 == L.q) own[k / 4] = v;
+  }
+  if (!L.valid) return;
+  const int row = perm ? perm[L.node] : L.node;
+  const bool first = kColored && ((mask >> (16 + L.a)) & 1);
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int k = 4 * h + L.q;
+    if (k >= 6) continue;
+    double* d = &res[6 * (size_t)row + k];
+    if (!kColored)
+      unsafeAtomicAdd(d, own[h]);
+    else
+      *d = first ? own[h] : *d + own[h];
+  }
+}
+
 template <bool kColored>
 __global__ void __launch_bounds__(64, GPUFEM_MFMA_MINWAVES)
     jacobian_mfma_kernel(int nelems, const int* __restrict__ elem_list,
@@ -603,128 +835,24 @@ __global__ void __launch_bounds__(64, GPUFEM_MFMA_MINWAVES)
                          const int* __restrict__ perm, double* kvals,
                          double* res) {
   __shared__ ElemMfma S[kMfmaElems];
-  __shared__ int s_blk[kMfmaElems][16];
-  __shared__ int s_mask[kMfmaElems];
-  const int lane = threadIdx.x;
-  // MFMA block (element) of the lane and its index 0..15 inside the block
-  const int grp = (lane >> 2) & 3, l16 = (lane & 3) | ((lane >> 4) << 2);
-  const int slot = blockIdx.x * kMfmaElems + grp;
-  const bool valid = slot < nelems;
-  const int e = valid ? (kColored ? elem_list[slot] : slot) : 0;
-  ElemMfma& s = S[grp];
-  if (valid) {
-    for (int v = l16; v < 40; v += 16) {
-      if (v < 12) {
-        s.X[v] = xpts[3 * (size_t)conn[4 * (size_t)e + v / 3] + v % 3];
-      } else if (v < 36) {
-        const int w = v - 12;
-        s.u[w] = vars ? vars[6 * (size_t)conn[4 * (size_t)e + w / 6] + w % 6]
-                      : 0.0;
-      } else {
-        s.data[v - 36] = data[4 * (size_t)e + (v - 36)];
-      }
-    }
-    s_blk[grp][l16] = elem_ind_map[16 * (size_t)e + l16];
-    if (l16 == 0) s_mask[grp] = kColored ? first_mask[slot] : 0;
-  }
-  __syncthreads();
-  if (valid) {
-    if (l16 < 4)
-      mitc4::geom_node(l16, s.X, s.g);
-    else if (l16 < 9)
-      mitc4::geom_tying_x(l16 - 4, s.X, s.g);
-  }
-  __syncthreads();
-  if (valid) {
-    if (l16 < 4)
-      mitc4::geom_quad(l16, s.X, s.g);
-    else if (l16 < 9)
-      mitc4::geom_tying_n(l16 - 4, s.g);
-  }
-  __syncthreads();
-  // the quadrature-independent part of each column, once per column
-  if (valid)
-    for (int j = l16; j < 24; j += 16) mitc4::b_column_prep(j, s.g, s.prep[j]);
-  __syncthreads();
-  // B_q columns j = i + 4J of this lane's quadrature point q, all 9 strains
-  const int i = l16 & 3, q = (l16 >> 2) & 3;
-  double Bv[6][9];
-  StressRows C{0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  double sc = 0.0;
-  if (valid) {
-    C.init(s.data);
-    sc = s.g.scale[q];
+  __shared__ int s_dst[16 * kMfmaElems];
+  const MfmaLane L(nelems, kColored ? elem_list : nullptr, conn);
+  ElemData& s = S[L.grp].d;
+  const int mask = kColored && L.valid ? first_mask[L.slot] : 0;
+  const int dst = mfma_dst<kColored>(L, elem_ind_map, mask);
+  LaneColumns c;
+  mfma_columns(s, L, xpts, vars, data, c);
+  if (res) {  // uniform; vars null: u = 0
+    double E[9], St[9];
 #pragma unroll
-    for (int J = 0; J < 6; J++)
-      mitc4::b_column_q(i + 4 * J, q, s.g, s.prep[i + 4 * J], Bv[J]);
-  } else {
-    // a block past the last element: zeros in, results discarded
-#pragma unroll
-    for (int J = 0; J < 6; J++)
-#pragma unroll
-      for (int k = 0; k < 9; k++) Bv[J][k] = 0.0;
+    for (int st = 0; st < 9; st++) E[st] = 0.0;
+    if (vars) point_strain(s, L, c, E);
+    point_stress(c, E, St);
+    mfma_residual<kColored>(L, c, St, perm, mask, res);
   }
-  // 21 tiles (I <= J) of the 6 x 6 grid of 4 x 4 tiles
   double acc[21];
-#pragma unroll
-  for (int t = 0; t < 21; t++) acc[t] = 0.0;
-#pragma unroll
-  for (int st = 0; st < 9; st++) {
-    double dv[6];
-#pragma unroll
-    for (int J = 0; J < 6; J++) dv[J] = sc * C.row(st, Bv[J]);
-    int t = 0;
-#pragma unroll
-    for (int I = 0; I < 6; I++)
-#pragma unroll
-      for (int J = I; J < 6; J++, t++)
-        acc[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(Bv[I][st], dv[J], acc[t],
-                                                    0, 0, 0);
-  }
-  __syncthreads();  // geometry no longer read: Ke reuses its LDS
-  if (valid) {
-    const int dr = mfma_d_row(l16), dc = mfma_d_col(l16);
-    int t = 0;
-#pragma unroll
-    for (int I = 0; I < 6; I++)
-#pragma unroll
-      for (int J = I; J < 6; J++, t++) {
-        s.Ke[4 * I + dr][4 * J + dc] = acc[t];
-        if (J != I) s.Ke[4 * J + dc][4 * I + dr] = acc[t];
-      }
-  }
-  __syncthreads();
-  // whole 6 x 6 blocks: entry f of the wavefront's 4 x 16 x 36 block values
-#pragma unroll 4
-  for (int f = lane; f < kMfmaElems * 576; f += 64) {
-    const int g = f / 576, rem = f % 576, ab = rem / 36, rc = rem % 36;
-    if (blockIdx.x * kMfmaElems + g >= nelems) continue;
-    const int a = ab >> 2, b = ab & 3, r = rc / 6, c = rc % 6;
-    const double v = S[g].Ke[6 * a + r][6 * b + c];
-    double* d = kvals + 36 * (size_t)s_blk[g][ab] + rc;
-    // colour-ordered: no other element of this launch touches the block,
-    // so the add without return is ordered by the launches alone (the same
-    // sum, bit for bit, as a read-add-write, without the read's latency)
-    if (kColored && ((s_mask[g] >> ab) & 1))
-      *d = v;
-    else
-      unsafeAtomicAdd(d, v);
-  }
-  if (!res) return;  // uniform across the workgroup
-  if (valid) {
-    for (int row = l16; row < 24; row += 16) {
-      double v = 0.0;
-#pragma unroll
-      for (int c = 0; c < 24; c++) v += s.Ke[row][c] * s.u[c];
-      const int node = conn[4 * (size_t)e + row / 6];
-      const int prow = perm ? perm[node] : node;
-      double* d = &res[6 * (size_t)prow + row % 6];
-      if (!kColored)
-        unsafeAtomicAdd(d, v);
-      else
-        *d = ((s_mask[grp] >> (16 + row / 6)) & 1) ? v : *d + v;
-    }
-  }
+  mfma_product(c, acc);
+  mfma_scatter<kColored>(S, L, acc, nelems, dst, s_dst, kvals);
 }
 
 // ---------------------------------------------------------------------------
@@ -736,7 +864,7 @@ __global__ void __launch_bounds__(64, GPUFEM_MFMA_MINWAVES)
 //   e5 += u0x(:,0).u1x(:,1) + u1x(:,0).u0x(:,1);
 // the tying strains and the director stay linear (physics.h:214-219,
 // 286-300).  With G0, G1 the maps of the element DOFs to the entries
-// (r, c < 2) of u0x, u1x (mitc4::grad_columns_q), B_q(u) = dE_q/du and
+// (r, c < 2) of u0x, u1x (mitc4::NodePoint), B_q(u) = dE_q/du and
 // S_q = detXd_q C E_q(u):
 //   R_e(u) = sum_q B_q(u)^T S_q                         (the gradient of
 //   U = sum_q 1/2 detXd_q E^T C E, physics.h:18-36),
@@ -746,29 +874,22 @@ __global__ void __launch_bounds__(64, GPUFEM_MFMA_MINWAVES)
 // reference's own nonlinear Jacobian routes its displacement gradients'
 // second-order terms into the residual, elem_group.h:286-289, and
 // overwrites the u0x sensitivity with the u1x one, basis.h:565-567.)
-// One element per 64-lane workgroup; per quadrature point lanes 0-23 form
-// column j of the linear B, G0 and G1 into LDS, 21 lanes form B u, G0 u and
-// G1 u, lane 0 the strain and stress, lanes 0-23 the column of B(u), C B(u)
-// and of W G1, W G0, and every lane adds a 3x3 tile of K_e.  Scatter as in
-// jacobian_kernel; R_e into res (6 perm[node] + k), the energy into
-// *energy; kvals, res or energy may be null.
-struct ElemNL {
-  double X[12];
-  double u[24];
-  double data[4];
-  mitc4::Geom g;
-  double B[9][24];   // B_q(u)
-  double D[9][24];   // detXd C B_q(u)
-  double G0[6][24];
-  double G1[6][24];
-  double P0[6][24];  // W G1
-  double P1[6][24];  // W G0
-  double eu[21];     // B_lin u, u0x entries, u1x entries
-  double S[9];       // detXd C E(u)
-};
-
+// Layout and scatter as in jacobian_mfma_kernel; R_e into res (6 perm[node] +
+// k), the energy into *energy; kvals, res or energy may be null.
+// All entries of G0 and G1 of node a are t_r[k] or (fn_a x t_r)[k] times the
+// four pairs of scalars of NodePoint, and the t_r are orthonormal: sums over
+// r of products of gradient entries do not need the frame.  With D_c the global vectors sum_a su_c u_a +
+// ru_c (q_a x fn_a) of u0x (and of sz, rz for u1x), sum_r u0x_rc u1x_rc' =
+// D0_c . D1_c'; the columns of B(u) take D0 and D1 alone; and the last two
+// terms of K_e are, for nodes a and b, three scalars
+//   SS, SR, RR = sum_q sum_c (pu_c (W pz)_c + pz_c (W pu)_c),  p = s or r,
+// times I, the cross-product matrix of fn_b and (fn_a . fn_b) I - fn_b fn_a^T:
+// 12 MFMAs instead of the 252 of the 24 x 24 x 48 product.
+// 131,328-node cylinder (131,072 elements), colour-ordered K and R: 3.31 ms
+// with one element a wavefront and 3 x 3 tiles through LDS, 0.47 ms so (the
+// four colours 85, 150, 100 and 136 us; bound as jacobian_mfma_kernel).
 template <bool kColored>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64, GPUFEM_MFMA_MINWAVES)
     tangent_kernel(int nelems, const int* __restrict__ elem_list,
                    const int* __restrict__ first_mask,
                    const int* __restrict__ conn,
@@ -778,224 +899,125 @@ __global__ void __launch_bounds__(64)
                    const int* __restrict__ elem_ind_map,
                    const int* __restrict__ perm, double* kvals, double* res,
                    double* energy) {
-  __shared__ ElemNL s;
-  if ((int)blockIdx.x >= nelems) return;
-  const int e = kColored ? elem_list[blockIdx.x] : (int)blockIdx.x;
-  const int mask = kColored ? first_mask[blockIdx.x] : 0;
-  const int lane = threadIdx.x;
-  if (lane < 12) {
-    s.X[lane] = xpts[3 * (size_t)conn[4 * (size_t)e + lane / 3] + lane % 3];
-  } else if (lane < 36) {
-    const int i = lane - 12;
-    s.u[i] = vars[6 * (size_t)conn[4 * (size_t)e + i / 6] + i % 6];
-  } else if (lane < 40) {
-    s.data[lane - 36] = data[4 * (size_t)e + (lane - 36)];
+  __shared__ ElemMfma S[kMfmaElems];
+  __shared__ int s_dst[16 * kMfmaElems];
+  const MfmaLane L(nelems, kColored ? elem_list : nullptr, conn);
+  ElemData& s = S[L.grp].d;
+  const int mask = kColored && L.valid ? first_mask[L.slot] : 0;
+  const int dst = kvals ? mfma_dst<kColored>(L, elem_ind_map, mask) : 0;
+  LaneColumns c;
+  mfma_columns(s, L, xpts, vars, data, c);
+  double E[9], St[9];
+  point_strain(s, L, c, E);
+  const mitc4::NodePoint& np = c.np;
+  {
+    double D0[2][3], D1[2][3];  // global gradient vectors of u0x, u1x
+    const double* u = &s.u[6 * L.a];
+    const double th[3] = {u[3], u[4], u[5]};
+    double d[3];
+    mitc4::cross(th, c.nf, d);
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+      for (int m = 0; m < 2; m++) {
+        D0[m][k] = quad_sum(np.su[m] * u[k] + np.ru[m] * d[k]);
+        D1[m][k] = quad_sum(np.sz[m] * u[k] + np.rz[m] * d[k]);
+      }
+    E[3] += mitc4::dot3(D0[0], D1[0]);
+    E[4] += mitc4::dot3(D0[1], D1[1]);
+    E[5] += mitc4::dot3(D0[0], D1[1]) + mitc4::dot3(D1[0], D0[1]);
+    // dE/du: the quadratic terms' derivative, per DOF of node a
+    double w[3][3], v[3][3];  // rows 3..5, displacements and directors
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      w[0][k] = np.su[0] * D1[0][k] + np.sz[0] * D0[0][k];
+      w[1][k] = np.su[1] * D1[1][k] + np.sz[1] * D0[1][k];
+      w[2][k] = np.su[0] * D1[1][k] + np.sz[1] * D0[0][k] +
+                np.sz[0] * D0[1][k] + np.su[1] * D1[0][k];
+      v[0][k] = np.ru[0] * D1[0][k] + np.rz[0] * D0[0][k];
+      v[1][k] = np.ru[1] * D1[1][k] + np.rz[1] * D0[1][k];
+      v[2][k] = np.ru[0] * D1[1][k] + np.rz[1] * D0[0][k] +
+                np.rz[0] * D0[1][k] + np.ru[1] * D1[0][k];
+    }
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+      double f[3];
+      mitc4::cross(c.nf, v[m], f);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        c.B[k][3 + m] += w[m][k];
+        c.B[3 + k][3 + m] += f[k];
+      }
+    }
   }
-  __syncthreads();
-  if (lane < 4)
-    mitc4::geom_node(lane, s.X, s.g);
-  else if (lane < 9)
-    mitc4::geom_tying_x(lane - 4, s.X, s.g);
-  __syncthreads();
-  if (lane < 4)
-    mitc4::geom_quad(lane, s.X, s.g);
-  else if (lane < 9)
-    mitc4::geom_tying_n(lane - 4, s.g);
-  __syncthreads();
-  mitc4::BColumnPrep prep;
-  if (lane < 24) mitc4::b_column_prep(lane, s.g, prep);
-  const int I = lane / 8, J = lane % 8;
-  double acc[3][3];
+  point_stress(c, E, St);
+  if (energy) mfma_energy(L, E, St, energy);  // uniform
+  if (res) mfma_residual<kColored>(L, c, St, perm, mask, res);
+  if (!kvals) return;  // uniform across the workgroup
+  double acc[21];
+  mfma_product(c, acc);
+  double ss = 0.0, sr = 0.0, rr = 0.0;
 #pragma unroll
-  for (int r = 0; r < 3; r++)
-#pragma unroll
-    for (int c = 0; c < 3; c++) acc[r][c] = 0.0;
-  double racc = 0.0, uacc = 0.0;
-#pragma unroll 1
-  for (int q = 0; q < 4; q++) {
-    const double sc = s.g.scale[q];
-    // linear B column and the gradient maps of DOF lane
-    double col[9], g0[6], g1[6];
-    if (lane < 24) {
-      mitc4::b_column_q(lane, q, s.g, prep, col);
-      mitc4::grad_columns_q(lane, q, s.g, g0, g1);
-#pragma unroll
-      for (int k = 0; k < 9; k++) s.B[k][lane] = col[k];
-#pragma unroll
-      for (int m = 0; m < 6; m++) {
-        s.G0[m][lane] = g0[m];
-        s.G1[m][lane] = g1[m];
-      }
-    }
-    __syncthreads();
-    if (lane < 21) {
-      const double* row = lane < 9 ? s.B[lane]
-                          : lane < 15 ? s.G0[lane - 9] : s.G1[lane - 15];
-      double v = 0.0;
-#pragma unroll
-      for (int j = 0; j < 24; j++) v += row[j] * s.u[j];
-      s.eu[lane] = v;
-    }
-    __syncthreads();
-    if (lane == 0) {
-      const double* U0 = &s.eu[9];
-      const double* U1 = &s.eu[15];
-      double E[9], st[9];
-#pragma unroll
-      for (int k = 0; k < 9; k++) E[k] = s.eu[k];
-      E[3] += U0[0] * U1[0] + U0[2] * U1[2] + U0[4] * U1[4];
-      E[4] += U0[1] * U1[1] + U0[3] * U1[3] + U0[5] * U1[5];
-      E[5] += U0[0] * U1[1] + U0[2] * U1[3] + U0[4] * U1[5] +
-              U1[0] * U0[1] + U1[2] * U0[3] + U1[4] * U0[5];
-      mitc4::stress(s.data, E, st);
-      double es = 0.0;
-#pragma unroll
-      for (int k = 0; k < 9; k++) {
-        s.S[k] = sc * st[k];
-        es += E[k] * st[k];
-      }
-      uacc += 0.5 * sc * es;
-    }
-    __syncthreads();
-    if (lane < 24) {
-      const double* U0 = &s.eu[9];
-      const double* U1 = &s.eu[15];
-      // dE/du_lane: the linear column plus the quadratic terms' derivative
-#pragma unroll
-      for (int r = 0; r < 3; r++) {
-        col[3] += g0[2 * r] * U1[2 * r] + U0[2 * r] * g1[2 * r];
-        col[4] += g0[2 * r + 1] * U1[2 * r + 1] + U0[2 * r + 1] * g1[2 * r + 1];
-        col[5] += g0[2 * r] * U1[2 * r + 1] + U0[2 * r] * g1[2 * r + 1] +
-                  g1[2 * r] * U0[2 * r + 1] + U1[2 * r] * g0[2 * r + 1];
-      }
-      double st[9];
-      mitc4::stress(s.data, col, st);
-      double rv = 0.0;
-#pragma unroll
-      for (int k = 0; k < 9; k++) {
-        s.B[k][lane] = col[k];
-        s.D[k][lane] = sc * st[k];
-        rv += col[k] * s.S[k];
-      }
-      racc += rv;
-      const double S3 = s.S[3], S4 = s.S[4], S5 = s.S[5];
-#pragma unroll
-      for (int r = 0; r < 3; r++) {
-        s.P0[2 * r][lane] = S3 * g1[2 * r] + S5 * g1[2 * r + 1];
-        s.P0[2 * r + 1][lane] = S5 * g1[2 * r] + S4 * g1[2 * r + 1];
-        s.P1[2 * r][lane] = S3 * g0[2 * r] + S5 * g0[2 * r + 1];
-        s.P1[2 * r + 1][lane] = S5 * g0[2 * r] + S4 * g0[2 * r + 1];
-      }
-    }
-    __syncthreads();
-    if (kvals) {
-#pragma unroll
-      for (int r = 0; r < 3; r++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          const int i = 3 * I + r, j = 3 * J + c;
-          double v = 0.0;
-#pragma unroll
-          for (int k = 0; k < 9; k++) v += s.B[k][i] * s.D[k][j];
-#pragma unroll
-          for (int m = 0; m < 6; m++)
-            v += s.G0[m][i] * s.P0[m][j] + s.G1[m][i] * s.P1[m][j];
-          acc[r][c] += v;
-        }
-    }
-    __syncthreads();
+  for (int m = 0; m < 2; m++) {
+    const double w0 = m ? St[5] : St[3], w1 = m ? St[4] : St[5];
+    const double wsz = w0 * np.sz[0] + w1 * np.sz[1];
+    const double wsu = w0 * np.su[0] + w1 * np.su[1];
+    const double wrz = w0 * np.rz[0] + w1 * np.rz[1];
+    const double wru = w0 * np.ru[0] + w1 * np.ru[1];
+    ss = __builtin_amdgcn_mfma_f64_4x4x4f64(np.su[m], wsz, ss, 0, 0, 0);
+    sr = __builtin_amdgcn_mfma_f64_4x4x4f64(np.su[m], wrz, sr, 0, 0, 0);
+    rr = __builtin_amdgcn_mfma_f64_4x4x4f64(np.ru[m], wrz, rr, 0, 0, 0);
+    ss = __builtin_amdgcn_mfma_f64_4x4x4f64(np.sz[m], wsu, ss, 0, 0, 0);
+    sr = __builtin_amdgcn_mfma_f64_4x4x4f64(np.sz[m], wru, sr, 0, 0, 0);
+    rr = __builtin_amdgcn_mfma_f64_4x4x4f64(np.rz[m], wru, rr, 0, 0, 0);
   }
-  if (kvals) {
-    const int a = I / 2, b = J / 2, r0 = 3 * (I % 2), c0 = 3 * (J % 2);
-    double* dst =
-        kvals + 36 * (size_t)elem_ind_map[16 * (size_t)e + 4 * a + b];
-    const bool first = (mask >> (4 * a + b)) & 1;
+  // the lane's result is block (q, a): rows of node q, columns of node a
+  const double* fq = s.fn[L.q];
+  const double* fa = c.nf;
+  const double fqa = mitc4::dot3(fq, fa);
+  int t = 0;
 #pragma unroll
-    for (int r = 0; r < 3; r++)
+  for (int I = 0; I < 6; I++)
 #pragma unroll
-      for (int c = 0; c < 3; c++) {
-        double* d = &dst[6 * (r0 + r) + c0 + c];
-        if (!kColored)
-          unsafeAtomicAdd(d, acc[r][c]);
-        else
-          *d = first ? acc[r][c] : *d + acc[r][c];
+    for (int J = I; J < 6; J++, t++) {
+      if (J < 3) {
+        if (I == J) acc[t] += ss;
+      } else if (I < 3) {
+        // sum_r t_r[k] (fn x t_r)[l] = eps_lmk fn[m]
+        const int k = I, l = J - 3;
+        if (l == (k + 1) % 3) acc[t] += sr * fa[3 - k - l];
+        if (l == (k + 2) % 3) acc[t] -= sr * fa[3 - k - l];
+      } else {
+        const int k = I - 3, l = J - 3;
+        acc[t] += rr * ((k == l ? fqa : 0.0) - fa[k] * fq[l]);
       }
-  }
-  if (res && lane < 24) {
-    const int node = conn[4 * (size_t)e + lane / 6];
-    const int row = perm ? perm[node] : node;
-    double* d = &res[6 * (size_t)row + lane % 6];
-    if (!kColored)
-      unsafeAtomicAdd(d, racc);
-    else
-      *d = ((mask >> (16 + lane / 6)) & 1) ? racc : *d + racc;
-  }
-  if (energy && lane == 0) unsafeAtomicAdd(energy, uacc);
+    }
+  mfma_scatter<kColored>(S, L, acc, nelems, dst, s_dst, kvals);
 }
 
-// Residual only: R_e = sum_q D_q^T (B_q u) (C symmetric).
-__global__ void __launch_bounds__(64)
+// Residual, R_e = sum_q B_q^T (detXd C B_q u), or energy, U = sum_e sum_q 1/2
+// detXd (B_q u) . C (B_q u), in the layout of jacobian_mfma_kernel.
+// 131 x 257 cylinder (33,667 elements), residual: 197 us with one element a
+// wavefront and B and D through LDS, 31 us so.
+template <bool kEnergy>
+__global__ void __launch_bounds__(64, GPUFEM_MFMA_MINWAVES)
     residual_kernel(int nelems, const int* __restrict__ conn,
                     const double* __restrict__ xpts,
                     const double* __restrict__ vars,
                     const double* __restrict__ data,
-                    const int* __restrict__ perm, double* res) {
-  __shared__ ElemLDS s;
-  __shared__ double Eu[4][9];
-  const int e = blockIdx.x;
-  const int lane = threadIdx.x;
-  if (e >= nelems) return;
-  load_element(s, e, lane, conn, xpts, vars, data);
-  __syncthreads();
-  element_geometry(s, lane);
-  element_bd(s, lane);
-  if (lane < 36) {
-    const int q = lane / 9, k = lane % 9;
-    double acc = 0.0;
-    for (int j = 0; j < 24; j++) acc += s.B[q][k][j] * s.u[j];
-    Eu[q][k] = acc;
-  }
-  __syncthreads();
-  if (lane < 24) {
-    double r = 0.0;
-    for (int q = 0; q < 4; q++)
-#pragma unroll
-      for (int k = 0; k < 9; k++) r += s.D[q][k][lane] * Eu[q][k];
-    const int node = conn[4 * (size_t)e + lane / 6];
-    const int row = perm ? perm[node] : node;
-    unsafeAtomicAdd(&res[6 * (size_t)row + lane % 6], r);
-  }
-}
-
-// Energy U = sum_e sum_q 1/2 detXd (B_q u) . C (B_q u)
-__global__ void __launch_bounds__(64)
-    energy_kernel(int nelems, const int* __restrict__ conn,
-                  const double* __restrict__ xpts,
-                  const double* __restrict__ vars,
-                  const double* __restrict__ data, double* energy) {
-  __shared__ ElemLDS s;
-  __shared__ double Eu[4][9];
-  const int e = blockIdx.x;
-  const int lane = threadIdx.x;
-  if (e >= nelems) return;
-  load_element(s, e, lane, conn, xpts, vars, data);
-  __syncthreads();
-  element_geometry(s, lane);
-  element_bd(s, lane);
-  if (lane < 36) {
-    const int q = lane / 9, k = lane % 9;
-    double acc = 0.0;
-    for (int j = 0; j < 24; j++) acc += s.B[q][k][j] * s.u[j];
-    Eu[q][k] = acc;
-  }
-  __syncthreads();
-  if (lane < 4) {
-    double st[9];
-    mitc4::stress(s.data, Eu[lane], st);
-    double u = 0.0;
-    for (int k = 0; k < 9; k++) u += Eu[lane][k] * st[k];
-    unsafeAtomicAdd(energy, 0.5 * s.g.scale[lane] * u);
-  }
+                    const int* __restrict__ perm, double* out) {
+  __shared__ ElemData S[kMfmaElems];
+  const MfmaLane L(nelems, nullptr, conn);
+  ElemData& s = S[L.grp];
+  LaneColumns c;
+  mfma_columns(s, L, xpts, vars, data, c);
+  double E[9], St[9];
+  point_strain(s, L, c, E);
+  point_stress(c, E, St);
+  if constexpr (kEnergy)
+    mfma_energy(L, E, St, out);
+  else
+    mfma_residual<false>(L, c, St, perm, 0, out);
 }
 
 }  // namespace
@@ -1180,7 +1202,8 @@ int gf_assemble_tangent_mitc4_f64(gf_context ctx, int nelems, int nnodes,
   if (energy)
     GF_HIP(ctx, hipMemsetAsync(energy, 0, sizeof(double), ctx->stream));
   if (nelems == 0) return GF_OK;
-  hipLaunchKernelGGL(gf::tangent_kernel<false>, dim3(nelems), dim3(64), 0,
+  hipLaunchKernelGGL(gf::tangent_kernel<false>,
+                     dim3(gf::div_up(nelems, gf::kMfmaElems)), dim3(64), 0,
                      ctx->stream, nelems, (const int*)nullptr,
                      (const int*)nullptr, conn, xpts, vars, data, elem_ind_map,
                      perm, kvals, res, energy);
@@ -1203,7 +1226,8 @@ int gf_assemble_tangent_colored_f64(gf_context ctx, gf_asm_plan pl,
                                ctx->stream));
   for (int c = 0; c < pl->ncolors; c++) {
     const int c0 = pl->color_ptr[c], cnt = pl->color_ptr[c + 1] - c0;
-    hipLaunchKernelGGL(gf::tangent_kernel<true>, dim3(cnt), dim3(64), 0,
+    hipLaunchKernelGGL(gf::tangent_kernel<true>,
+                       dim3(gf::div_up(cnt, gf::kMfmaElems)), dim3(64), 0,
                        ctx->stream, cnt, pl->elems + c0, pl->mask + c0, conn,
                        xpts, vars, data, elem_ind_map, perm, kvals, res,
                        (double*)nullptr);
@@ -1219,7 +1243,8 @@ int gf_assemble_residual_mitc4_f64(gf_context ctx, int nelems, int nnodes,
       !data || !res)
     return gf::set_error(ctx, GF_ERR_INVALID, "assemble_residual: bad args");
   if (nelems == 0) return GF_OK;
-  hipLaunchKernelGGL(gf::residual_kernel, dim3(nelems), dim3(64), 0,
+  hipLaunchKernelGGL(gf::residual_kernel<false>,
+                     dim3(gf::div_up(nelems, gf::kMfmaElems)), dim3(64), 0,
                      ctx->stream, nelems, conn, xpts, vars, data, perm, res);
   return gf::check_launch(ctx, "residual_kernel");
 }
@@ -1231,8 +1256,10 @@ int gf_energy_mitc4_f64(gf_context ctx, int nelems, const int* conn,
     return gf::set_error(ctx, GF_ERR_INVALID, "energy: bad args");
   GF_HIP(ctx, hipMemsetAsync(energy, 0, sizeof(double), ctx->stream));
   if (nelems == 0) return GF_OK;
-  hipLaunchKernelGGL(gf::energy_kernel, dim3(nelems), dim3(64), 0,
-                     ctx->stream, nelems, conn, xpts, vars, data, energy);
+  hipLaunchKernelGGL(gf::residual_kernel<true>,
+                     dim3(gf::div_up(nelems, gf::kMfmaElems)), dim3(64), 0,
+                     ctx->stream, nelems, conn, xpts, vars, data,
+                     (const int*)nullptr, energy);
   return gf::check_launch(ctx, "energy_kernel");
 }
 

@@ -125,9 +125,10 @@ struct Geom {
   double scale[4];     // detXd * weight
 };
 
-// Node-point stage (one lane per node a = 0..3).
-__device__ __forceinline__ void geom_node(int a, const double X[12],
-                                          Geom& g) {
+// Normal and drill vectors of node a.
+__device__ __forceinline__ void node_frame(int a, const double X[12],
+                                           double fn[3], double dn[3],
+                                           double dv[3], double dw[3]) {
   const double xi = -1.0 + 2.0 * (a % 2), eta = -1.0 + 2.0 * (a / 2);
   double N[4], Nx[4], Ne[4];
   shape(xi, eta, N, Nx, Ne);
@@ -137,7 +138,6 @@ __device__ __forceinline__ void geom_node(int a, const double X[12],
       Xxi[k] += Nx[b] * X[3 * b + k];
       Xeta[k] += Ne[b] * X[3 * b + k];
     }
-  double fn[3];
   cross(Xxi, Xeta, fn);
   const double inv = 1.0 / sqrt(dot3(fn, fn));
   for (int k = 0; k < 3; k++) fn[k] *= inv;
@@ -151,14 +151,17 @@ __device__ __forceinline__ void geom_node(int a, const double X[12],
   inv3(Xd, Xdi);
   mm3(Xdi, T, W);
   const double t0[3] = {T[0], T[3], T[6]}, t1[3] = {T[1], T[4], T[7]};
-  double n[3];
-  cross(t0, t1, n);
+  cross(t0, t1, dn);
   for (int k = 0; k < 3; k++) {
-    g.fn[a][k] = fn[k];
-    g.dn[a][k] = n[k];
-    g.dv[a][k] = W[0] * t1[k] - W[1] * t0[k];
-    g.dw[a][k] = W[3] * t1[k] - W[4] * t0[k];
+    dv[k] = W[0] * t1[k] - W[1] * t0[k];
+    dw[k] = W[3] * t1[k] - W[4] * t0[k];
   }
+}
+
+// Node-point stage (one lane per node a = 0..3).
+__device__ __forceinline__ void geom_node(int a, const double X[12],
+                                          Geom& g) {
+  node_frame(a, X, g.fn[a], g.dn[a], g.dv[a], g.dw[a]);
 }
 
 // Tying-location stage, geometry part (lane per location l = 0..4).
@@ -190,9 +193,12 @@ __device__ __forceinline__ void geom_tying_n(int l, Geom& g) {
   }
 }
 
-// Quadrature-point stage (lane per point q = 0..3; needs node normals).
-__device__ __forceinline__ void geom_quad(int q, const double X[12],
-                                          Geom& g) {
+// Frame of quadrature point q (needs node normals): A = Xd^-1 T,
+// Z = -Xd^-1 Xdz Xd^-1 T, the first two columns of T; returns detXd * weight.
+__device__ __forceinline__ double quad_frame(int q, const double X[12],
+                                             const double (*fn)[3],
+                                             double A[9], double Z[9],
+                                             double T2[6]) {
   const double xi = (q % 2 == 0) ? -kRt3 : kRt3;
   const double eta = (q / 2 == 0) ? -kRt3 : kRt3;
   double N[4], Nx[4], Ne[4];
@@ -203,9 +209,9 @@ __device__ __forceinline__ void geom_quad(int q, const double X[12],
     for (int m = 0; m < 4; m++) {
       a += Nx[m] * X[3 * m + k];
       b += Ne[m] * X[3 * m + k];
-      c += N[m] * g.fn[m][k];
-      d += Nx[m] * g.fn[m][k];
-      e += Ne[m] * g.fn[m][k];
+      c += N[m] * fn[m][k];
+      d += Nx[m] * fn[m][k];
+      e += Ne[m] * fn[m][k];
     }
     Xxi[k] = a;
     Xeta[k] = b;
@@ -213,7 +219,7 @@ __device__ __forceinline__ void geom_quad(int q, const double X[12],
     nxi[k] = d;
     neta[k] = e;
   }
-  double Xd[9], Xdz[9], T[9], Xdi[9], A[9], tmp[9], Z[9];
+  double Xd[9], Xdz[9], T[9], Xdi[9], tmp[9];
   for (int i = 0; i < 3; i++) {
     Xd[3 * i] = Xxi[i];
     Xd[3 * i + 1] = Xeta[i];
@@ -227,31 +233,46 @@ __device__ __forceinline__ void geom_quad(int q, const double X[12],
   mm3(Xdi, T, A);
   mm3(Xdi, Xdz, tmp);
   mm3(tmp, A, Z);
-  for (int i = 0; i < 9; i++) {
-    g.A[q][i] = A[i];
-    g.Z[q][i] = -Z[i];
-  }
-  g.T[q][0] = T[0];
-  g.T[q][1] = T[3];
-  g.T[q][2] = T[6];
-  g.T[q][3] = T[1];
-  g.T[q][4] = T[4];
-  g.T[q][5] = T[7];
-  g.scale[q] = det * 1.0;
-  // e0ty(i,j) = A0i A0j g11 + A1i A1j g22 + (A0i A1j + A1i A0j) g12
-  //           + (A1i A2j + A2i A1j) g23 + (A0i A2j + A2i A0j) g13
+  for (int i = 0; i < 9; i++) Z[i] = -Z[i];
+  T2[0] = T[0];
+  T2[1] = T[3];
+  T2[2] = T[6];
+  T2[3] = T[1];
+  T2[4] = T[4];
+  T2[5] = T[7];
+  return det * 1.0;
+}
+
+// Row m of the map from the tying strains (g11, g22, g12, g23, g13) to the
+// tensor strains (E0, E1, E2, E6, E7):
+// e0ty(i,j) = A0i A0j g11 + A1i A1j g22 + (A0i A1j + A1i A0j) g12
+//           + (A1i A2j + A2i A1j) g23 + (A0i A2j + A2i A0j) g13
+__device__ __forceinline__ void tying_row(int m, const double A[9],
+                                          double c[5]) {
   const int ii[5] = {0, 1, 0, 1, 0}, jj[5] = {0, 1, 1, 2, 2};
   const double fac[5] = {1.0, 1.0, 2.0, 2.0, 2.0};
-  for (int m = 0; m < 5; m++) {
-    const int i = ii[m], j = jj[m];
-    const double A0i = A[i], A1i = A[3 + i], A2i = A[6 + i];
-    const double A0j = A[j], A1j = A[3 + j], A2j = A[6 + j];
-    g.coef[q][5 * m + 0] = fac[m] * A0i * A0j;
-    g.coef[q][5 * m + 1] = fac[m] * A1i * A1j;
-    g.coef[q][5 * m + 2] = fac[m] * (A0i * A1j + A1i * A0j);
-    g.coef[q][5 * m + 3] = fac[m] * (A1i * A2j + A2i * A1j);
-    g.coef[q][5 * m + 4] = fac[m] * (A0i * A2j + A2i * A0j);
+  const int i = ii[m], j = jj[m];
+  const double A0i = A[i], A1i = A[3 + i], A2i = A[6 + i];
+  const double A0j = A[j], A1j = A[3 + j], A2j = A[6 + j];
+  c[0] = fac[m] * A0i * A0j;
+  c[1] = fac[m] * A1i * A1j;
+  c[2] = fac[m] * (A0i * A1j + A1i * A0j);
+  c[3] = fac[m] * (A1i * A2j + A2i * A1j);
+  c[4] = fac[m] * (A0i * A2j + A2i * A0j);
+}
+
+// Quadrature-point stage (lane per point q = 0..3; needs node normals).
+__device__ __forceinline__ void geom_quad(int q, const double X[12],
+                                          Geom& g) {
+  double A[9], Z[9], T[6];
+  g.scale[q] = quad_frame(q, X, g.fn, A, Z, T);
+  for (int i = 0; i < 9; i++) {
+    g.A[q][i] = A[i];
+    g.Z[q][i] = Z[i];
   }
+  for (int i = 0; i < 6; i++) g.T[q][i] = T[i];
+#pragma unroll
+  for (int m = 0; m < 5; m++) tying_row(m, A, &g.coef[q][5 * m]);
 }
 
 // Shape function of node a and its derivatives at (xi, eta):
@@ -392,56 +413,127 @@ __device__ __forceinline__ void b_column_q(int j, int q, const Geom& g,
   out[8] = et;
 }
 
-// Column j of the local displacement gradients at quadrature point q, the
-// entries (r, c), c = 0, 1, of u0x = T^T [U_xi | U_eta | d0] Xd^-1 T and
-// u1x = T^T ([d0_xi | d0_eta | 0] Xd^-1 T + [U_xi | U_eta | d0] Z)
-// (basis.h:470-492), in the order (0,0) (0,1) (1,0) (1,1) (2,0) (2,1):
-//   displacement DOF (a, k):  u0x_rc = t_r[k] (N_a,xi A_0c + N_a,eta A_1c)
-//                             u1x_rc = t_r[k] (N_a,xi Z_0c + N_a,eta Z_1c)
-//   rotation DOF (a, k):      u0x_rc = (fn_a x t_r)[k] N_a A_2c
-//                             u1x_rc = (fn_a x t_r)[k] (N_a,xi A_0c +
-//                                       N_a,eta A_1c + N_a Z_2c)
-// with A = Xd^-1 T, Z = -Xd^-1 Xdz Xd^-1 T and t_r the columns of T
-// (d_a = q_a x fn_a, director.h:98-107).  Entries (0,0), (1,1), (0,1) + (1,0)
-// of u1x are the linear bending strains of b_column_q.
-__device__ __forceinline__ void grad_columns_q(int j, int q, const Geom& g,
-                                               double g0[6], double g1[6]) {
-  const int a = j / 6, k = j % 6;
-  const bool rot = k >= 3;
-  const int kk = rot ? k - 3 : k;
+// What the lane of (node a, quadrature point q) holds of that point.  The
+// local displacement gradients (basis.h:470-492)
+//   u0x = T^T [U_xi | U_eta | d0] Xd^-1 T
+//   u1x = T^T ([d0_xi | d0_eta | 0] Xd^-1 T + [U_xi | U_eta | d0] Z)
+// with d_a = q_a x fn_a (director.h:98-107) take from node a's displacement
+// DOFs  u0x_rc = t_r[k] su[c], u1x_rc = t_r[k] sz[c], and from its rotations
+// u0x_rc = (fn_a x t_r)[k] ru[c], u1x_rc = (fn_a x t_r)[k] rz[c], c = 0, 1.
+struct NodePoint {
+  double su[2], sz[2], ru[2], rz[2];
+  __device__ __forceinline__ void init(int a, int q, const double A[9],
+                                       const double Z[9]) {
+    const double xi = (q & 1) ? kRt3 : -kRt3;
+    const double eta = (q & 2) ? kRt3 : -kRt3;
+    double N, Nx, Ne;
+    shape_a(a, xi, eta, N, Nx, Ne);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      su[c] = Nx * A[c] + Ne * A[3 + c];
+      sz[c] = Nx * Z[c] + Ne * Z[3 + c];
+      ru[c] = N * A[6 + c];
+      rz[c] = Nx * A[c] + Ne * A[3 + c] + N * Z[6 + c];
+    }
+  }
+};
+
+// The six columns 6a + k of B_q of node a at quadrature point q:
+// out[k][s], s = 0..8 (the values of b_column_q).  fn, dv, dw: the node
+// normals and drill vectors of the element; nf, nd: node a's normal and drill
+// normal.
+__device__ __forceinline__ void node_columns_q(
+    int a, int q, const double X[12], const double (*fn)[3],
+    const double (*dv)[3], const double (*dw)[3], const double nf[3],
+    const double nd[3], const double A[9], const double T[6],
+    const NodePoint& np, double (&out)[6][9]) {
   const double xi = (q & 1) ? kRt3 : -kRt3;
   const double eta = (q & 2) ? kRt3 : -kRt3;
-  double Na, Nxa, Nea;
-  shape_a(a, xi, eta, Na, Nxa, Nea);
-  const double* A = g.A[q];
-  const double* Z = g.Z[q];
-  const double t0[3] = {g.T[q][0], g.T[q][1], g.T[q][2]};
-  const double t1[3] = {g.T[q][3], g.T[q][4], g.T[q][5]};
-  double t2[3];
-  cross(t0, t1, t2);  // the normal column of the orthonormal T
-  double f[3];        // t_r[k] or (fn_a x t_r)[k]
-  if (!rot) {
-    f[0] = t0[kk];
-    f[1] = t1[kk];
-    f[2] = t2[kk];
-  } else {
-    double c[3];
-    cross(g.fn[a], t0, c);
-    f[0] = c[kk];
-    cross(g.fn[a], t1, c);
-    f[1] = c[kk];
-    cross(g.fn[a], t2, c);
-    f[2] = c[kk];
+  const double hxm = 0.5 * (1.0 - xi), hxp = 0.5 * (1.0 + xi);
+  const double hem = 0.5 * (1.0 - eta), hep = 0.5 * (1.0 + eta);
+  double N[5], Nx[5], Ne[5];  // node a's shape functions at the tying points
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    double x, e;
+    tying_loc(l, x, e);
+    shape_a(a, x, e, N[l], Nx[l], Ne[l]);
+  }
+  // tangents and normals at the tying points, with the weights of their
+  // interpolation to q: g11 and g13 along eta, g22 and g23 along xi
+  double gt[3][5], gr[3][2];
+  double x0[3], x1[3], e2[3], e3[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    x0[k] = 0.5 * (X[3 + k] - X[k]);
+    x1[k] = 0.5 * (X[9 + k] - X[6 + k]);
+    e2[k] = 0.5 * (X[6 + k] - X[k]);
+    e3[k] = 0.5 * (X[9 + k] - X[3 + k]);
+    const double xm = 0.5 * (x0[k] + x1[k]), em = 0.5 * (e2[k] + e3[k]);
+    gt[k][0] = hem * (Nx[0] * x0[k]) + hep * (Nx[1] * x1[k]);
+    gt[k][1] = hxm * (Ne[2] * e2[k]) + hxp * (Ne[3] * e3[k]);
+    gt[k][2] = 0.5 * (Nx[4] * em + Ne[4] * xm);
+    const double n0 = 0.5 * (fn[0][k] + fn[1][k]);
+    const double n1 = 0.5 * (fn[2][k] + fn[3][k]);
+    const double n2 = 0.5 * (fn[0][k] + fn[2][k]);
+    const double n3 = 0.5 * (fn[1][k] + fn[3][k]);
+    gt[k][3] = hxm * (0.5 * Ne[2] * n2) + hxp * (0.5 * Ne[3] * n3);
+    gt[k][4] = hem * (0.5 * Nx[0] * n0) + hep * (0.5 * Nx[1] * n1);
+  }
+  {
+    double c2[3], c3[3];
+    cross(nf, e2, c2);
+    cross(nf, e3, c3);
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      gr[k][0] = hxm * (0.5 * N[2] * c2[k]) + hxp * (0.5 * N[3] * c3[k]);
+    cross(nf, x0, c2);
+    cross(nf, x1, c3);
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      gr[k][1] = hem * (0.5 * N[0] * c2[k]) + hep * (0.5 * N[1] * c3[k]);
   }
 #pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const double pa = rot ? Na * A[6 + c] : Nxa * A[c] + Nea * A[3 + c];
-    const double pz = rot ? Nxa * A[c] + Nea * A[3 + c] + Na * Z[6 + c]
-                          : Nxa * Z[c] + Nea * Z[3 + c];
+  for (int m = 0; m < 5; m++) {
+    double c[5];
+    tying_row(m, A, c);
+    const int row = m < 3 ? m : m + 3;
 #pragma unroll
-    for (int r = 0; r < 3; r++) {
-      g0[2 * r + c] = f[r] * pa;
-      g1[2 * r + c] = f[r] * pz;
+    for (int k = 0; k < 3; k++) {
+      out[k][row] = c[0] * gt[k][0] + c[1] * gt[k][1] + c[2] * gt[k][2] +
+                    c[3] * gt[k][3] + c[4] * gt[k][4];
+      out[3 + k][row] = c[3] * gr[k][0] + c[4] * gr[k][1];
+    }
+  }
+  // bending
+  {
+    const double t0[3] = {T[0], T[1], T[2]}, t1[3] = {T[3], T[4], T[5]};
+    double f0[3], f1[3];
+    cross(nf, t0, f0);
+    cross(nf, t1, f1);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      out[k][3] = np.sz[0] * t0[k];
+      out[k][4] = np.sz[1] * t1[k];
+      out[k][5] = np.sz[1] * t0[k] + np.sz[0] * t1[k];
+      out[3 + k][3] = np.rz[0] * f0[k];
+      out[3 + k][4] = np.rz[1] * f1[k];
+      out[3 + k][5] = np.rz[1] * f0[k] + np.rz[0] * f1[k];
+    }
+  }
+  // drill: N_a,xi at node b is +-1/2 for the two nodes b of a's eta row,
+  // N_a,eta for the two of its xi column
+  {
+    const double xa = (a & 1) ? 0.25 : -0.25, ea = (a & 2) ? 0.25 : -0.25;
+    const double wx = (a & 2) ? hep : hem, we = (a & 1) ? hxp : hxm;
+    const double vx0 = xa * (hxm * wx), vx1 = xa * (hxp * wx);
+    const double ve0 = ea * (we * hem), ve1 = ea * (we * hep);
+    const double na = we * wx;  // N_a at q
+    const double *p0 = dv[a & 2], *p1 = dv[(a & 2) + 1], *p2 = dw[a & 1],
+                 *p3 = dw[(a & 1) + 2];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      out[k][8] = vx0 * p0[k] + vx1 * p1[k] + ve0 * p2[k] + ve1 * p3[k];
+      out[3 + k][8] = -na * nd[k];
     }
   }
 }
