@@ -52,7 +52,7 @@ struct gf_ilu_s {
   std::vector<int> lmaxlen;                // longest row of each L level
   // sync-free sweep state
   int *lchunk = nullptr, *uchunk = nullptr; // chunk offsets (see below)
-  int4 *lmeta = nullptr, *umeta = nullptr;  // {row, k0, k1, 0} per
+  int4 *lmeta = nullptr, *umeta = nullptr;  // {row, k0, k1, level} per
                                             // position in hand-out order
   int nlchunk = 0, nuchunk = 0;
   bool lchains = false, uchains = false;  // chunks are chains in row order
@@ -69,6 +69,9 @@ struct gf_ilu_s {
   // sweeps over row groups (trsv_group_kernel; none: nlgroup == 0)
   int *lgroup = nullptr, *ugroup = nullptr;  // group records
   int nlgroup = 0, nugroup = 0, ggrid = 0;
+  // small system: both sweeps by one workgroup (trsv_small_kernel) over the
+  // level-ordered rows of lmeta and umeta
+  bool small = false;
   // dependency level of every group, or of every chunk where there are no
   // groups (host; batched sweeps merge the items of several systems level by
   // level)
@@ -1525,6 +1528,170 @@ __global__ void __launch_bounds__(kSweepThreads, GPUFEM_SWEEP_MINWAVES)
   }
 }
 
+// ---- both sweeps of a small system in one workgroup ----
+// A level of the kernels above costs a trip through memory from one CU to
+// another, and a small system has little else.  Here one workgroup takes the
+// whole pair: the solution stays in LDS, a level ends at a barrier, and a
+// wavefront takes every sixteenth row in level order and keeps the blocks of
+// its next rows in flight, so that what follows a barrier is the
+// dependencies' entries from LDS, their products, three adds across eight
+// lanes and the 6 x 6 triangle.  Lane 8 r + t (r < 6) takes scalar row r of
+// the row's block t.  No sentinel: tmp is not used.
+// What bounds it: the chain of a level (0.5 us) in the smallest systems,
+// then one CU's loads (0.08 us a row and sweep).  Natural-order ILU(0) of a
+// 10x10 plate (31 levels a sweep), FP64: sentinel, L and U kernels 4 + 36 +
+// 38 us, so 36 us.  16 wavefronts with 3 rows each in flight, 8 with 5: the
+// same at 121 rows, 120 and 133 us at 625; one row in flight is no slower at
+// 121 rows.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallBlocks = 8;  // blocks of a row on either side, at most
+constexpr int kSmallRing = 3;    // rows of a wavefront whose blocks are in flight
+
+// Sum over eight consecutive lanes, in each of them.
+template <int kCtrl, typename T>
+__device__ __forceinline__ T dpp_move(T v) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(
+        T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf,
+                                    0xf, true));
+  } else {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, kCtrl, 0xf, 0xf, true);
+    const int hi =
+        __builtin_amdgcn_mov_dpp((int)(b >> 32), kCtrl, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, ((long long)hi << 32) | (unsigned)lo);
+  }
+}
+template <typename T>
+__device__ __forceinline__ T sum8(T v) {
+  v += dpp_move<0xb1>(v);           // lanes 1 0 3 2
+  v += dpp_move<0x4e>(v);           // lanes 2 3 0 1
+  return v + dpp_move<0x141>(v);    // lanes 7 .. 0 of each eight
+}
+
+// A barrier for data in LDS alone: __syncthreads also waits for the loads
+// and stores that the wavefront has in flight to memory.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ int4 uniform(int4 v) {
+  return make_int4(__builtin_amdgcn_readfirstlane(v.x),
+                   __builtin_amdgcn_readfirstlane(v.y),
+                   __builtin_amdgcn_readfirstlane(v.z),
+                   __builtin_amdgcn_readfirstlane(v.w));
+}
+
+template <typename T, bool kLower>
+__device__ __forceinline__ void small_sweep(const SweepSlot<T>& S, int nlev,
+                                            T* xs) {
+  const int4* __restrict__ meta = kLower ? S.lmeta : S.umeta;
+  const int* __restrict__ cols = S.cols;
+  const T* __restrict__ lu = S.lu;
+  constexpr int R = kSmallRing, nw = kSmallThreads / 64;
+  const int lane = threadIdx.x % 64;
+  const int r = lane >> 3, t = lane & 7, rr = r < 6 ? r : 5;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  constexpr int kNone = 0x7fffffff;  // level of no row
+  // the ring: rows w + nw (R k + s) of the level order in slot s, their
+  // descriptors (m: of the row held, mv: of the next row, not yet waited for),
+  // blocks, diagonal blocks and right-hand sides
+  int4 m[R], mv[R];
+  T a[R][6], d[R][6], b[R];
+  int col[R];
+  auto fetch = [&](int p) {
+    return p < S.n ? meta[p] : make_int4(0, 0, 0, kNone);
+  };
+  // lanes without a block of the row load nothing and what they hold is
+  // dropped; lane 8 r alone has row r of the diagonal block
+  auto load = [&](int s) {
+    if (m[s].w == kNone) return;
+    const int di = kLower ? m[s].z : m[s].y - 1;
+    const int q = m[s].y + t;
+    if (r < 6 && q < m[s].z) {
+      col[s] = cols[q];
+      const T* ap = lu + 36 * (size_t)q + 6 * r;
+#pragma unroll
+      for (int c = 0; c < 6; c++) a[s][c] = ap[c];
+    }
+    if (r < 6 && t == 0) {
+      const T* dp = lu + 36 * (size_t)di + 6 * r;
+#pragma unroll
+      for (int c = 0; c < 6; c++) d[s][c] = dp[c];
+      if constexpr (kLower) b[s] = S.b[6 * (size_t)m[s].x + r];
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < R; s++) mv[s] = fetch(w + nw * s);
+#pragma unroll
+  for (int s = 0; s < R; s++) {
+    m[s] = uniform(mv[s]);
+    load(s);
+    mv[s] = fetch(w + nw * (R + s));
+  }
+  int lev = 0, next = w + nw * 2 * R;
+  for (;;) {
+#pragma unroll
+    for (int s = 0; s < R; s++) {
+      const int4 mm = m[s];
+      if (mm.w == kNone) goto done;
+      for (; lev < mm.w; lev++) lds_barrier();
+      T v = kLower ? b[s] : xs[6 * mm.x + rr], dinv = T(0);
+      T acc = T(0);
+      if (r < 6 && mm.y + t < mm.z) {
+        const T* xv = xs + 6 * col[s];
+#pragma unroll
+        for (int c = 0; c < 6; c++) acc += a[s][c] * xv[c];
+      }
+      if constexpr (!kLower) {
+        T dd = d[s][0];
+#pragma unroll
+        for (int c = 1; c < 6; c++) dd = rr == c ? d[s][c] : dd;
+        dinv = T(1) / dd;
+      }
+      v -= sum8(acc);
+      if constexpr (kLower) {
+#pragma unroll
+        for (int c = 0; c < 5; c++) {
+          const T y = read_lane(v, 8 * c);
+          v = r > c ? v - d[s][c] * y : v;
+        }
+      } else {
+#pragma unroll
+        for (int c = 5; c >= 0; c--) {
+          v = r == c ? v * dinv : v;
+          const T y = read_lane(v, 8 * c);
+          v = r < c ? v - d[s][c] * y : v;
+        }
+      }
+      if (r < 6 && t == 0) {
+        xs[6 * mm.x + r] = v;
+        if constexpr (!kLower) S.x[6 * (size_t)mm.x + r] = v;
+      }
+      m[s] = uniform(mv[s]);
+      load(s);
+      mv[s] = fetch(next);
+      next += nw;
+    }
+  }
+done:
+  for (; lev < nlev; lev++) lds_barrier();
+}
+
+// kBatched: workgroup k takes system k of the slots, if it is a small one.
+template <typename T, bool kBatched>
+__global__ void __launch_bounds__(kSmallThreads)
+    trsv_small_kernel(SweepSlot<T> one, const SweepSlot<T>* __restrict__ slots) {
+  extern __shared__ __align__(16) unsigned char small_lds[];
+  T* xs = reinterpret_cast<T*>(small_lds);
+  const SweepSlot<T> S = kBatched ? slots[blockIdx.x] : one;
+  if (kBatched && (S.nllev == 0 || *S.go != 1)) return;
+  small_sweep<T, true>(S, S.nllev, xs);
+  small_sweep<T, false>(S, S.nulev, xs);
+}
+
 // ---- sweeps over row groups ----
 // A level of a few rows costs a row's whole latency, from a dependency's
 // store to the row's own (1.2 us on an idle device, 1.6-2.1 us under load).
@@ -2023,6 +2190,18 @@ int group_records(const int* rowp, const int* cols, const int* diag,
 
 }  // namespace
 
+// Which systems trsv_small_kernel sweeps: those whose rows fit its lanes
+// (kSmallBlocks a side) and LDS, with few enough rows a level.  FP64 pair in
+// one workgroup / by the kernels of larger systems, with the host's calls:
+// plates in natural order, ILU(0), 10x10 (121 rows, 31 levels) 55 / 99 us,
+// 24x24 (625, 73) 140 / 198, 35x35 (1,296, 106) 250 / 276; RCM 24x24 (625,
+// 96) 152 / 200; AMD 10x10 (121, 14) 45 / 55, 16x16 (289, 18) 68 / 68,
+// 32x32 (1,089, 18) 167 / 70.
+constexpr int kSmallRows = 1300;  // 6 FP64 values a row in 64 KB of LDS
+constexpr int kSmallWidth = 12;   // rows a level, on average
+static bool small_sweeps(int n, int nlev) {
+  return n <= kSmallRows && n <= kSmallWidth * nlev;
+}
 size_t ilu_counter_bytes() {
   return sizeof(unsigned long long) * kCounterStride *
          (1 + kSweepThreads / 64);
@@ -2119,7 +2298,16 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
   h->level_sweeps = tenv && std::string(tenv) == "level";
   // row groups, by the rule at kGroupRatio
   std::vector<int> lgr, ugr;
-  if (!use_chains && !h->level_sweeps) {
+  int side = 0;  // most blocks of a row on one side of the diagonal
+  for (int i = 0; i < n; i++)
+    side = std::max({side, diag[i] - rowp[i], rowp[i + 1] - diag[i] - 1});
+  // (GPUFEM_TRSV set to anything else: the kernels of larger systems)
+  if (!tenv)
+    h->small = side <= gf::kSmallBlocks && gf::small_sweeps(
+                   n, (int)std::max(h->lptr.size(), h->uptr.size()) - 1);
+  else if (std::string(tenv) == "small")
+    h->small = side <= gf::kSmallBlocks && n <= gf::kSmallRows;
+  if (!use_chains && !h->level_sweeps && !h->small) {
     gf::SweepGroups sg;
     gf::sweep_groups(n, rowp, cols, diag.data(), h->lptr, lrows, sg);
     const int gl = gf::group_records(rowp, cols, diag.data(), sg, true, lgr,
@@ -2155,7 +2343,7 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
     levels_of(uch, h->uptr, h->ulevel);
   }
   // row descriptors in hand-out order, one 16-byte load per row: {row, first
-  // block, end block, 0}; the diagonal block is the end (L) or one before the
+  // block, end block, level}; the diagonal block is the end (L) or one before the
   // first (U)
   std::vector<int4> lm(n), um(n);
   for (int p = 0; p < n; p++) {
@@ -2163,6 +2351,14 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
     lm[p] = make_int4(li, rowp[li], diag[li], 0);
     const int ui = use_chains ? n - 1 - p : urows[p];
     um[p] = make_int4(ui, diag[ui] + 1, rowp[ui + 1], 0);
+  }
+  auto levels_into = [](const std::vector<int>& lp, std::vector<int4>& mt) {
+    for (size_t l = 0; l + 1 < lp.size(); l++)
+      for (int p = lp[l]; p < lp[l + 1]; p++) mt[p].w = (int)l;
+  };
+  if (!use_chains) {
+    levels_into(h->lptr, lm);
+    levels_into(h->uptr, um);
   }
   auto up = [&](int** dst, const int* src, size_t cnt) -> int {
     GF_TRY(gf::dmalloc(ctx, (void**)dst, sizeof(int) * (cnt ? cnt : 1)));
@@ -2300,6 +2496,8 @@ int ilu_view(gf_ilu h, IluView* v) {
   v->llevel = &h->llevel;
   v->ulevel = &h->ulevel;
   v->grid = h->grid;
+  v->nllev = h->small ? (int)h->lptr.size() - 1 : 0;
+  v->nulev = h->small ? (int)h->uptr.size() - 1 : 0;
   return GF_OK;
 }
 
@@ -2338,6 +2536,10 @@ int launch_batch_sweeps(hipStream_t s, const SweepSlot<T>* slots,
   };
   sweep(std::true_type{});
   sweep(std::false_type{});
+  if (it.small_rows > 0)
+    hipLaunchKernelGGL((trsv_small_kernel<T, true>), dim3(it.nslots),
+                       dim3(kSmallThreads), sizeof(T) * 6 * it.small_rows, s,
+                       SweepSlot<T>{}, slots);
   return hipGetLastError() == hipSuccess ? GF_OK : GF_ERR_DEVICE;
 }
 template int launch_batch_sweeps<double>(hipStream_t, const SweepSlot<double>*,
@@ -2594,6 +2796,22 @@ int ilu_apply(gf_ilu h, const T* lu, const T* b, T* tmp, T* x) {
   if (!h || !lu || !b || !tmp || !x || b == tmp || tmp == x)
     return GF_ERR_INVALID;
   gf_context ctx = h->ctx;
+  if (h->small) {
+    gf::SweepSlot<T> one{};
+    one.lmeta = h->lmeta;
+    one.umeta = h->umeta;
+    one.cols = h->cols;
+    one.lu = lu;
+    one.b = b;
+    one.x = x;
+    one.n = h->n;
+    one.nllev = (int)h->lptr.size() - 1;
+    one.nulev = (int)h->uptr.size() - 1;
+    hipLaunchKernelGGL((gf::trsv_small_kernel<T, false>), dim3(1),
+                       dim3(gf::kSmallThreads), sizeof(T) * 6 * (size_t)h->n,
+                       ctx->stream, one, (const gf::SweepSlot<T>*)nullptr);
+    return gf::check_launch(ctx, "trsv_small_kernel");
+  }
   if (!h->level_sweeps) {
     const size_t N = 6 * (size_t)h->n;
     hipLaunchKernelGGL(gf::fill_sentinel_kernel<T>, dim3(gf::div_up(N, 256)),

@@ -95,6 +95,7 @@ struct SweepSlot {
   T* tmp;
   T* x;
   const int* go;  // batched launches sweep the system only while *go == 1
+  int n, nllev, nulev;  // rows and levels of a small system (nllev > 0)
 };
 // The device schedule of an ILU analysis (row groups where it has them, else
 // chunks) and the dependency level of each item.
@@ -106,13 +107,18 @@ struct IluView {
   const std::vector<int>* llevel = nullptr;  // of each group, or each chunk
   const std::vector<int>* ulevel = nullptr;
   int grid = 0;
+  int nllev = 0, nulev = 0;  // small system: swept by one workgroup
 };
 // Work items {system, chunk or group} of a batched sweep pair on the device:
 // nc chunks of the systems without row groups, then ng groups of the others,
 // each part merged level by level.
+// Small systems have none: one workgroup a slot takes those of the nslots
+// systems, the largest of small_rows rows (0: none is small).
 struct SweepItems {
   const int2 *l = nullptr, *u = nullptr;
   int lc = 0, lg = 0, uc = 0, ug = 0;
+  int nslots = 0;
+  size_t small_rows = 0;
 };
 // tickets counters of a batched sweep pair (device, unsigned long long each)
 constexpr int kBatchCounters = 4;

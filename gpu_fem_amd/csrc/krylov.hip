@@ -1224,6 +1224,9 @@ SweepSlot<T> sweep_entry(const Solve* v, const int* go) {
     e.x = (T*)p->t32c;
   }
   e.go = go;
+  e.n = v->iv.n;
+  e.nllev = v->iv.nllev;
+  e.nulev = v->iv.nulev;
   return e;
 }
 }  // namespace
@@ -1287,6 +1290,7 @@ int BatchEngine::rebuild() {
     for (int lev = 0;; lev++) {
       bool any = false;
       for (int i = 0; i < ns; i++) {
+        if (act[i]->iv.nllev > 0) continue;
         if ((act[i]->iv.lgroup != nullptr) != groups) continue;
         const std::vector<int>& cl =
             lower ? *act[i]->iv.llevel : *act[i]->iv.ulevel;
@@ -1307,6 +1311,11 @@ int BatchEngine::rebuild() {
   items.uc = (int)um.size();
   merge(false, true, um);
   items.ug = (int)um.size() - items.uc;
+  items.nslots = ns;
+  items.small_rows = 0;
+  for (const Solve* v : act)
+    if (v->iv.nllev > 0)
+      items.small_rows = std::max(items.small_rows, (size_t)v->iv.n);
   ntot = voff[ns];
   nrows = roff[ns];
   grid = std::max(1, std::min(gsum, std::max(1, waves_per_cu * ctx->num_cus / 4)));
@@ -1455,8 +1464,13 @@ int BatchEngine::start(Solve* v) {
   v->solo = SweepItems{};
   v->solo.l = v->d_sl;
   v->solo.u = v->d_su;
-  (v->iv.lgroup ? v->solo.lg : v->solo.lc) = nsl;
-  (v->iv.lgroup ? v->solo.ug : v->solo.uc) = nsu;
+  v->solo.nslots = 1;
+  if (v->iv.nllev > 0) {
+    v->solo.small_rows = (size_t)v->n;
+  } else {
+    (v->iv.lgroup ? v->solo.lg : v->solo.lc) = nsl;
+    (v->iv.lgroup ? v->solo.ug : v->solo.uc) = nsu;
+  }
   GF_HIP(ctx, hipMemcpyAsync(v->d_solo, v->h_solo.data(), v->h_solo.size(),
                              hipMemcpyHostToDevice, s));
   GF_HIP(ctx, hipMemcpyAsync(v->d_sl, v->h_sl.data(), sizeof(int2) * nsl,
