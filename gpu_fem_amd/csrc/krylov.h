@@ -22,6 +22,7 @@ struct KrylovWork {
   double *hc = nullptr, *dd = nullptr, *co = nullptr, *rho = nullptr;
   float *a32 = nullptr, *b32 = nullptr, *c32 = nullptr;
   double* host_scal = nullptr;  // pinned: two (estimate, h_{j+1,j}) slots
+  double* dev_scal = nullptr;   // the same memory's device address
   // Z_i = M^-1 V_i kept beside the basis (m vectors; null when not kept):
   // the cycle's update is then x += Z y, without a preconditioner
   // application

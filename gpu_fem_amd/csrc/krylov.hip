@@ -21,13 +21,20 @@
 namespace gf {
 namespace {
 
-constexpr int kDotBlocks = 256;  // slices of the index range
+constexpr int kDotBlocks = 256;  // slices of the index range, at most
 constexpr int kDotThreads = 256;
 constexpr int kDotChunk = 8;
+// Slices of N entries: a thread has at least one entry.  (256 slices of 726
+// entries kept three threads of 256 busy: 16.6 us a product of a 10x10
+// plate's basis, 7.2 us so.)
+__host__ __device__ inline int dot_slices(size_t N) {
+  const size_t k = (N + kDotThreads - 1) / kDotThreads;
+  return k < 1 ? 1 : k > (size_t)kDotBlocks ? kDotBlocks : (int)k;
+}
 
 // partial[b * nvec + i] = sum over slice b of V_i . w.  Grid: x = slice of
-// the index range (kDotBlocks slices), y = chunk of kDotChunk vectors, so a
-// long basis spreads over kDotBlocks x ceil(nvec / kDotChunk) workgroups.
+// the index range (dot_slices), y = chunk of kDotChunk vectors, so a long
+// basis spreads over dot_slices x ceil(nvec / kDotChunk) workgroups.
 __global__ void __launch_bounds__(kDotThreads)
     multi_dot_partial(size_t N, int nvec, const double* __restrict__ V,
                       size_t ldv, const double* __restrict__ w,
@@ -306,6 +313,10 @@ __global__ void __launch_bounds__(kDotThreads)
                     blockIdx.y);
 }
 
+// Short vectors: so few slices are added by the coefficients kernel itself
+// (multi_dot_final took 4.6 us of a step of a 10x10 plate).
+constexpr int kFuseSlices = 4;
+
 // Workgroup sum of v (256 threads), result in every thread.
 __device__ double block_sum256(double v, double* red) {
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
@@ -370,12 +381,30 @@ __device__ __forceinline__ void dcgs2_coeffs_body(
     __syncthreads();
     if (tid == 0) {
       const int jc = j - 1;
-      for (int i = 0; i < jc; i++) {
-        const double a = col[i], c = col[i + 1];
-        col[i] = lcs[i] * a + lsn[i] * c;
-        col[i + 1] = -lsn[i] * a + lcs[i] * c;
+      // the recurrence in a register, its operands read ahead of it
+      double a = col[0];
+      int i = 0;
+      constexpr int K = 8;
+      for (; i + K <= jc; i += K) {
+        double cv[K], cs_[K], sn_[K];
+#pragma unroll
+        for (int z = 0; z < K; z++) {
+          cv[z] = col[i + 1 + z];
+          cs_[z] = lcs[i + z];
+          sn_[z] = lsn[i + z];
+        }
+#pragma unroll
+        for (int z = 0; z < K; z++) {
+          col[i + z] = cs_[z] * a + sn_[z] * cv[z];
+          a = -sn_[z] * a + cs_[z] * cv[z];
+        }
       }
-      const double a = col[jc], c = col[jc + 1];
+      for (; i < jc; i++) {
+        const double c = col[i + 1], x = lcs[i], y = lsn[i];
+        col[i] = x * a + y * c;
+        a = -y * a + x * c;
+      }
+      const double c = col[jc + 1];
       const double den = sqrt(a * a + c * c);
       const double cj = den > 0.0 ? a / den : 1.0;
       const double sj = den > 0.0 ? c / den : 0.0;
@@ -410,7 +439,18 @@ __device__ __forceinline__ void dcgs2_coeffs_body(
     // all lanes walk k together so each load is one coalesced row segment;
     // entries below the subdiagonal (k < i - 1) are skipped, not read
     double hs = 0.0;
-    for (int k = 0; k < j; k++)
+    int k = 0;
+    constexpr int K = 8;
+    for (; k + K <= j; k += K) {
+      double h[K];
+#pragma unroll
+      for (int z = 0; z < K; z++)
+        h[z] = k + z + 1 >= i ? Hc[(size_t)(k + z) * ldh + i] : 0.0;
+#pragma unroll
+      for (int z = 0; z < K; z++)
+        if (k + z + 1 >= i) hs += h[z] * ls[k + z];
+    }
+    for (; k < j; k++)
       if (k + 1 >= i) hs += Hc[(size_t)k * ldh + i] * ls[k];
     const double ci = i < j ? t[i] : cj;
     hj[i] = (ci - hs) * inva;
@@ -434,11 +474,57 @@ __device__ __forceinline__ void dcgs2_coeffs_body(
 }
 
 __global__ void __launch_bounds__(256)
-    dcgs2_coeffs(int j, int m, const double* __restrict__ d, double* Hc,
-                 double* rho, double* st, double* co, double* out,
-                 int finalize) {
+    dcgs2_coeffs(int j, int m, double* d, double* Hc, double* rho, double* st,
+                 double* co, double* out, int finalize,
+                 const double* __restrict__ partial, int nslices) {
   extern __shared__ double sh[];
+  if (partial) {  // d from at most kFuseSlices slices, as multi_dot_final adds
+    const int nout = 2 * j + 3;
+    for (int i = threadIdx.x; i < nout; i += 256) {
+      double p[kFuseSlices];
+#pragma unroll
+      for (int b = 0; b < kFuseSlices; b++)
+        p[b] = b < nslices ? partial[(size_t)b * nout + i] : 0.0;
+      d[i] = (p[0] + p[2]) + (p[1] + p[3]);
+    }
+    __syncthreads();
+  }
   dcgs2_coeffs_body(j, m, d, Hc, rho, st, co, out, finalize, sh);
+}
+
+// a1 = sum_{i<j} c1[i] V_i[t], and a2 with c2 (may be null).  Vector i goes to
+// running sum i % kParts: with one sum an entry every load waited for the
+// previous one (10x10 plate, 80 vectors and their preconditioned ones: 12.8 us
+// a step, 5.4 us with eight; eight lanes an entry instead measured the same
+// from 1,700 to 88,000 entries).
+constexpr int kParts = 8;
+__device__ __forceinline__ double parts_total(const double (&a)[kParts]) {
+  static_assert(kParts == 8, "");
+  return ((a[0] + a[4]) + (a[2] + a[6])) + ((a[1] + a[5]) + (a[3] + a[7]));
+}
+__device__ __forceinline__ void basis_sums(size_t t, int j,
+                                           const double* __restrict__ V,
+                                           size_t ldv,
+                                           const double* __restrict__ c1,
+                                           const double* __restrict__ c2,
+                                           double& a1, double& a2) {
+  double s1[kParts], s2[kParts];
+#pragma unroll
+  for (int k = 0; k < kParts; k++) s1[k] = s2[k] = 0.0;
+  auto add = [&](int i, int k) {
+    const double v = V[(size_t)(i + k) * ldv + t];
+    s1[k] += c1[i + k] * v;
+    if (c2) s2[k] += c2[i + k] * v;
+  };
+  int i = 0;
+  for (; i + kParts <= j; i += kParts)
+#pragma unroll
+    for (int k = 0; k < kParts; k++) add(i, k);
+#pragma unroll
+  for (int k = 0; k < kParts - 1; k++)
+    if (i + k < j) add(i, k);
+  a1 = parts_total(s1);
+  a2 = c2 ? parts_total(s2) : 0.0;
 }
 
 // One pass over V[0..j-1]: q_j = (V_j - sum s_i V_i) / alpha (final) and
@@ -448,14 +534,9 @@ __device__ __forceinline__ void update2_body(size_t t, int j, int m,
                                              size_t ldv,
                                              const double* __restrict__ w,
                                              const double* __restrict__ co) {
-  const double* sc = co;
   const double* cc = co + m + 1;
-  double as = 0.0, ac = 0.0;
-  for (int i = 0; i < j; i++) {
-    const double v = V[(size_t)i * ldv + t];
-    as += sc[i] * v;
-    ac += cc[i] * v;
-  }
+  double as, ac;
+  basis_sums(t, j, V, ldv, co, cc, as, ac);
   const double qf = j > 0 ? (V[(size_t)j * ldv + t] - as) * co[2 * m + 2]
                           : V[t];
   if (j > 0) V[(size_t)j * ldv + t] = qf;
@@ -471,8 +552,8 @@ __device__ __forceinline__ void update_z_body(size_t t, int j, int m,
                                               size_t ldv,
                                               const double* __restrict__ co) {
   if (j > 0) {
-    double az = 0.0;
-    for (int i = 0; i < j; i++) az += co[i] * Z[(size_t)i * ldv + t];
+    double az, none;
+    basis_sums(t, j, Z, ldv, co, nullptr, az, none);
     zj = (zj - az) * co[2 * m + 2];
   }
   Z[(size_t)j * ldv + t] = zj;
@@ -535,6 +616,8 @@ int KrylovWork::init(gf_context c, size_t N_, int m_, bool mixed,
     GF_TRY(check_hip(ctx, hipHostMalloc((void**)&ctx->pinned, sizeof(double) * 8),
                      "hipHostMalloc"));
   host_scal = ctx->pinned;
+  GF_TRY(check_hip(ctx, hipHostGetDevicePointer((void**)&dev_scal, host_scal, 0),
+                   "hipHostGetDevicePointer"));
   GF_TRY(check_hip(ctx, hipEventCreateWithFlags(&ev[0], hipEventDisableTiming),
                    "event"));
   GF_TRY(check_hip(ctx, hipEventCreateWithFlags(&ev[1], hipEventDisableTiming),
@@ -573,11 +656,11 @@ void KrylovWork::release() {
 int KrylovWork::dots(const double* Vb, size_t ldv, int nvec, const double* x,
                      double* out, int mode, const int* gate) {
   hipLaunchKernelGGL(multi_dot_partial,
-                     dim3(kDotBlocks, div_up(nvec, kDotChunk)),
+                     dim3(dot_slices(N), div_up(nvec, kDotChunk)),
                      dim3(kDotThreads), 0, ctx->stream, N, nvec, Vb, ldv, x,
                      partial, gate);
   hipLaunchKernelGGL(multi_dot_final, dim3(nvec), dim3(kDotThreads), 0,
-                     ctx->stream, (int)kDotBlocks, nvec, partial, out, mode,
+                     ctx->stream, dot_slices(N), nvec, partial, out, mode,
                      gate);
   return check_launch(ctx, "multi_dot");
 }
@@ -712,6 +795,9 @@ int gmres_solve(KrylovWork& W, const Operator& op, const double* b, double* x,
       // once step js+1 is queued.
       const size_t shm = sizeof(double) * (4 * (size_t)m + 2);
       double e1 = 0.0, e2 = 0.0;  // the last two estimates of the cycle
+      // the step's estimate goes straight to the pinned host memory that
+      // is read once the step's event has passed
+      auto est_out = [&](int js) { return W.dev_scal + 2 * (js % 2); };
       while (!stop) {
         if (issued <= limit) {
           const int js = issued;
@@ -727,7 +813,8 @@ int gmres_solve(KrylovWork& W, const Operator& op, const double* b, double* x,
               e1 * (e1 / e2) <= kPeekMargin * tol_abs) {
             GF_TRY(W.dots(W.V, N, js + 1, vj, W.dd, 0));
             hipLaunchKernelGGL(dcgs2_coeffs, dim3(1), dim3(256), shm, s, js,
-                               m, W.dd, W.hc, W.rho, W.state, W.co, W.scal, 2);
+                               m, W.dd, W.hc, W.rho, W.state, W.co, W.scal,
+                               2, (const double*)nullptr, 0);
             GF_HIP(ctx, hipMemcpyAsync(W.host_scal + 4, W.scal,
                                        2 * sizeof(double),
                                        hipMemcpyDeviceToHost, s));
@@ -736,7 +823,7 @@ int gmres_solve(KrylovWork& W, const Operator& op, const double* b, double* x,
             if (!std::isfinite(est) || est <= tol_abs || hn == 0.0) {
               hipLaunchKernelGGL(dcgs2_coeffs, dim3(1), dim3(256), shm, s, js,
                                  m, W.dd, W.hc, W.rho, W.state, W.co, W.scal,
-                                 1);
+                                 1, (const double*)nullptr, 0);
               GF_TRY(check_launch(ctx, "arnoldi finalisation"));
               last_est = est;
               j = js;
@@ -750,14 +837,18 @@ int gmres_solve(KrylovWork& W, const Operator& op, const double* b, double* x,
                                    keep_z ? W.Z + (size_t)js * N : nullptr));
             const int nv = js + 1, nout = 2 * nv + 1;
             hipLaunchKernelGGL(multi_dot2_partial,
-                               dim3(kDotBlocks, div_up(nv, kDotChunk)),
+                               dim3(dot_slices(N), div_up(nv, kDotChunk)),
                                dim3(kDotThreads), 0, s, N, nv, W.V, N, vj,
                                W.w, W.partial);
-            hipLaunchKernelGGL(multi_dot_final, dim3(nout), dim3(kDotThreads),
-                               0, s, (int)kDotBlocks, nout, W.partial, W.dd,
-                               0, (const int*)nullptr);
+            const int nsl = dot_slices(N);
+            const bool fuse = nsl <= kFuseSlices;
+            if (!fuse)
+              hipLaunchKernelGGL(multi_dot_final, dim3(nout),
+                                 dim3(kDotThreads), 0, s, nsl, nout, W.partial,
+                                 W.dd, 0, (const int*)nullptr);
             hipLaunchKernelGGL(dcgs2_coeffs, dim3(1), dim3(256), shm, s, js,
-                               m, W.dd, W.hc, W.rho, W.state, W.co, W.scal, 0);
+                               m, W.dd, W.hc, W.rho, W.state, W.co, est_out(js),
+                               0, fuse ? W.partial : nullptr, fuse ? nsl : 0);
             if (keep_z)
               hipLaunchKernelGGL(update2z, grid1(N), dim3(256), 0, s, N, js,
                                  m, W.V, N, W.w, W.co, W.Z);
@@ -767,15 +858,11 @@ int gmres_solve(KrylovWork& W, const Operator& op, const double* b, double* x,
           } else {
             GF_TRY(W.dots(W.V, N, js + 1, vj, W.dd, 0));
             hipLaunchKernelGGL(dcgs2_coeffs, dim3(1), dim3(256), shm, s, js,
-                               m, W.dd, W.hc, W.rho, W.state, W.co, W.scal, 1);
+                               m, W.dd, W.hc, W.rho, W.state, W.co, est_out(js),
+                               1, (const double*)nullptr, 0);
           }
           GF_TRY(check_launch(ctx, "arnoldi step"));
-          if (js >= 1) {
-            GF_HIP(ctx, hipMemcpyAsync(W.host_scal + 2 * (js % 2), W.scal,
-                                       2 * sizeof(double),
-                                       hipMemcpyDeviceToHost, s));
-            GF_HIP(ctx, hipEventRecord(W.ev[js % 2], s));
-          }
+          if (js >= 1) GF_HIP(ctx, hipEventRecord(W.ev[js % 2], s));
           issued++;
         }
         // iteration count j + 1 is reported by step j + 1; it is read once
@@ -1013,7 +1100,7 @@ __global__ void __launch_bounds__(256)
   k.w[6 * (size_t)row + r] = acc;
 }
 
-// grid (kBatchSlices, vector chunks, solves)
+// grid (kBatchSlices, vector chunks, solves); a solve uses dot_slices of them
 __global__ void __launch_bounds__(kDotThreads)
     batch_dot2_partial(const KrySlot* ks, const SlotState* st) {
   const int s = blockIdx.z;
@@ -1022,9 +1109,11 @@ __global__ void __launch_bounds__(kDotThreads)
   const int j = st[s].j, nv = j + 1;
   if ((int)blockIdx.y * kDotChunk >= nv) return;
   const KrySlot& k = ks[s];
+  const int slices = dot_slices((size_t)k.N);
+  if ((int)blockIdx.x >= slices) return;
   dot2_partial_body((size_t)k.N, nv, k.V, (size_t)k.N,
-                    k.V + (size_t)j * k.N, k.w, k.partial, blockIdx.x,
-                    kBatchSlices, blockIdx.y);
+                    k.V + (size_t)j * k.N, k.w, k.partial, blockIdx.x, slices,
+                    blockIdx.y);
 }
 
 // grid (outputs, solves): dd[i] = sum over slices of partial, in the
@@ -1040,7 +1129,8 @@ __global__ void __launch_bounds__(kDotThreads)
   const KrySlot& k = ks[s];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   double v = 0.0;
-  for (int b = threadIdx.x; b < kBatchSlices; b += kDotThreads)
+  const int slices = dot_slices((size_t)k.N);
+  for (int b = threadIdx.x; b < slices; b += kDotThreads)
     v += k.partial[(size_t)b * nout + i];
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
   if (lane == 0) red[wave] = v;
@@ -1478,11 +1568,11 @@ int BatchEngine::start(Solve* v) {
   GF_HIP(ctx, hipMemcpyAsync(v->d_su, v->h_su.data(), sizeof(int2) * nsu,
                              hipMemcpyHostToDevice, s));
   KrylovWork& W = p->kw;
-  hipLaunchKernelGGL(multi_dot_partial, dim3(kDotBlocks, 1), dim3(kDotThreads),
+  hipLaunchKernelGGL(multi_dot_partial, dim3(dot_slices(v->N), 1), dim3(kDotThreads),
                      0, s, v->N, 1, p->rhs, v->N, p->rhs, W.partial,
                      (const int*)nullptr);
   hipLaunchKernelGGL(multi_dot_final, dim3(1), dim3(kDotThreads), 0, s,
-                     (int)kDotBlocks, 1, W.partial, W.scal, 2,
+                     dot_slices(v->N), 1, W.partial, W.scal, 2,
                      (const int*)nullptr);
   GF_HIP(ctx, hipMemcpyAsync(h_norm + 2 * v->hidx + 1, W.scal, sizeof(double),
                              hipMemcpyDeviceToHost, s));
@@ -1496,11 +1586,11 @@ int BatchEngine::residual_issue(Solve* v) {
   KrylovWork& W = p->kw;
   GF_TRY(gf_bsr_resid_comp_f64(ctx, p->nnodes, p->krowp, p->kcols, p->kvals,
                                p->sol, p->rhs, W.r));
-  hipLaunchKernelGGL(multi_dot_partial, dim3(kDotBlocks, 1), dim3(kDotThreads),
+  hipLaunchKernelGGL(multi_dot_partial, dim3(dot_slices(v->N), 1), dim3(kDotThreads),
                      0, s, v->N, 1, W.r, v->N, W.r, W.partial,
                      (const int*)nullptr);
   hipLaunchKernelGGL(multi_dot_final, dim3(1), dim3(kDotThreads), 0, s,
-                     (int)kDotBlocks, 1, W.partial, W.nrm, 2,
+                     dot_slices(v->N), 1, W.partial, W.nrm, 2,
                      (const int*)nullptr);
   GF_HIP(ctx, hipMemcpyAsync(h_norm + 2 * v->hidx, W.nrm, sizeof(double),
                              hipMemcpyDeviceToHost, s));
