@@ -56,54 +56,59 @@ __global__ void bc_vec_kernel(int nbcs, const int* __restrict__ bcs,
   vec[idx] = 0.0;
 }
 
-// One wave per target row, in chunks of 64 target blocks: lane l finds the
-// source block of target block l of the chunk (binary search in the short
-// source row, once per block), the indices go through LDS, and the chunk's
-// 36 * 64 values are written with consecutive lanes on consecutive values
-// (most target blocks are fill: zeros).
-__global__ void __launch_bounds__(256)
-    copy_pattern_kernel(int nnodes, const int* __restrict__ rowp,
+// One workgroup per target row, in chunks of a block a thread: each thread
+// finds the source block of its target block (binary search in the source
+// row's columns, in LDS), and the chunk's values are written with consecutive
+// threads on consecutive V (most target blocks are fill: zeros).
+// What bounds it: the writes; a row's pieces of 288 bytes read in between
+// cost the rate of a plain fill (6.6 TB/s).  400x400 plate into its AMD +
+// ILU(96) pattern (4.1 GB), with the Jacobian: 1.76 ms with a wavefront a row
+// and 8-byte stores, 1.55 with 16-byte ones, 1.53 with two wavefronts a row
+// (one, four, eight: 1.55, 1.52, 1.65; into its own pattern 0.65, 0.77, 0.91
+// against 0.70 with two).  Rows handed to the XCDs in contiguous parts: 2.85.
+// Zeros first and K's blocks after them: 1.43, but 0.78 into its own pattern.
+constexpr int kCopyThreads = 128;
+typedef double double2v __attribute__((ext_vector_type(2)));
+template <typename V>
+__global__ void __launch_bounds__(kCopyThreads)
+    copy_pattern_kernel(const int* __restrict__ rowp,
                         const int* __restrict__ cols,
                         const double* __restrict__ vals,
                         const int* __restrict__ trowp,
                         const int* __restrict__ tcols, double* tvals) {
-  __shared__ int s_src[4][64];
-  const int w = threadIdx.x / 64;
-  const int row = blockIdx.x * 4 + w;
-  const int lane = threadIdx.x % 64;
-  if (row >= nnodes) return;
+  constexpr int kPer = 36 * sizeof(double) / sizeof(V);  // V per block
+  constexpr int kCols = 64;  // a source row's columns in LDS, at most
+  __shared__ int s_src[kCopyThreads], s_col[kCols];
+  const int tid = threadIdx.x, row = blockIdx.x;
   const int t0 = trowp[row], t1 = trowp[row + 1];
-  const int s0 = rowp[row], s1 = rowp[row + 1];
-  for (int c0 = t0; c0 < t1; c0 += 64) {
-    const int nb = min(64, t1 - c0);
-    int src = -1;
-    if (lane < nb) {
-      const int col = tcols[c0 + lane];
-      int lo = s0, hi = s1;  // lower_bound of col in the source row
+  const int s0 = rowp[row], ns = rowp[row + 1] - s0;
+  if (tid < min(ns, kCols)) s_col[tid] = cols[s0 + tid];
+  const int* sc = ns <= kCols ? s_col : cols + s0;
+  const V* from = reinterpret_cast<const V*>(vals);
+  for (int c0 = t0; c0 < t1; c0 += kCopyThreads) {
+    const int nb = min(kCopyThreads, t1 - c0);
+    const int col = tid < nb ? tcols[c0 + tid] : -1;
+    __syncthreads();  // the last chunk's indices were read
+    if (tid < nb) {
+      int lo = 0, hi = ns;  // lower_bound of col in the source row
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (cols[mid] < col)
+        if (sc[mid] < col)
           lo = mid + 1;
         else
           hi = mid;
       }
-      src = (lo < s1 && cols[lo] == col) ? lo : -1;
+      s_src[tid] = (lo < ns && sc[lo] == col) ? s0 + lo : -1;
     }
-    s_src[w][lane] = src;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    double* dst = tvals + 36 * (size_t)c0;
-    const int nval = 36 * nb;
-#pragma unroll 4
-    for (int v = lane; v < nval; v += 64) {
-      const int sb = s_src[w][v / 36];
-      dst[v] = sb >= 0 ? vals[36 * (size_t)sb + v % 36] : 0.0;
+    __syncthreads();
+    V* dst = reinterpret_cast<V*>(tvals) + kPer * (size_t)c0;
+#pragma unroll 6
+    for (int v = tid; v < kPer * nb; v += kCopyThreads) {
+      const int sb = s_src[v / kPer];
+      V z = V(0.0);
+      if (sb >= 0) z = from[kPer * (size_t)sb + v % kPer];
+      dst[v] = z;
     }
-    // the next chunk's indices overwrite s_src
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 }
 
@@ -372,9 +377,11 @@ int gf_bsr_copy_to_pattern(gf_context ctx, int nnodes, const int* rowp,
   if (!ctx || nnodes <= 0 || !rowp || !cols || !vals || !trowp || !tcols ||
       !tvals)
     return gf::set_error(ctx, GF_ERR_INVALID, "copy_to_pattern: bad args");
-  hipLaunchKernelGGL(gf::copy_pattern_kernel, dim3(gf::div_up(nnodes, 4)),
-                     dim3(256), 0, ctx->stream, nnodes, rowp, cols, vals,
-                     trowp, tcols, tvals);
+  const bool wide = ((uintptr_t)vals | (uintptr_t)tvals) % 16 == 0;
+  hipLaunchKernelGGL(wide ? gf::copy_pattern_kernel<gf::double2v>
+                          : gf::copy_pattern_kernel<double>,
+                     dim3(nnodes), dim3(gf::kCopyThreads), 0, ctx->stream,
+                     rowp, cols, vals, trowp, tcols, tvals);
   return gf::check_launch(ctx, "copy_pattern_kernel");
 }
 
