@@ -492,15 +492,16 @@ __global__ void __launch_bounds__(kIluThreads)
 }
 
 // Rows too long for LDS, with the pivots applied in runs.  The values of row
-// i stay in global memory.  A window of up to nbatch pivots is prepared ahead,
-// final or not: where the columns of their U parts lie in row i depends on
-// the pattern alone.  The pivots of the window that are final form a run:
-// wavefront 0 forms their L_ik in order, each applied at once to the run's
-// own later L-part blocks (held in LDS), and one pass reads every block of the
-// rest of the row that a pivot of the run updates once, subtracts the run's
-// contributions L_ik U_kj in pivot order and writes it once.  Every entry
-// sees the operations of ilu_row_kernel in the same order, so the factors
-// agree bit for bit.
+// i stay in global memory.  A window of up to 2 nbatch pivots is prepared
+// ahead, final or not: where the columns of their U parts lie in row i depends
+// on the pattern alone.  Up to nbatch pivots of the window that are final form
+// a run: wavefront 0 forms their L_ik in order, each applied at once to the
+// run's own later L-part blocks (held in LDS), while the other wavefronts
+// prepare the pivots that enter the window; then one pass reads every block of
+// the rest of the row that a pivot of the run updates once, subtracts the
+// run's contributions L_ik U_kj in pivot order and writes it once.  Every
+// entry sees the operations of ilu_row_kernel in the same order, so the
+// factors agree bit for bit.
 // A thread takes kBatchCols columns of a block: it loads whole rows of U_kj
 // in wide loads (one column per thread takes four times the load
 // instructions, each touching as many lines), the next pivot's while the
@@ -508,8 +509,12 @@ __global__ void __launch_bounds__(kIluThreads)
 // them.
 // Dynamic LDS per position of row i: its column index, its place in the list
 // of the run's blocks, and per pivot of the window the index (+ 1) of the
-// position in the pivot's U part (0: not updated) and, as a list, the position
-// of each of its U-part columns (or -1).
+// position in the pivot's U part (0: not updated).
+// What bounds it: the rows' own time more than the chain of pivots.  400x400
+// plate, AMD + ILU(96), FP32: 9,266 such rows of 370 to 1,750 blocks take 2.5
+// ms each on 512 places; a run of 7.7 pivots took 42 us with the window of
+// one run, 9 of them preparing the next one after it, 6 forming L_ik, 5
+// loading the pivots' edges, 12 the update, 9 waiting.
 #ifndef GPUFEM_ILU_BATCH
 #define GPUFEM_ILU_BATCH 8
 #endif
@@ -519,20 +524,32 @@ constexpr int kIluPairSlots = kIluBatch * (kIluBatch - 1) / 2;
 __device__ __forceinline__ int batch_pair(int p, int q) {
   return p * (2 * kIluBatch - p - 1) / 2 + (q - p - 1);
 }
-// dynamic LDS bytes per position of the longest row, window of nbatch
-__host__ __device__ constexpr size_t batch_lds_per_pos(int nbatch) {
-  return sizeof(int) + sizeof(short) * (size_t)(2 * nbatch + 1);
+// dynamic LDS of a row of at most maxlen positions, runs of nbatch
+__host__ __device__ constexpr int batch_stride(int maxlen) {
+  return (maxlen + 7) / 8 * 8;
+}
+__host__ __device__ constexpr size_t batch_lds(int nbatch, int maxlen) {
+  return (sizeof(short) * (size_t)(2 * nbatch + 1) + sizeof(int)) *
+         batch_stride(maxlen);
 }
 // 400x400 plate, AMD + ILU(96), whole factorisation, columns per thread:
 // FP64 1 / 2 / 3 / 6: 96 / 89 / 122 / 126 ms (3 and 6 leave room for one
 // workgroup a CU), FP32 2 / 3 / 6: 78 / 78 / 101 ms; 256 or 1,024 threads
 // 102 or 109 ms FP64.  (One column per thread, batches that waited for all
 // their pivots' lists, and the row's pairs found by walking the U parts:
-// 111 ms FP64, 97 ms FP32.)
+// 111 ms FP64, 97 ms FP32.)  Those with rows in LDS up to its whole size and a
+// window of one run; up to half of it 83 / 65 ms, and with the next run
+// prepared while L_ik are formed 72.7 / 54.9 ms (256x256 FP64 28.2 -> 23.7).
+// Two columns a lane searched for at once; one or four 0.4 or 2 ms more.
 constexpr int kBatchThreads = 512;
+// A run waits for this many pivots unless it is the row's last one: rows far
+// behind the chain would otherwise be read and written once a pivot.  75x150
+// cylinder, FP64, with 1 / 2 / 4 / 8: 10.65 / 10.06 / 9.84 / 10.7 ms; plates
+// the same within 1%.
+constexpr int kRunLeast = 4;
 template <typename T> constexpr int kBatchCols = sizeof(T) == 8 ? 2 : 3;
 template <typename T, bool kFlow>
-__global__ void __launch_bounds__(kBatchThreads)
+__global__ void __launch_bounds__(kBatchThreads, 4)
     ilu_row_batch_kernel(const int* __restrict__ level_rows, int nrows,
                          const int* __restrict__ rowp,
                          const int* __restrict__ cols,
@@ -544,7 +561,7 @@ __global__ void __launch_bounds__(kBatchThreads)
   constexpr int kTail = kEdgeBlocks<T>, kHead = kEdgeBlocks<T> - 1;
   constexpr int kEdge = 1 + kTail + kHead;  // with the diagonal block
   extern __shared__ __align__(16) unsigned char ilu_bdyn[];
-  __shared__ int s_u0[kIluBatch], s_nu[kIluBatch];  // per window slot
+  __shared__ int s_u0[2 * kIluBatch], s_nu[2 * kIluBatch];  // per window slot
   __shared__ __align__(16) T s_edge[kIluBatch][kEdge][36];
   __shared__ T s_udi[kIluBatch][6];  // 1 / diagonal of U_kk
   __shared__ __align__(16) T s_lik[kIluBatch][36];
@@ -555,60 +572,90 @@ __global__ void __launch_bounds__(kBatchThreads)
   if (i < 0) return;
   const int tid = threadIdx.x, nth = kBatchThreads;
   const int r0 = rowp[i], r1 = rowp[i + 1], nb = r1 - r0, dl = diag[i] - r0;
-  int* scol = reinterpret_cast<int*>(ilu_bdyn);
-  // hit[s * maxlen + pl] = 1 + index in U(k) of position pl for the pivot k in
-  // slot s, or 0; upos[s * maxlen + t] = position of U(k)'s column t, or -1
-  unsigned short* hit = reinterpret_cast<unsigned short*>(scol + maxlen);
-  short* upos = reinterpret_cast<short*>(hit + (size_t)nbatch * maxlen);
-  unsigned short* list =
-      reinterpret_cast<unsigned short*>(upos + (size_t)nbatch * maxlen);
+  // hit[s * stride + pl] = 1 + index in U(k) of position pl for the pivot k
+  // in slot s, or 0
+  const int stride = batch_stride(maxlen), nwin = 2 * nbatch;
+  unsigned short* hit = reinterpret_cast<unsigned short*>(ilu_bdyn);
+  unsigned short* list = hit + (size_t)nwin * stride;
+  int* scol = reinterpret_cast<int*>(list + stride);
   for (int t = tid; t < nb; t += nth) scol[t] = cols[r0 + t];
-  for (int e = tid; e < nbatch * maxlen; e += nth) hit[e] = 0;
+  for (int e = tid; e < nwin * stride / 8; e += nth)
+    reinterpret_cast<int4*>(hit)[e] = make_int4(0, 0, 0, 0);
   if (tid == 0) s_rdy[0] = s_cnt = 0;
   int par = 0;
   __syncthreads();
-  // position of column j among scol[lo..nb), or -1
-  auto find = [&](int j, int lo) {
-    int hi = nb;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (scol[mid] < j)
-        lo = mid + 1;
-      else
-        hi = mid;
+  // pivots [k0, k1) of the row into their slots (pivot k: slot k % nwin, its
+  // hits cleared) by wavefronts w0 .. 7: segments of kSeg columns of their U
+  // parts in turn, kFind columns a lane in flight, searched for together
+  constexpr int kFind = 2, kSeg = 64 * kFind;
+  auto prepare = [&](int k0, int k1, int w0) {
+    const int lane = tid % 64, nw = nth / 64 - w0;
+    int lu0 = 0, lnu = 0;
+    if (lane < k1 - k0) {
+      const int k = scol[k0 + lane];
+      lu0 = diag[k] + 1;
+      lnu = rowp[k + 1] - lu0;
     }
-    return (lo < nb && scol[lo] == j) ? lo : -1;
-  };
-  // pivots [k0, k1) of the row into their slots (pivot k: slot k % nbatch)
-  auto prepare = [&](int k0, int k1) {
-    if (tid < k1 - k0) {
-      const int k = scol[k0 + tid], s = (k0 + tid) % nbatch;
-      const int u0 = diag[k] + 1;
-      s_u0[s] = u0;
-      s_nu[s] = rowp[k + 1] - u0;
+    if (tid / 64 == w0 && lane < k1 - k0) {
+      s_u0[(k0 + lane) % nwin] = lu0;
+      s_nu[(k0 + lane) % nwin] = lnu;
     }
-    __syncthreads();
+    int turn = tid / 64 - w0;
     for (int k = k0; k < k1; k++) {
-      const int s = k % nbatch, u0 = s_u0[s], nu = s_nu[s];
-      for (int t = tid; t < nu; t += nth) {
-        const int pl = find(cols[u0 + t], k + 1);
-        upos[s * maxlen + t] = (short)pl;
-        if (pl >= 0) hit[s * maxlen + pl] = (unsigned short)(t + 1);
+      const int u0 = __builtin_amdgcn_readlane(lu0, k - k0);
+      const int nu = __builtin_amdgcn_readlane(lnu, k - k0);
+      unsigned short* const h = hit + (k % nwin) * stride;
+      const int lo0 = k + 1;
+      int top = 1;
+      while (2 * top <= nb - lo0) top *= 2;
+      int b = kSeg * turn;
+      for (; b < nu; b += kSeg * nw) {
+        int j[kFind], lo[kFind];
+#pragma unroll
+        for (int z = 0; z < kFind; z++) {
+          const int t = b + 64 * z + lane;
+          j[z] = t < nu ? cols[u0 + t] : 0;
+          lo[z] = lo0;
+        }
+        for (int st = top; st > 0; st /= 2)
+#pragma unroll
+          for (int z = 0; z < kFind; z++) {
+            const int at = lo[z] + st;
+            if (at <= nb && scol[at - 1] < j[z]) lo[z] = at;
+          }
+#pragma unroll
+        for (int z = 0; z < kFind; z++) {
+          const int t = b + 64 * z + lane;
+          if (t < nu && lo[z] < nb && scol[lo[z]] == j[z])
+            h[lo[z]] = (unsigned short)(t + 1);
+        }
       }
+      turn = (b - nu) / kSeg;  // segments past this pivot's end
     }
-    __syncthreads();
   };
-  int kb = 0, kw = min(nbatch, dl);  // the window: pivots [kb, kw)
-  if (dl > 0) prepare(0, kw);
+  // prepared pivots [kb, kw): runs are of at most nbatch, so that the next
+  // ones can be prepared while a run's L_ik are formed
+  int kb = 0, kw = min(nwin, dl);
+  if (dl > 0) {
+    prepare(0, kw, 0);
+    __syncthreads();
+  }
   while (kb < dl) {
-    int pe = kw;  // the run [kb, pe)
+    int pe = min(kw, kb + nbatch);  // the run [kb, pe)
     if (kFlow) {
-      flow_wait<false>(scol, dl, kb, s_rdy, par, f);
+      flow_wait<false>(scol, dl, pe < dl ? min(pe, kb + kRunLeast) - 1 : kb, s_rdy,
+                       par, f);
       pe = min(pe, s_rdy[par]);
     }
-    const int np = pe - kb, sb = kb % nbatch;
+    const int np = pe - kb, sb = kb % nwin;
+    const int kn = min(kb + nwin, dl);  // pivots [kw, kn) are prepared now
     // slot of the run's pivot p
-    auto slot = [&](int p) { return sb + p >= nbatch ? sb + p - nbatch : sb + p; };
+    auto slot = [&](int p) { return sb + p >= nwin ? sb + p - nwin : sb + p; };
+    for (int e = tid; e < (kn - kw) * (stride / 8); e += nth) {
+      const int s = (kw + e / (stride / 8)) % nwin;
+      reinterpret_cast<int4*>(hit + s * stride)[e % (stride / 8)] =
+          make_int4(0, 0, 0, 0);
+    }
     // U_kk and the edge blocks of the pivots' U parts, and A_ik
     for (int e = tid; e < 36 * kEdge * np; e += nth) {
       const int p = e / (36 * kEdge), b = e / 36 % kEdge, q = e % 36;
@@ -629,7 +676,7 @@ __global__ void __launch_bounds__(kBatchThreads)
       for (int e = tid; e < 36 * np * np; e += nth) {
         const int pq = e / 36, m = e % 36, p = pq / np, q = pq % np;
         if (q <= p) continue;
-        const int v = hit[slot(p) * maxlen + kb + q];
+        const int v = hit[slot(p) * stride + kb + q];
         if (v)
           s_uq[batch_pair(p, q)][m] = load_pivot<T, kFlow>(
               vals + 36 * (size_t)(s_u0[slot(p)] + v - 1) + m,
@@ -638,7 +685,7 @@ __global__ void __launch_bounds__(kBatchThreads)
     // the blocks past the run's L part that a pivot of the run updates
     for (int pl = pe + tid; pl < nb; pl += nth) {
       unsigned any = 0;
-      for (int p = 0; p < np; p++) any |= hit[slot(p) * maxlen + pl];
+      for (int p = 0; p < np; p++) any |= hit[slot(p) * stride + pl];
       if (any) list[atomicAdd(&s_cnt, 1)] = (unsigned short)pl;
     }
     __syncthreads();
@@ -649,7 +696,7 @@ __global__ void __launch_bounds__(kBatchThreads)
     T* A = nullptr;
     auto load_u = [&](int p) {  // false: pivot p does not update the block
       const int s = slot(p);
-      const int tt = pl >= 0 ? (int)hit[s * maxlen + pl] - 1 : -1;
+      const int tt = pl >= 0 ? (int)hit[s * stride + pl] - 1 : -1;
       if (tt < 0) return false;
       const int nu = s_nu[s];
       if (kFlow && edge_block<T>(tt, nu)) {
@@ -682,7 +729,9 @@ __global__ void __launch_bounds__(kBatchThreads)
       on = load_u(0);
     };
     load_item(tid);
-    if (tid < 64) {
+    if (tid >= 64) {
+      if (kn > kw) prepare(kw, kn, 1);
+    } else {
       // wavefront 0: L_ik of each pivot, each applied to the run's later
       // L-part blocks before the next is formed
       for (int p = 0; p < np; p++) {
@@ -706,7 +755,7 @@ __global__ void __launch_bounds__(kBatchThreads)
         __builtin_amdgcn_wave_barrier();
         for (int e = tid; e < 36 * (np - 1 - p); e += 64) {
           const int q = p + 1 + e / 36, r = e % 36 / 6, c = e % 6;
-          if (!hit[slot(p) * maxlen + kb + q]) continue;
+          if (!hit[slot(p) * stride + kb + q]) continue;
           const T* U = s_uq[batch_pair(p, q)];
           T acc = 0;
 #pragma unroll
@@ -753,18 +802,7 @@ __global__ void __launch_bounds__(kBatchThreads)
         for (int c = 0; c < C; c++) A[6 * r + c] = a[r][c];
     }
     __syncthreads();
-    // the run's slots are free: clear their hits, prepare the next pivots
-    for (int p = 0; p < np; p++) {
-      const int s = slot(p);
-      for (int t = tid; t < s_nu[s]; t += nth) {
-        const int q = upos[s * maxlen + t];
-        if (q >= 0) hit[s * maxlen + q] = 0;
-      }
-    }
-    __syncthreads();
     kb = pe;
-    const int kn = min(kb + nbatch, dl);
-    if (kn > kw) prepare(kw, kn);
     kw = kn;
   }
   __syncthreads();
@@ -2633,15 +2671,15 @@ int ilu_factor(gf_ilu h, T* vals, int* zero_pivot) {
     // two workgroups per CU where the LDS allows
     const size_t cap2 = std::min(batch_cap[ti], batch_cap2[ti]);
     for (int nbt = gf::kIluBatch; nbt >= 1 && !nbatch; nbt--)
-      if (gf::batch_lds_per_pos(nbt) * maxlen <= cap2) nbatch = nbt;
+      if (gf::batch_lds(nbt, maxlen) <= cap2) nbatch = nbt;
     for (int nbt = gf::kIluBatch; nbt >= 1 && !nbatch; nbt--)
-      if (gf::batch_lds_per_pos(nbt) * maxlen <= batch_cap[ti]) nbatch = nbt;
+      if (gf::batch_lds(nbt, maxlen) <= batch_cap[ti]) nbatch = nbt;
     if (const char* benv = getenv("GPUFEM_ILU_BATCH_N"))
       nbatch = std::min(nbatch, std::max(1, atoi(benv)));
     const char* kenv = getenv("GPUFEM_ILU_GLOBAL_KERNEL");
     if (kenv && std::string(kenv) == "pivot") nbatch = 0;
   }
-  const size_t bdyn = gf::batch_lds_per_pos(nbatch) * (size_t)maxlen;
+  const size_t bdyn = gf::batch_lds(nbatch, maxlen);
   auto launch_global = [&](bool flow, const int* rows, int cnt,
                            const gf::Flow& f) {
     if (nbatch > 0) {
