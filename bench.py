@@ -240,8 +240,12 @@ def live_pmc_traffic(args):
         units = max(1, len(f) // launches_per_unit)
         return (sum(f) * 1024 * ff + sum(w) * 1024 * wf) / units
 
-    lo = bytes_of("trsv_syncfree_kernel<double, true")
-    up = bytes_of("trsv_syncfree_kernel<double, false")
+    # rows in groups, or row by row where the pattern has no chains
+    def sweep_of(lower):
+        return (bytes_of(f"trsv_group_kernel<double, {lower}")
+                or bytes_of(f"trsv_syncfree_kernel<double, {lower}"))
+
+    lo, up = sweep_of("true"), sweep_of("false")
     nasm = len(vals("jacobian_mfma_kernel<true>", "FETCH_SIZE"))
     return {"sweep_bytes_per_launch": (None if lo is None or up is None
                                        else (lo + up) / 2),
@@ -590,7 +594,7 @@ def main():
         "paths": {k: {kk: vv for kk, vv in v.items() if kk != "x_host"}
                   for k, v in results.items()},
         "roofline": {"bound": "hbm",
-                     "kernel": "trsv_syncfree_kernel<double> (L and U)",
+                     "kernel": "trsv_group_kernel<double> (L and U)",
                      "achieved": sweep_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": sweep_gbs / HBM_PEAK_GBS,
                      "traffic": (pmc["sweep_bytes_per_launch"] if pmc
@@ -606,7 +610,7 @@ def main():
         "residual_floor": floor,
         # the dominant kernel of the mixed paths (FP32 factors and vectors)
         "roofline_fp32_sweep": {
-            "bound": "hbm", "kernel": "trsv_syncfree_kernel<float> (L and U)",
+            "bound": "hbm", "kernel": "trsv_group_kernel<float> (L and U)",
             "achieved": sweep32_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": sweep32_gbs / HBM_PEAK_GBS,
             "bytes_per_launch": sweep32_bytes_launch,

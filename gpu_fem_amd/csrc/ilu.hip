@@ -276,24 +276,25 @@ __device__ __forceinline__ void flow_publish(int i, const Flow& f) {
 template <typename T>
 __device__ __forceinline__ void factor_diag(T (&d)[6], int lane, int i,
                                             int* pivot) {
+  bool live = true;  // (uniform) no zero pivot so far
+#pragma unroll
   for (int c = 0; c < 6; c++) {
+    if (!live) continue;
     T u[6];
 #pragma unroll
-    for (int m = 0; m < 6; m++) u[m] = read_lane(d[m], c);
-    T piv = u[0], dc = d[0];
-#pragma unroll
-    for (int m = 1; m < 6; m++) {
-      piv = m == c ? u[m] : piv;
-      dc = m == c ? d[m] : dc;
-    }
-    if (piv == T(0)) {
+    for (int m = c; m < 6; m++) u[m] = read_lane(d[m], c);
+    if (u[c] == T(0)) {
       if (lane == 0) atomicMin(pivot, i);
-      break;
+      live = false;
+      continue;
     }
-    const T l = dc / piv;
+    if (c == 5) continue;  // no row below
+    const T l = d[c] / u[c];
+    if (lane > c) {
+      d[c] = l;
 #pragma unroll
-    for (int m = 0; m < 6; m++)
-      if (lane > c && m >= c) d[m] = m == c ? l : d[m] - l * u[m];
+      for (int m = c + 1; m < 6; m++) d[m] = d[m] - l * u[m];
+    }
   }
 }
 
