@@ -944,13 +944,19 @@ __global__ void __launch_bounds__(kThreads)
   T uv[kIluPairs][6], un[kIluPairs][6];
   int pc[kIluCols];
   T pd = T(0);
+  // (block, column) pairs of a pivot: w0, w0 + sn, ...  Where the last pivot
+  // was waited for (a chain), they are left to wavefronts 1 .., and wavefront
+  // 0 updates the diagonal block and factors it meanwhile: 0.7 us of the 5.2
+  // of a row of the chain.
+  bool split = false;
   auto load_u = [&](int kl, T (&dst)[kIluPairs][6]) {
     const int u0 = kl < dl ? ubs[2 * kl] : 0;
     const int nu = kl < dl ? ubs[2 * kl + 1] - u0 : 0;
+    const int w0 = split ? tid - 64 : tid, sn = split ? nth - 64 : nth;
 #pragma unroll
     for (int sp = 0; sp < kIluPairs; sp++) {
-      const int w = tid + sp * nth;
-      const bool ok = w < 6 * nu;
+      const int w = w0 + sp * sn;
+      const bool ok = w0 >= 0 && w < 6 * nu;
       const T* U =
           vals + 36 * (size_t)(u0 + (ok ? w / 6 : 0)) + (ok ? w % 6 : 0);
       const bool edge = edge_block<T>(w / 6, nu);
@@ -996,15 +1002,47 @@ __global__ void __launch_bounds__(kThreads)
     for (int t = tid; t < nu; t += nth) pos[0][t] = find(cols[u0 + t], 1);
     load_cols(1);
   }
+  // the diagonal block (no pivoting), by wavefront 0
+  T* const D = row + 36 * dl;
+  auto factor = [&]() {
+    const int r = tid < 6 ? tid : 5;
+    T d[6];
+#pragma unroll
+    for (int m = 0; m < 6; m++) d[m] = D[6 * r + m];
+    factor_diag(d, tid, i, pivot);
+    if (tid < 6) {
+#pragma unroll
+      for (int m = 0; m < 6; m++) D[6 * r + m] = d[m];
+    }
+  };
   bool have = false;  // pivot kl's values are staged
   __syncthreads();
   for (int kl = 0; kl < dl; kl++) {
     const int cur = kl & 1;
     const int u0 = ubs[2 * kl], nu = ubs[2 * kl + 1] - u0;
+    bool upd = false;  // the last pivot updates the diagonal block
+    // wavefront 0, which has no pairs of it: column tid % 6 of U_ki into uv[0]
+    auto load_ud = [&]() {
+      int at = -1;
+      for (int t = 0; t < nu && at < 0; t += 64) {
+        const unsigned long long m =
+            __ballot(t + tid < nu && pos[cur][t + tid] == dl);
+        if (m) at = t + __ffsll((long long)m) - 1;
+      }
+      upd = at >= 0;
+      if (!upd) return;
+      const T* U = vals + 36 * (size_t)(u0 + at) + tid % 6;
+      const bool edge = edge_block<T>(at, nu);
+#pragma unroll
+      for (int m = 0; m < 6; m++)
+        uv[0][m] = load_pivot<T, kFlow>(U + 6 * m, edge);
+    };
     if (!have) {
       wait_for(kl);
+      split = kFlow && kl == dl - 1;
       load_u(kl, uv);
       load_diag(kl);
+      if (split && tid < 64) load_ud();
       stage_diag(cur);
       __syncthreads();
     }
@@ -1040,12 +1078,25 @@ __global__ void __launch_bounds__(kThreads)
     }
     __syncthreads();
     // A_ij -= L_ik U_kj on the LDS row
+    const int w0 = split ? tid - 64 : tid, sn = split ? nth - 64 : nth;
+    if (split && tid < 64) {
+      if (upd && tid < 36) {
+        const int r = tid / 6;
+        T v = 0;
+#pragma unroll
+        for (int m = 0; m < 6; m++) v += lik[6 * r + m] * uv[0][m];
+        row[36 * dl + tid] -= v;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      factor();
+    }
 #pragma unroll
     for (int sp = 0; sp < kIluPairs; sp++) {
-      const int w = tid + sp * nth;
-      if (w < 6 * nu) {
+      const int w = w0 + sp * sn;
+      if (w0 >= 0 && w < 6 * nu) {
         const int pl = pos[cur][w / 6], c = w % 6;
-        if (pl >= 0) {
+        if (pl >= 0 && !(split && pl == dl)) {
 #pragma unroll
           for (int r = 0; r < 6; r++) {
             T v = 0;
@@ -1056,9 +1107,9 @@ __global__ void __launch_bounds__(kThreads)
         }
       }
     }
-    for (int w = tid + kIluPairs * nth; w < 6 * nu; w += nth) {
+    for (int w = w0 + kIluPairs * sn; w0 >= 0 && w < 6 * nu; w += sn) {
       const int pl = pos[cur][w / 6], c = w % 6;
-      if (pl < 0) continue;
+      if (pl < 0 || (split && pl == dl)) continue;
       const T* U = vals + 36 * (size_t)(u0 + w / 6) + c;
       const bool edge = edge_block<T>(w / 6, nu);
       T um[6];
@@ -1080,20 +1131,10 @@ __global__ void __launch_bounds__(kThreads)
       for (int m = 0; m < 6; m++) uv[sp][m] = un[sp][m];
     have = next;
   }
-  // factor the diagonal block (no pivoting)
-  T* D = row + 36 * dl;
-  if (tid < 64) {
-    const int r = tid < 6 ? tid : 5;
-    T d[6];
-#pragma unroll
-    for (int m = 0; m < 6; m++) d[m] = D[6 * r + m];
-    factor_diag(d, tid, i, pivot);
-    if (tid < 6) {
-#pragma unroll
-      for (int m = 0; m < 6; m++) D[6 * r + m] = d[m];
-    }
+  if (!split) {
+    if (tid < 64) factor();
+    __syncthreads();
   }
-  __syncthreads();
   // U_ij = L_ii^-1 A_ij for the blocks right of the diagonal
   const int nr = nb - (dl + 1);
   for (int w = tid; w < 6 * nr; w += nth) {
