@@ -4,7 +4,9 @@
 // residual path add_residual_cpu (include/base/elem_group.h:40-79) and
 // add_energy (assembler.h:198-229).
 //
-// Layout: one 64-lane workgroup per element.
+// The default kernels (jacobian_mfma_kernel, tangent_kernel, residual_kernel)
+// take four elements a wavefront, see there.  Layout of jacobian_kernel
+// (GPUFEM_ASSEMBLY=element): one 64-lane workgroup per element.
 //   stage 1  lanes 0-3: node frames; lanes 4-8: tying-point geometry
 //   stage 2  lanes 0-3: quadrature frames; lanes 4-8: tying normals
 //   stage 3  lanes 0-23: column j of B_q (4 x 9) and D_q = detXd C B_q -> LDS

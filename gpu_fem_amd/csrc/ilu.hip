@@ -19,7 +19,8 @@
 //     instead.  The arithmetic of a row is the same either way, so the two
 //     schedules give bitwise-identical factors.
 //   sweeps: over groups of up to eight rows of a chain (trsv_group_kernel,
-//     below) or, for patterns without such chains, over rows.  One
+//     below) or, for patterns without such chains, over rows; small systems
+//     in one workgroup (trsv_small_kernel).  Otherwise one
 //     persistent launch per sweep, synchronised through the data:
 //     the output vector is pre-filled with a signalling-NaN sentinel, each
 //     entry is written once with a relaxed agent-scope atomic store, and a
@@ -880,9 +881,10 @@ constexpr int kIluCols = 4;   // prefetched column indices per staging thread
 // wavefronts a CU, one 512-thread row or three 256-thread ones, and a short
 // row spends its time in per-row latency (ticket, loads of its pattern and
 // pivot bounds, diagonal factorisation, write-back and release), not in its
-// few pivot updates.  400x400 plate, AMD + ILU(96), FP64 factorisation:
-// 135 ms with 512 threads throughout, 129 ms with rows up to 128 blocks in
-// 256-thread workgroups, 123 ms up to 256 or 512 blocks.  (The staging
+// few pivot updates.  400x400 plate, AMD + ILU(96), FP64 / FP32
+// factorisation: 83.4 / 59.1 ms with 512 threads throughout, 76.8 / 58.9 with
+// rows up to 128 blocks in 256-thread workgroups, 73.0 / 55.4 up to 256; 75x150
+// cylinder FP64 10.33, 9.93 and 9.86.  (The staging
 // threads hold 4 * (256 - 6) column indices: pivot U parts up to 1,000.)
 constexpr int kIluShortThreads = 256;
 constexpr int kIluShortRow = 256;  // longest row (blocks) taken that way
