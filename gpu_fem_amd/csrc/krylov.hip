@@ -495,7 +495,7 @@ __global__ void __launch_bounds__(256)
 // a1 = sum_{i<j} c1[i] V_i[t], and a2 with c2 (may be null).  Vector i goes to
 // running sum i % kParts: with one sum an entry every load waited for the
 // previous one (10x10 plate, 80 vectors and their preconditioned ones: 12.8 us
-// a step, 5.4 us with eight; eight lanes an entry instead measured the same
+// a step, 6.4 us with eight; eight lanes an entry instead measured the same
 // from 1,700 to 88,000 entries).
 constexpr int kParts = 8;
 __device__ __forceinline__ double parts_total(const double (&a)[kParts]) {
