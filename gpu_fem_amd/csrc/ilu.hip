@@ -1775,6 +1775,18 @@ __global__ void __launch_bounds__(kSmallThreads)
   small_sweep<T, false>(S, S.nulev, xs);
 }
 
+// Neither infinite nor NaN.  Sweep pair of a 256x256 plate, RCM ILU(3), with
+// the check in front of a group's stores, integer comparison / v_cmp_class /
+// no check: FP64 2.41 / 2.44 / 2.37 ms, FP32 2.53 / 2.46 / 2.43 ms.
+__device__ __forceinline__ bool finite(double v) {
+  const unsigned hi =
+      (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32);
+  return hi << 1 < 0xffe00000u;
+}
+__device__ __forceinline__ bool finite(float v) {
+  return !__builtin_amdgcn_classf(v, 0x207);
+}
+
 // ---- sweeps over row groups ----
 // A level of a few rows costs a row's whole latency, from a dependency's
 // store to the row's own (1.2 us on an idle device, 1.6-2.1 us under load).
@@ -1841,6 +1853,8 @@ __global__ void __launch_bounds__(kGroupThreads, 4)
   __shared__ T ext[kGroupRows][60];    // external sums of a wavefront's slots
   __shared__ T coef[6 * kGroupRows][6 * kGroupRows];  // [column][scalar row]
   __shared__ T diag[6 * kGroupRows];   // U: diagonal entries
+  // of a row: bit q: block (row, row q) exists; row; dependency blocks
+  __shared__ int4 info[kGroupRows];
   // group count for which a wavefront has written its coefficients, its sums
   __shared__ int staged[kGroupRows], arrived[kGroupRows];
   __shared__ int s_ticket;
@@ -1946,6 +1960,11 @@ __global__ void __launch_bounds__(kGroupThreads, 4)
           if (q == p && (kLower ? c >= a : c <= a)) v[z] = T(0);
           coef[6 * q + c][6 * p + a] = v[z];
         }
+        const int i = 32 + 8 * p + lane % 8;
+        const int b0 = __shfl(rec0, i & 63, 64), b1 = __shfl(rec1, i & 63, 64);
+        const unsigned blocks = (unsigned)__ballot((i < 64 ? b0 : b1) >= 0);
+        const int row = __builtin_amdgcn_readlane(rec0, 8 + p);
+        if (lane == 0) info[p] = make_int4(blocks & 255, row, k0, k1);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         if (lane == 0)
           __hip_atomic_store(&staged[w], seq, __ATOMIC_RELAXED,
@@ -2074,6 +2093,7 @@ __global__ void __launch_bounds__(kGroupThreads, 4)
         for (int u = sp; u < kGroupRows; u += n) mine |= 1u << u;
         bool taken = !live;
         T es = T(0);  // external sum of this lane's row
+        const T s0 = s;
         unsigned arr = 0;  // wavefronts seen to have arrived
 #pragma unroll
         for (int q = 0; q < kGroupRows; q++) {
@@ -2114,9 +2134,49 @@ __global__ void __launch_bounds__(kGroupThreads, 4)
               const T y = read_lane(kLower ? s : s * dinv, 6 * q + m);
               s -= cf[q & 1][m] * y;
             }
-            if (sp == q && live)
-              store_value(x + 6 * (size_t)srow + sa, kLower ? s : s * dinv);
+            // Blocks that do not exist, the other triangle and the group's
+            // own blocks in the external sums are products with a zero, NaN
+            // where the other factor is infinite or NaN: a finite value is
+            // right, the others are formed again below.
+            const T v = kLower ? s : s * dinv;
+            if (sp == q && finite(v))
+              store_value(x + 6 * (size_t)srow + sa, v);
           }
+        }
+        const bool odd = live && !finite(kLower ? s : s * dinv);
+        if (__any(odd)) {
+          // the record once more, without products that are not in the sums
+          const int lr = live ? sp : 0;
+          const int4 in = info[lr];
+          if (live && !finite(es)) {
+            bool inf = false;  // in a coefficient of the group's own blocks
+            for (int c = 0; c < 6 * lr; c++) inf |= !finite(coef[c][lc]);
+            if (inf) {
+              es = T(0);
+              for (int k = in.z; k < in.w; k++) {
+                const int j = cols[k];
+                bool own = false;
+                for (int u = 0; u < n; u++) own |= j == info[u].y;
+                for (int c = 0; c < 6 && !own; c++)
+                  es += lu[36 * (size_t)k + 6 * sa + c] *
+                        __builtin_bit_cast(T, load_bits(x + 6 * (size_t)j + c));
+              }
+            }
+          }
+          s = s0 - es;
+#pragma unroll 1
+          for (int q = 0; q < n; q++) {
+            const bool below = sp > q && (in.x >> q & 1);
+#pragma unroll 1
+            for (int z = 0; z < 6; z++) {
+              const int m = kLower ? z : 5 - z;
+              const T y = read_lane(kLower ? s : s * dinv, 6 * q + m);
+              const bool tri = sp == q && (kLower ? sa > m : sa < m);
+              if (live && (below || tri)) s -= coef[6 * q + m][lc] * y;
+            }
+          }
+          if (odd)
+            store_value(x + 6 * (size_t)srow + sa, kLower ? s : s * dinv);
         }
       }
     }
