@@ -123,8 +123,14 @@ __global__ void permute_kernel(int nnodes, const int* __restrict__ perm,
 // column indices, blocks and entries of x of up to kSpmvBlocks blocks are in
 // flight together: a row waits for memory twice (indices, entries), not once
 // a block.  400x400 plate (1.45 M blocks, nine a row), FP64 / FP32: 111 / 44
-// us with one block at a time, 95 / 46 with 2, 92 / 44 with 5, 89 / 39 with
-// 9, the row of a node among quadrilaterals (4.95 TB/s, the rate of a copy).
+// us with one block at a time, 95 / 46 with 2, 92 / 44 with 5, 81 / 35 with
+// 9, the row of a node among quadrilaterals (5.3 TB/s).  A wavefront none of
+// whose rows has a block u any more takes no further ones: with all nine of
+// the last group loaded (a row's missing ones from its first block) rows of
+// 10 to 17 blocks were slower than one at a time (128x128 plate RCM ILU(1)
+// FP64 12.8 us one at a time, 14.7 so, 12.8 now; wingbox K 15.3, 16.7, 14.4),
+// and so were rows of 3 (25.5, 37.2, 25.9).  The first group asks three times
+// only: a branch a block costs 6% on the 128x128 plate's rows of nine.
 constexpr int kSpmvBlocks = 9;
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -138,11 +144,16 @@ __global__ void __launch_bounds__(256)
   if (row >= nnodes) return;
   const int k1 = rowp[row + 1];
   T acc = 0;
+  bool more = false;  // past the first group
   for (int k = rowp[row]; k < k1; k += kSpmvBlocks) {
     T a[kSpmvBlocks][6], xb[kSpmvBlocks][6];
     int j[kSpmvBlocks];
+    auto ask = [&](int u) {  // whether any row still has blocks
+      return u && (more || u == 1 || u == 3 || u == 5);
+    };
 #pragma unroll
     for (int u = 0; u < kSpmvBlocks; u++) {
+      if (ask(u) && !__any(k + u < k1)) break;
       const int q = k + u < k1 ? k + u : k;
       j[u] = cols[q];
       const T* ap = vals + 36 * (size_t)q + 6 * r;
@@ -150,14 +161,17 @@ __global__ void __launch_bounds__(256)
       for (int c = 0; c < 6; c++) a[u][c] = ap[c];
     }
 #pragma unroll
-    for (int u = 0; u < kSpmvBlocks; u++)
+    for (int u = 0; u < kSpmvBlocks; u++) {
+      if (ask(u) && !__any(k + u < k1)) break;
 #pragma unroll
       for (int c = 0; c < 6; c++) xb[u][c] = x[6 * (size_t)j[u] + c];
+    }
 #pragma unroll
     for (int u = 0; u < kSpmvBlocks; u++)
       if (k + u < k1)
 #pragma unroll
         for (int c = 0; c < 6; c++) acc += a[u][c] * xb[u][c];
+    more = true;
   }
   y[6 * (size_t)row + r] = acc;
 }
