@@ -107,6 +107,7 @@ _SIGS = {
     "gf_ilu_create": [_P, _I, _P, _P, ctypes.POINTER(_P)],
     "gf_ilu_destroy": [_P],
     "gf_ilu_info": [_P, _PI, _PI, _PI],
+    "gf_ilu_sweep_info": [_P, _PI, _PI, _PI],
     "gf_ilu_device_rowp": [_P],
     "gf_ilu_device_cols": [_P],
     "gf_ilu_check": [_P],
@@ -433,6 +434,16 @@ class Ilu:
                           ctypes.byref(c))
         return {"nnzb": a.value, "levels_lower": b.value,
                 "levels_upper": c.value}
+
+    SWEEPS = ("levels", "chains", "rows", "groups", "small")
+
+    def sweep_info(self):
+        """How the sweeps run (one of SWEEPS) and their numbers of items."""
+        a, b, c = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+        self.ctx.check(lib().gf_ilu_sweep_info(
+            self.h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(c)))
+        return {"kind": self.SWEEPS[a.value], "lower": b.value,
+                "upper": c.value}
 
     def factor(self, d_vals):
         zp = ctypes.c_int(-1)

@@ -2453,13 +2453,15 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
   int side = 0;  // most blocks of a row on one side of the diagonal
   for (int i = 0; i < n; i++)
     side = std::max({side, diag[i] - rowp[i], rowp[i + 1] - diag[i] - 1});
-  // (GPUFEM_TRSV set to anything else: the kernels of larger systems)
+  const std::string mode = tenv ? tenv : "";
   if (!tenv)
     h->small = side <= gf::kSmallBlocks && gf::small_sweeps(
                    n, (int)std::max(h->lptr.size(), h->uptr.size()) - 1);
-  else if (std::string(tenv) == "small")
+  else if (mode == "small")
     h->small = side <= gf::kSmallBlocks && n <= gf::kSmallRows;
-  if (!use_chains && !h->level_sweeps && !h->small) {
+  // groups: whatever their ratio.  Any other value: row by row.
+  const bool force = mode == "groups";
+  if (!h->small && (!tenv || force || mode == "small")) {
     gf::SweepGroups sg;
     gf::sweep_groups(n, rowp, cols, diag.data(), h->lptr, lrows, sg);
     auto ur = std::async(policy, [&] {
@@ -2471,8 +2473,8 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
     const int gu = ur.get();
     const size_t most = gf::kGroupInts * gf::group_records_max(n);
     if (lgr.size() <= most && ugr.size() <= most &&
-        gf::kGroupRatio * std::max(gl, gu) <=
-            (double)std::max(h->lptr.size(), h->uptr.size()) - 1) {
+        (force || gf::kGroupRatio * std::max(gl, gu) <=
+                      (double)std::max(h->lptr.size(), h->uptr.size()) - 1)) {
       h->nlgroup = (int)(lgr.size() / gf::kGroupInts);
       h->nugroup = (int)(ugr.size() / gf::kGroupInts);
     } else {
@@ -2609,6 +2611,23 @@ int gf_ilu_info(gf_ilu h, int* nnzb, int* nl, int* nu) {
   if (nu) *nu = (int)h->uptr.size() - 1;
   return GF_OK;
 }
+int gf_ilu_sweep_info(gf_ilu h, int* kind, int* nlower, int* nupper) {
+  if (!h) return GF_ERR_INVALID;
+  const bool levels = h->small || h->level_sweeps;
+  if (kind)
+    *kind = h->small          ? GF_SWEEP_SMALL
+            : h->level_sweeps ? GF_SWEEP_LEVELS
+            : h->nlgroup      ? GF_SWEEP_GROUPS
+            : h->lchains      ? GF_SWEEP_CHAINS
+                              : GF_SWEEP_ROWS;
+  const auto items = [&](const std::vector<int>& lptr, int groups, int chunks) {
+    return levels ? (int)lptr.size() - 1 : groups ? groups : chunks;
+  };
+  if (nlower) *nlower = items(h->lptr, h->nlgroup, h->nlchunk);
+  if (nupper) *nupper = items(h->uptr, h->nugroup, h->nuchunk);
+  return GF_OK;
+}
+
 const int* gf_ilu_device_rowp(gf_ilu h) { return h ? h->rowp : nullptr; }
 
 int gf_ilu_check(gf_ilu h) {

@@ -215,6 +215,18 @@ int gf_ilu_create(gf_context ctx, int nnodes, const int* rowp, const int* cols,
 int gf_ilu_destroy(gf_ilu ilu);
 int gf_ilu_info(gf_ilu ilu, int* nnzb, int* nlevels_lower,
                 int* nlevels_upper);
+/* How the triangular sweeps of this pattern run: by levels (a launch each),
+ * by chains or by rows (trsv_syncfree_kernel), by groups of rows
+ * (trsv_group_kernel), or both in one workgroup (trsv_small_kernel); and the
+ * items of the L and the U sweep (levels; chains, chunks of rows or group
+ * records).  The pattern decides; GPUFEM_TRSV = level, chains, groups or small
+ * (where it fits) chooses, any other value chooses rows. */
+#define GF_SWEEP_LEVELS 0
+#define GF_SWEEP_CHAINS 1
+#define GF_SWEEP_ROWS 2
+#define GF_SWEEP_GROUPS 3
+#define GF_SWEEP_SMALL 4
+int gf_ilu_sweep_info(gf_ilu ilu, int* kind, int* nlower, int* nupper);
 const int* gf_ilu_device_rowp(gf_ilu ilu);
 const int* gf_ilu_device_cols(gf_ilu ilu);
 /* GF_ERR_TIMEOUT if a sweep's bounded dependency wait expired since the last
