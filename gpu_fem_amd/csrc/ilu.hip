@@ -70,6 +70,7 @@ struct gf_ilu_s {
   int epoch = 0;
   // sweeps over row groups (trsv_group_kernel; none: nlgroup == 0)
   int *lgroup = nullptr, *ugroup = nullptr;  // group records
+  int *lgrows = nullptr, *ugrows = nullptr;  // and their rows
   int nlgroup = 0, nugroup = 0, ggrid = 0;
   // small system: both sweeps by one workgroup (trsv_small_kernel) over the
   // level-ordered rows of lmeta and umeta
@@ -2184,6 +2185,45 @@ __global__ void __launch_bounds__(kGroupThreads, 4)
   }
 }
 
+// The records of a sweep's groups from their rows, a wavefront each: lane
+// 8 p + q looks row q up in row p's blocks.  (Analysis of a 256x256 plate, RCM
+// ILU(3), with the records formed on the host and uploaded: 4.3 ms, so 2.1.)
+__global__ void __launch_bounds__(256)
+    group_records_kernel(int nrec, bool lower, const int* __restrict__ rows,
+                         const int* __restrict__ rowp,
+                         const int* __restrict__ cols,
+                         const int* __restrict__ diag, int* records) {
+  const int r = (int)(blockIdx.x * 256 + threadIdx.x) / 64;
+  const int lane = threadIdx.x % 64, p = lane / 8, q = lane % 8;
+  if (r >= nrec) return;
+  const int i = rows[kGroupRows * (size_t)r + p];
+  const int j = rows[kGroupRows * (size_t)r + q];
+  int k0 = -1, k1 = -1, blk = -1;
+  if (i >= 0) {
+    const int d = diag[i];
+    k0 = lower ? rowp[i] : d + 1;
+    k1 = lower ? d : rowp[i + 1];
+    if (q == p) {
+      blk = d;
+    } else if (q < p) {
+      int lo = k0, hi = k1;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (cols[mid] < j)
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      if (lo < k1 && cols[lo] == j) blk = lo;
+    }
+  }
+  const int n = __popcll(__ballot(i >= 0)) / 8;
+  int* const rec = records + kGroupInts * (size_t)r;
+  rec[32 + lane] = blk;
+  if (q < 4)
+    rec[8 * q + p] = q == 0 ? (p == 0 ? n : -1) : q == 1 ? i : q == 2 ? k0 : k1;
+}
+
 // Row groups of a pattern (host).  A row joins the group of the child whose
 // first U column it is (the child latest in level order, when it has
 // several), as long as the group stays free of cycles: no row outside the
@@ -2198,85 +2238,125 @@ struct SweepGroups {
   std::vector<SweepGroup> g;
   std::vector<int> gid;    // group of a row
   std::vector<int> llev;   // group level of the lower sweep
+  int nllev = 0;
   std::vector<int> order;  // groups by last row
 };
-void sweep_groups(int n, const int* rowp, const int* cols, const int* diag,
-                  const std::vector<int>& lptr, const std::vector<int>& lrows,
-                  SweepGroups& sg) {
-  std::vector<int> best(n, -1), lev(n);
-  for (size_t l = 0; l + 1 < lptr.size(); l++)
-    for (int q = lptr[l]; q < lptr[l + 1]; q++) lev[lrows[q]] = (int)l;
-  for (int i = 0; i < n; i++) {
-    if (diag[i] + 1 >= rowp[i + 1]) continue;
-    const int j = cols[diag[i] + 1];
-    if (best[j] < 0 || lev[i] >= lev[best[j]]) best[j] = i;
-  }
-  std::vector<int>& gid = sg.gid;
-  gid.assign(n, -1);
+// The groups, and each row's level in the lower sweep (lev, returned: their
+// number).  One pass over the L part: the group levels are kept per row, with
+// the rows of row i's own group at -1 meanwhile, so that an entry costs two
+// loads and a store (400x400 plate, AMD + ILU(96), one core: 14 ms; 23 with
+// the levels first and the group of every entry looked up).
+int sweep_groups(int n, const int* rowp, const int* cols, const int* diag,
+                 SweepGroups& sg, std::vector<int>& levels) {
+  levels.assign(n, 0);
+  sg.gid.assign(n, -1);
   sg.g.clear();
   sg.g.reserve(n / 2 + 1);
   sg.llev.clear();
-  std::vector<char> closed;  // a row outside depends on a member
+  sg.llev.reserve(n / 2 + 1);
+  sg.nllev = 0;
+  // child of which a row is the first U column; group level of a row; U
+  // blocks of a row up to here are known to be in its group; a row outside
+  // the group depends on the row
+  std::vector<int> best_(n, -1), glev_(n), next_(n);
+  std::vector<unsigned char> used_(n, 0);
+  int *lev = levels.data(), *gid = sg.gid.data(), *best = best_.data(),
+      *glev = glev_.data(), *next = next_.data();
+  unsigned char* used = used_.data();
+  int nlev = 0;
   for (int i = 0; i < n; i++) {
+    const int c = best[i], d = diag[i];
     int g = -1;
-    const int c = best[i];
     if (c >= 0) {
       g = gid[c];
       const SweepGroup& m = sg.g[g];
-      bool ok = m.n < kGroupRows && m.row[m.n - 1] == c && !closed[g];
-      for (int q = 0; ok && q < m.n; q++)
-        for (int k = diag[m.row[q]] + 1;
-             ok && k < rowp[m.row[q] + 1] && cols[k] < i; k++)
-          ok = gid[cols[k]] == g;
+      bool ok = m.n < kGroupRows && m.row[m.n - 1] == c;
+      if (c < i - 1) {  // (no row between them otherwise)
+        for (int q = 0; ok && q < m.n; q++) ok = !used[m.row[q]];
+        for (int q = 0; ok && q < m.n; q++) {
+          const int r = m.row[q], k1 = rowp[r + 1];
+          int k = next[r];
+          while (k < k1 && cols[k] < i && gid[cols[k]] == g) k++;
+          next[r] = k;
+          ok = k == k1 || cols[k] >= i;
+        }
+      }
       if (!ok) g = -1;
     }
     if (g < 0) {
       g = (int)sg.g.size();
       sg.g.emplace_back();
       sg.llev.push_back(0);
-      closed.push_back(0);
     }
-    gid[i] = g;
+    SweepGroup& m = sg.g[g];
     // the groups this row depends on take no more rows, so their levels are
     // final
-    int l = sg.llev[g];
-    for (int k = rowp[i]; k < diag[i]; k++) {
-      const int h = gid[cols[k]];
-      if (h == g) continue;
-      closed[h] = 1;
-      l = std::max(l, sg.llev[h] + 1);
+    int l = 0, gl = -1, k = rowp[i];
+    const int first = m.n ? m.row[0] : i;
+    for (; k < d && cols[k] < first; k++) {
+      const int j = cols[k];
+      l = std::max(l, lev[j] + 1);
+      gl = std::max(gl, glev[j]);
+      used[j] = 1;
     }
-    sg.llev[g] = l;
-    sg.g[g].row[sg.g[g].n++] = i;
+    for (; k < d; k++) {  // its own group's rows among others
+      const int j = cols[k];
+      l = std::max(l, lev[j] + 1);
+      if (gid[j] == g) continue;
+      gl = std::max(gl, glev[j]);
+      used[j] = 1;
+    }
+    lev[i] = l;
+    gid[i] = g;
+    next[i] = d + 1;
+    m.row[m.n++] = i;
+    glev[i] = sg.llev[g];
+    if (gl + 1 > sg.llev[g]) {
+      sg.llev[g] = gl + 1;
+      for (int q = 0; q < m.n; q++) glev[m.row[q]] = gl + 1;
+    }
+    sg.nllev = std::max(sg.nllev, sg.llev[g] + 1);
+    nlev = std::max(nlev, l + 1);
+    if (d + 1 < rowp[i + 1]) {
+      const int j = cols[d + 1];
+      if (best[j] < 0 || l >= lev[best[j]]) best[j] = i;
+    }
   }
   sg.order.clear();
+  sg.order.reserve(sg.g.size());
   for (int i = 0; i < n; i++) {
     const SweepGroup& m = sg.g[gid[i]];
     if (m.row[m.n - 1] == i) sg.order.push_back(gid[i]);
   }
+  return nlev;
 }
 
-// Group records of one sweep, in hand-out order (by group level).
-// level: the group level of each record; returns the number of levels.
-int group_records(const int* rowp, const int* cols, const int* diag,
-                  const SweepGroups& sg, bool lower, std::vector<int>& out,
-                  std::vector<int>& level) {
-  const int ng = (int)sg.g.size();
-  std::vector<int> lev(ng, 0);
+// Group levels of the upper sweep; returns their number.
+int upper_group_levels(const int* rowp, const int* cols, const int* diag,
+                       const SweepGroups& sg, std::vector<int>& lev) {
+  std::vector<int> glev(sg.gid.size(), -1);  // of a row
+  lev.assign(sg.g.size(), 0);
   int nlev = 0;
-  for (int q = 0; q < ng; q++) {
-    const int g = sg.order[lower ? q : ng - 1 - q];
-    const SweepGroup& m = sg.g[g];
-    int l = lower ? sg.llev[g] : 0;
-    if (!lower)
-      for (int z = 0; z < m.n; z++)
-        for (int k = diag[m.row[z]] + 1; k < rowp[m.row[z] + 1]; k++) {
-          const int h = sg.gid[cols[k]];
-          if (h != g) l = std::max(l, lev[h] + 1);
-        }
-    lev[g] = l;
+  for (size_t q = sg.order.size(); q-- > 0;) {
+    const SweepGroup& m = sg.g[sg.order[q]];
+    int l = -1;
+    for (int z = 0; z < m.n; z++)
+      for (int k = diag[m.row[z]] + 1; k < rowp[m.row[z] + 1]; k++)
+        l = std::max(l, glev[cols[k]]);
+    l++;
+    for (int z = 0; z < m.n; z++) glev[m.row[z]] = l;
+    lev[sg.order[q]] = l;
     nlev = std::max(nlev, l + 1);
   }
+  return nlev;
+}
+
+// Rows of the group records of one sweep, kGroupRows each (-1: none), in
+// hand-out order (by group level).
+// lev, nlev: the groups' levels; level: the level of each record.
+void group_rows(const SweepGroups& sg, bool lower, const std::vector<int>& lev,
+                int nlev, std::vector<int>& out, std::vector<int>& level) {
+  const int ng = (int)sg.g.size();
   std::vector<int> ptr(nlev + 1, 0);
   for (int g = 0; g < ng; g++) ptr[lev[g] + 1]++;
   for (int l = 0; l < nlev; l++) ptr[l + 1] += ptr[l];
@@ -2288,47 +2368,30 @@ int group_records(const int* rowp, const int* cols, const int* diag,
   // Groups of one level share a record as long as it holds their rows: the
   // largest group left, then the largest that still fit.
   out.clear();
-  out.reserve((size_t)kGroupInts * (ng / 2 + 1));
+  out.reserve(sg.gid.size() + sg.gid.size() / 2 + 64);
   level.clear();
   std::vector<int> bySize[kGroupRows + 1];
   for (int l = 0, q0 = 0; l < nlev; q0 = ptr[l++]) {
     for (int q = ptr[l] - 1; q >= q0; q--)
       bySize[sg.g[order[q]].n].push_back(order[q]);
     for (;;) {
-      int used = 0, *rec = nullptr;
+      int used = 0;
       for (int sz = kGroupRows; sz > 0;) {
         if (sz > kGroupRows - used || bySize[sz].empty()) {
           sz--;
           continue;
         }
-        const SweepGroup& m = sg.g[bySize[sz].back()];
+        const int* row = sg.g[bySize[sz].back()].row;
         bySize[sz].pop_back();
-        if (!used) {
-          out.resize(out.size() + kGroupInts, -1);
-          rec = out.data() + out.size() - kGroupInts;
-          level.push_back(l);
-        }
-        for (int z = 0; z < sz; z++) {
-          const int i = m.row[lower ? z : sz - 1 - z], p = used + z;
-          const int k0 = lower ? rowp[i] : diag[i] + 1;
-          const int k1 = lower ? diag[i] : rowp[i + 1];
-          rec[8 + p] = i;
-          rec[16 + p] = k0;
-          rec[24 + p] = k1;
-          rec[32 + 8 * p + p] = diag[i];
-          for (int q = used; q < p; q++) {
-            const int* c = std::lower_bound(cols + k0, cols + k1, rec[8 + q]);
-            if (c < cols + k1 && *c == rec[8 + q])
-              rec[32 + 8 * p + q] = (int)(c - cols);
-          }
-        }
+        if (!used) level.push_back(l);
+        for (int z = 0; z < sz; z++)
+          out.push_back(row[lower ? z : sz - 1 - z]);
         used += sz;
-        rec[0] = used;
       }
       if (!used) break;
+      out.resize(out.size() + (kGroupRows - used), -1);
     }
   }
-  return nlev;
 }
 
 }  // namespace
@@ -2352,6 +2415,88 @@ size_t ilu_counter_bytes() {
 size_t ilu_group_bytes(size_t n) {
   return sizeof(int) * kGroupInts * group_records_max(n);
 }
+// Host analysis of a pattern: its levels, and how the sweeps run.
+int ilu_plan(int n, const int* rowp, const int* cols, IluPlan& pl,
+             std::string* why) {
+  auto fail = [&](const std::string& msg) {
+    if (why) *why = "ilu_create: " + msg;
+    return GF_ERR_INVALID;
+  };
+  pl = IluPlan{};
+  pl.diag.resize(n);
+  int maxlen = 0;
+  int side = 0;  // most blocks of a row on one side of the diagonal
+  for (int i = 0; i < n; i++) {
+    const int k0 = rowp[i], k1 = rowp[i + 1];
+    bool bad = k1 > k0 && (cols[k0] < 0 || cols[k1 - 1] >= n);
+    for (int k = k0 + 1; k < k1; k++) bad |= cols[k] <= cols[k - 1];
+    if (bad) return fail("row " + std::to_string(i) + " not sorted/in range");
+    const int d = (int)(std::lower_bound(cols + k0, cols + k1, i) - cols);
+    if (d >= k1 || cols[d] != i)
+      return fail("row " + std::to_string(i) + " has no diagonal block");
+    pl.diag[i] = d;
+    maxlen = std::max(maxlen, k1 - k0);
+    side = std::max({side, d - k0, k1 - d - 1});
+  }
+  if (maxlen > kMaxRowBlocks)
+    return fail("row length " + std::to_string(maxlen) + " exceeds " +
+                std::to_string(kMaxRowBlocks) + " blocks");
+  pl.max_row_len = maxlen;
+  const int* diag = pl.diag.data();
+  const char* tenv = getenv("GPUFEM_TRSV");
+  const std::string mode = tenv ? tenv : "";
+  pl.chains = mode == "chains";
+  pl.levels = mode == "level";
+  // The levels of the two sweeps of a large pattern are found at the same time
+  // (here, one after the other, if the library can start no thread).
+  // gf_ilu_create without row groups / with the groups' levels and records
+  // found on the host, row by row / now: 400x400 plate, AMD + ILU(96) (14 M
+  // blocks) 30.8 / 41.8 / 19.7 ms, 256x256 plate RCM ILU(3) 2.90 / 5.07 /
+  // 2.13 ms, 45x45 AMD ILU(12) 0.27 / 0.40 / 0.23 ms.
+  const auto policy = rowp[n] >= 200000
+                          ? std::launch::async | std::launch::deferred
+                          : std::launch::deferred;
+  auto upper = std::async(policy, [&] {
+    level_schedule(n, rowp, cols, false, pl.uptr, pl.urows);
+  });
+  // groups: whatever their ratio.  Any value but these: row by row.
+  const bool force = mode == "groups";
+  const bool small_fits = side <= kSmallBlocks && n <= kSmallRows;
+  const bool groups = !tenv || force || mode == "small";
+  SweepGroups sg;
+  if (groups && (force || !small_fits)) {
+    std::vector<int> lev;
+    const int nlev = sweep_groups(n, rowp, cols, diag, sg, lev);
+    order_levels(n, lev, nlev, true, pl.lptr, pl.lrows);
+  } else {
+    level_schedule(n, rowp, cols, true, pl.lptr, pl.lrows);
+  }
+  upper.get();
+  pl.lmaxlen.assign(pl.lptr.size() - 1, 0);
+  for (size_t l = 0; l + 1 < pl.lptr.size(); l++)
+    for (int q = pl.lptr[l]; q < pl.lptr[l + 1]; q++)
+      pl.lmaxlen[l] = std::max(
+          pl.lmaxlen[l], rowp[pl.lrows[q] + 1] - rowp[pl.lrows[q]]);
+  const int nlev = (int)std::max(pl.lptr.size(), pl.uptr.size()) - 1;
+  if (small_fits && !force)
+    pl.small = mode == "small" || (!tenv && small_sweeps(n, nlev));
+  if (!groups || pl.small) return GF_OK;
+  if (sg.g.empty()) {
+    std::vector<int> lev;
+    sweep_groups(n, rowp, cols, diag, sg, lev);
+  }
+  auto pays = [&](int glev) { return force || kGroupRatio * glev <= nlev; };
+  if (!pays(sg.nllev)) return GF_OK;
+  std::vector<int> ulev;
+  const int nulev = upper_group_levels(rowp, cols, diag, sg, ulev);
+  if (!pays(nulev)) return GF_OK;
+  group_rows(sg, true, sg.llev, sg.nllev, pl.lgroup, pl.llevel);
+  group_rows(sg, false, ulev, nulev, pl.ugroup, pl.ulevel);
+  if (std::max(pl.llevel.size(), pl.ulevel.size()) > group_records_max(n))
+    for (auto* v : {&pl.lgroup, &pl.ugroup, &pl.llevel, &pl.ulevel})
+      v->clear();
+  return GF_OK;
+}
 }  // namespace gf
 
 extern "C" {
@@ -2360,46 +2505,29 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
                   gf_ilu* out) {
   if (!ctx || n <= 0 || !rowp || !cols || !out)
     return gf::set_error(ctx, GF_ERR_INVALID, "ilu_create: bad args");
-  std::vector<int> diag(n, -1);
-  int maxlen = 0;
-  for (int i = 0; i < n; i++) {
-    maxlen = std::max(maxlen, rowp[i + 1] - rowp[i]);
-    for (int k = rowp[i]; k < rowp[i + 1]; k++) {
-      if (cols[k] < 0 || cols[k] >= n || (k > rowp[i] && cols[k] <= cols[k - 1]))
-        return gf::set_error(ctx, GF_ERR_INVALID,
-                             "ilu_create: row %d not sorted/in range", i);
-      if (cols[k] == i) diag[i] = k;
-    }
-    if (diag[i] < 0)
-      return gf::set_error(ctx, GF_ERR_INVALID,
-                           "ilu_create: row %d has no diagonal block", i);
-  }
-  if (maxlen > gf::kMaxRowBlocks)
-    return gf::set_error(ctx, GF_ERR_INVALID,
-                         "ilu_create: row length %d exceeds %d blocks", maxlen,
-                         gf::kMaxRowBlocks);
+  gf::IluPlan pl;
+  std::string why;
+  const int st = gf::ilu_plan(n, rowp, cols, pl, &why);
+  if (st != GF_OK) return gf::set_error(ctx, st, "%s", why.c_str());
+  return gf::ilu_create_planned(ctx, n, rowp, cols, pl, out);
+}
+
+}  // extern "C"
+
+namespace gf {
+int ilu_create_planned(gf_context ctx, int n, const int* rowp,
+                       const int* cols, IluPlan& pl, gf_ilu* out) {
   auto* h = new gf_ilu_s;
   h->ctx = ctx;
   h->n = n;
   h->nnzb = rowp[n];
-  h->max_row_len = maxlen;
-  std::vector<int> lrows, urows;
-  // the passes over a large pattern run two at a time (400x400 plate, 14 M
-  // blocks: create 62 -> 51 ms); the library runs the second one here if it can
-  // start no thread
-  const auto policy = rowp[n] >= 200000
-                          ? std::launch::async | std::launch::deferred
-                          : std::launch::deferred;
-  auto upper = std::async(policy, [&] {
-    gf::level_schedule(n, rowp, cols, false, h->uptr, urows);
-  });
-  gf::level_schedule(n, rowp, cols, true, h->lptr, lrows);
-  upper.get();
-  h->lmaxlen.assign(h->lptr.size() - 1, 0);
-  for (size_t l = 0; l + 1 < h->lptr.size(); l++)
-    for (int q = h->lptr[l]; q < h->lptr[l + 1]; q++)
-      h->lmaxlen[l] = std::max(h->lmaxlen[l],
-                               rowp[lrows[q] + 1] - rowp[lrows[q]]);
+  h->max_row_len = pl.max_row_len;
+  h->lptr.swap(pl.lptr);
+  h->uptr.swap(pl.uptr);
+  h->lmaxlen.swap(pl.lmaxlen);
+  h->small = pl.small;
+  h->level_sweeps = pl.levels;
+  const std::vector<int>&diag = pl.diag, &lrows = pl.lrows, &urows = pl.urows;
   // chunks: runs of rows of one level, sized so that a level still spreads
   // over the resident wavefronts (one row per chunk for small levels)
   const int target_waves =
@@ -2438,55 +2566,20 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
   // wavefront forwards a chain's rows in registers) serialises the rows of a
   // chain behind each other's memory latency and measured 1.7x slower on the
   // natural-order plates.
-  std::vector<int> lch, uch, lcn, ucn;
-  const char* tenv = getenv("GPUFEM_TRSV");
-  const bool use_chains = tenv && std::string(tenv) == "chains";
-  if (use_chains) {
-    chains(true, lcn);
-    chains(false, ucn);
-  }
-  h->lchains = use_chains;
-  h->uchains = use_chains;
-  h->level_sweeps = tenv && std::string(tenv) == "level";
-  // row groups, by the rule at kGroupRatio
-  std::vector<int> lgr, ugr;
-  int side = 0;  // most blocks of a row on one side of the diagonal
-  for (int i = 0; i < n; i++)
-    side = std::max({side, diag[i] - rowp[i], rowp[i + 1] - diag[i] - 1});
-  const std::string mode = tenv ? tenv : "";
-  if (!tenv)
-    h->small = side <= gf::kSmallBlocks && gf::small_sweeps(
-                   n, (int)std::max(h->lptr.size(), h->uptr.size()) - 1);
-  else if (mode == "small")
-    h->small = side <= gf::kSmallBlocks && n <= gf::kSmallRows;
-  // groups: whatever their ratio.  Any other value: row by row.
-  const bool force = mode == "groups";
-  if (!h->small && (!tenv || force || mode == "small")) {
-    gf::SweepGroups sg;
-    gf::sweep_groups(n, rowp, cols, diag.data(), h->lptr, lrows, sg);
-    auto ur = std::async(policy, [&] {
-      return gf::group_records(rowp, cols, diag.data(), sg, false, ugr,
-                               h->ulevel);
-    });
-    const int gl = gf::group_records(rowp, cols, diag.data(), sg, true, lgr,
-                                     h->llevel);
-    const int gu = ur.get();
-    const size_t most = gf::kGroupInts * gf::group_records_max(n);
-    if (lgr.size() <= most && ugr.size() <= most &&
-        (force || gf::kGroupRatio * std::max(gl, gu) <=
-                      (double)std::max(h->lptr.size(), h->uptr.size()) - 1)) {
-      h->nlgroup = (int)(lgr.size() / gf::kGroupInts);
-      h->nugroup = (int)(ugr.size() / gf::kGroupInts);
-    } else {
-      lgr.clear();
-      ugr.clear();
-    }
-  }
-  if (h->lchains) lch = lcn; else chunks(h->lptr, lch);
-  if (h->uchains) uch = ucn; else chunks(h->uptr, uch);
-  h->nlchunk = (int)lch.size() - 1;
-  h->nuchunk = (int)uch.size() - 1;
-  if (!use_chains && !h->nlgroup) {
+  std::vector<int> lch, uch;
+  const bool use_chains = pl.chains;
+  h->lchains = h->uchains = use_chains;
+  h->nlgroup = (int)pl.llevel.size();
+  h->nugroup = (int)pl.ulevel.size();
+  if (h->nlgroup) {
+    h->llevel.swap(pl.llevel);
+    h->ulevel.swap(pl.ulevel);
+  } else if (use_chains) {
+    chains(true, lch);
+    chains(false, uch);
+  } else {
+    chunks(h->lptr, lch);
+    chunks(h->uptr, uch);
     auto levels_of = [](const std::vector<int>& ch, const std::vector<int>& lp,
                         std::vector<int>& out) {
       out.resize(ch.size() - 1);
@@ -2501,21 +2594,27 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
   }
   // row descriptors in hand-out order, one 16-byte load per row: {row, first
   // block, end block, level}; the diagonal block is the end (L) or one before the
-  // first (U)
-  std::vector<int4> lm(n), um(n);
-  for (int p = 0; p < n; p++) {
-    const int li = use_chains ? p : lrows[p];
-    lm[p] = make_int4(li, rowp[li], diag[li], 0);
-    const int ui = use_chains ? n - 1 - p : urows[p];
-    um[p] = make_int4(ui, diag[ui] + 1, rowp[ui + 1], 0);
-  }
-  auto levels_into = [](const std::vector<int>& lp, std::vector<int4>& mt) {
-    for (size_t l = 0; l + 1 < lp.size(); l++)
-      for (int p = lp[l]; p < lp[l + 1]; p++) mt[p].w = (int)l;
-  };
-  if (!use_chains) {
-    levels_into(h->lptr, lm);
-    levels_into(h->uptr, um);
+  // first (U).  Row groups need neither these nor the chunks.
+  std::vector<int4> lm, um;
+  if (!h->nlgroup) {
+    h->nlchunk = (int)lch.size() - 1;
+    h->nuchunk = (int)uch.size() - 1;
+    lm.resize(n);
+    um.resize(n);
+    for (int p = 0; p < n; p++) {
+      const int li = use_chains ? p : lrows[p];
+      lm[p] = make_int4(li, rowp[li], diag[li], 0);
+      const int ui = use_chains ? n - 1 - p : urows[p];
+      um[p] = make_int4(ui, diag[ui] + 1, rowp[ui + 1], 0);
+    }
+    auto levels_into = [](const std::vector<int>& lp, std::vector<int4>& mt) {
+      for (size_t l = 0; l + 1 < lp.size(); l++)
+        for (int p = lp[l]; p < lp[l + 1]; p++) mt[p].w = (int)l;
+    };
+    if (!use_chains) {
+      levels_into(h->lptr, lm);
+      levels_into(h->uptr, um);
+    }
   }
   auto up = [&](int** dst, const int* src, size_t cnt) -> int {
     GF_TRY(gf::dmalloc(ctx, (void**)dst, sizeof(int) * (cnt ? cnt : 1)));
@@ -2524,16 +2623,20 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
     return GF_OK;
   };
   int st = GF_OK;
-  if ((st = up(&h->lgroup, lgr.data(), lgr.size())) ||
-      (st = up(&h->ugroup, ugr.data(), ugr.size())) ||
+  if ((st = up(&h->lgrows, pl.lgroup.data(), pl.lgroup.size())) ||
+      (st = up(&h->ugrows, pl.ugroup.data(), pl.ugroup.size())) ||
       (st = up(&h->rowp, rowp, n + 1)) || (st = up(&h->cols, cols, rowp[n])) ||
       (st = up(&h->diag, diag.data(), n)) ||
       (st = up(&h->lrows, lrows.data(), n)) ||
       (st = up(&h->urows, urows.data(), n)) ||
       (st = up(&h->lchunk, lch.data(), lch.size())) ||
-      (st = up((int**)&h->lmeta, (const int*)lm.data(), 4 * (size_t)n)) ||
-      (st = up((int**)&h->umeta, (const int*)um.data(), 4 * (size_t)n)) ||
+      (st = up((int**)&h->lmeta, (const int*)lm.data(), 4 * lm.size())) ||
+      (st = up((int**)&h->umeta, (const int*)um.data(), 4 * um.size())) ||
       (st = up(&h->uchunk, uch.data(), uch.size())) ||
+      (st = gf::dmalloc(ctx, (void**)&h->lgroup,
+                        sizeof(int) * kGroupInts * (size_t)h->nlgroup)) ||
+      (st = gf::dmalloc(ctx, (void**)&h->ugroup,
+                        sizeof(int) * kGroupInts * (size_t)h->nugroup)) ||
       (st = gf::dmalloc(ctx, (void**)&h->pivot, sizeof(int))) ||
       (st = gf::dmalloc(ctx, (void**)&h->counter, gf::ilu_counter_bytes())) ||
       (st = gf::dmalloc(ctx, (void**)&h->err, 2 * sizeof(int))) ||
@@ -2546,6 +2649,19 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
                           "memset"))) {
     gf_ilu_destroy(h);
     return st;
+  }
+  if (h->nlgroup) {
+    auto records = [&](bool lower, int nrec, const int* rows, int* out) {
+      hipLaunchKernelGGL(group_records_kernel, dim3(div_up(nrec, 4)), dim3(256),
+                         0, ctx->stream, nrec, lower, rows, h->rowp, h->cols,
+                         h->diag, out);
+    };
+    records(true, h->nlgroup, h->lgrows, h->lgroup);
+    records(false, h->nugroup, h->ugrows, h->ugroup);
+    if ((st = check_launch(ctx, "group_records_kernel"))) {
+      gf_ilu_destroy(h);
+      return st;
+    }
   }
   {
     // enough wavefronts to cover the device, capped by the chunks and by
@@ -2576,6 +2692,9 @@ int gf_ilu_create(gf_context ctx, int n, const int* rowp, const int* cols,
   *out = h;
   return GF_OK;
 }
+}  // namespace gf
+
+extern "C" {
 
 int gf_ilu_destroy(gf_ilu h) {
   if (!h) return GF_OK;
@@ -2590,6 +2709,8 @@ int gf_ilu_destroy(gf_ilu h) {
   gf::dfree(h->ctx, h->umeta);
   gf::dfree(h->ctx, h->lgroup);
   gf::dfree(h->ctx, h->ugroup);
+  gf::dfree(h->ctx, h->lgrows);
+  gf::dfree(h->ctx, h->ugrows);
   gf::dfree(h->ctx, h->uchunk);
   gf::dfree(h->ctx, h->counter);
   gf::dfree(h->ctx, h->err);

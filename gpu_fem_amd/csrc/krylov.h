@@ -98,6 +98,22 @@ struct SweepSlot {
   const int* go;  // batched launches sweep the system only while *go == 1
   int n, nllev, nulev;  // rows and levels of a small system (nllev > 0)
 };
+// Host analysis of an ILU pattern: rows by level of the two sweeps, and how
+// the sweeps run.
+struct IluPlan {
+  int max_row_len = 0;
+  std::vector<int> diag, lptr, lrows, uptr, urows;
+  std::vector<int> lmaxlen;         // longest row of each L level
+  std::vector<int> lgroup, ugroup;  // rows of the group records (empty: none)
+  std::vector<int> llevel, ulevel;  // and the records' levels
+  bool small = false, chains = false, levels = false;
+};
+// GF_ERR_INVALID, with the reason, for a pattern that gf_ilu_create refuses
+int ilu_plan(int n, const int* rowp, const int* cols, IluPlan& pl,
+             std::string* why);
+// uploads a plan (and takes its vectors)
+int ilu_create_planned(gf_context ctx, int n, const int* rowp,
+                       const int* cols, IluPlan& pl, gf_ilu* out);
 // The device schedule of an ILU analysis (row groups where it has them, else
 // chunks) and the dependency level of each item.
 struct IluView {

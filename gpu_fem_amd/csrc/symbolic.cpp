@@ -257,6 +257,21 @@ int bandwidth(int n, const int* rowp, const int* cols) {
   return bw;
 }
 
+void order_levels(int n, const std::vector<int>& lev, int nlev, bool lower,
+                  std::vector<int>& level_ptr, std::vector<int>& level_rows) {
+  level_ptr.assign(nlev + 1, 0);
+  for (int i = 0; i < n; i++) level_ptr[lev[i] + 1]++;
+  for (int l = 0; l < nlev; l++) level_ptr[l + 1] += level_ptr[l];
+  level_rows.resize(n);
+  std::vector<int> pos(level_ptr.begin(), level_ptr.end() - 1);
+  // rows inside a level keep ascending (lower) / descending (upper) order
+  if (lower) {
+    for (int i = 0; i < n; i++) level_rows[pos[lev[i]]++] = i;
+  } else {
+    for (int i = n - 1; i >= 0; i--) level_rows[pos[lev[i]]++] = i;
+  }
+}
+
 void level_schedule(int n, const int* rowp, const int* cols, bool lower,
                     std::vector<int>& level_ptr, std::vector<int>& level_rows) {
   std::vector<int> lev(n, 0);
@@ -278,17 +293,7 @@ void level_schedule(int n, const int* rowp, const int* cols, bool lower,
       nlev = std::max(nlev, l + 1);
     }
   }
-  level_ptr.assign(nlev + 1, 0);
-  for (int i = 0; i < n; i++) level_ptr[lev[i] + 1]++;
-  for (int l = 0; l < nlev; l++) level_ptr[l + 1] += level_ptr[l];
-  level_rows.resize(n);
-  std::vector<int> pos(level_ptr.begin(), level_ptr.end() - 1);
-  // rows inside a level keep ascending (lower) / descending (upper) order
-  if (lower) {
-    for (int i = 0; i < n; i++) level_rows[pos[lev[i]]++] = i;
-  } else {
-    for (int i = n - 1; i >= 0; i--) level_rows[pos[lev[i]]++] = i;
-  }
+  order_levels(n, lev, nlev, lower, level_ptr, level_rows);
 }
 
 void element_coloring(int nelems, int nnodes, int npe, const int* conn,

@@ -31,6 +31,9 @@ int transpose_map(int n, const int* rowp, const int* cols,
                   std::vector<int>& trowp, std::vector<int>& tcols,
                   std::vector<int>& tmap);
 int bandwidth(int n, const int* rowp, const int* cols);
+// rows ordered by the given levels 0 .. nlev - 1
+void order_levels(int n, const std::vector<int>& lev, int nlev, bool lower,
+                  std::vector<int>& level_ptr, std::vector<int>& level_rows);
 // rows grouped by dependency level for the lower (L) or upper (U) sweep
 void level_schedule(int n, const int* rowp, const int* cols, bool lower,
                     std::vector<int>& level_ptr, std::vector<int>& level_rows);

@@ -64,3 +64,19 @@ def test_chosen_kind(gpu_ctx, kind, n, mode, dtype, monkeypatch):
 def test_kind_by_the_pattern(gpu_ctx, kind, n, want):
     print(f"[gpu] sweep kind by the pattern {kind} n={n}", flush=True)
     check(gpu_ctx, *make(kind, n), np.float64, want)
+
+
+@pytest.mark.parametrize("rowp,cols", [
+    ([0, 2, 4], [1, 0, 0, 1]),       # not sorted
+    ([0, 2, 4], [0, 0, 0, 1]),       # a column twice
+    ([0, 2, 4], [0, 2, 0, 1]),       # out of range
+    ([0, 2, 4], [-1, 0, 0, 1]),
+    ([0, 1, 3], [1, 0, 1]),          # no diagonal block
+    ([0, 0, 1], [1]),                # an empty row
+    ([0, 1, 1], [0]),
+])
+def test_refused_patterns(gpu_ctx, rowp, cols):
+    print(f"[gpu] refused pattern {rowp} {cols}", flush=True)
+    with pytest.raises(G.GfError) as e:
+        G.Ilu(gpu_ctx, np.array(rowp, np.int32), np.array(cols, np.int32))
+    assert e.value.code == -1 and "ilu_create: row" in str(e.value)
