@@ -133,7 +133,8 @@ int problem_setup(gf_problem p, gf::ProblemPlan& pl, const int* conn,
   GF_TRY(upload(ctx, &p->trowp, pl.tr.data(), pl.tr.size()));
   GF_TRY(upload(ctx, &p->tcols, pl.tc.data(), pl.tc.size()));
   GF_TRY(upload(ctx, &p->tmap, pl.tm.data(), pl.tm.size()));
-  GF_TRY(gf_ilu_create(ctx, n, pl.mrp.data(), pl.mcl.data(), &p->ilu));
+  GF_TRY(gf::ilu_create_planned(ctx, n, pl.mrp.data(), pl.mcl.data(), pl.ilu,
+                                &p->ilu));
   const size_t N = 6 * (size_t)n;
   GF_TRY(dalloc(ctx, &p->kvals, 36 * (size_t)p->nnzb_k));
   GF_TRY(dalloc(ctx, &p->mvals, 36 * (size_t)p->nnzb_m));
@@ -198,6 +199,7 @@ int problem_plan(int n, int ne, const int* conn, int nbcs, const int* bcs,
                          pl.kcl));
   GF_TRY(iluk_symbolic(n, pl.krp.data(), pl.kcl.data(), opt.lev_fill, pl.mrp,
                        pl.mcl, nullptr));
+  GF_TRY(ilu_plan(n, pl.mrp.data(), pl.mcl.data(), pl.ilu, why));
   pl.emap.resize((size_t)16 * ne);
   GF_TRY(elem_ind_map(ne, 4, conn, pl.krp.data(), pl.kcl.data(),
                       pl.perm.data(), pl.emap.data()));
@@ -223,13 +225,19 @@ size_t ProblemPlan::device_bytes(bool caching) const {
   add(n * I); add(n * I); add((n + 1) * I); add(nk * I); add(16 * ne * I);
   add(ne * I); add(ne * I);
   add((n + 1) * I); add(nk * I); add(nk * I);
-  // ILU analysis: pattern, diagonal, level orders, chunk offsets (at most
-  // one chunk per row), row descriptors, pivot, counter, flags, done
+  // ILU analysis: pattern, diagonal, level orders, pivot, counter, flags, done
   add((n + 1) * I); add(nm * I); add(n * I); add(n * I); add(n * I);
-  add((n + 1) * I); add(4 * n * I); add(4 * n * I); add((n + 1) * I);
   add(I); add(ilu_counter_bytes()); add(2 * I); add(n * I);
-  // row groups of the two sweeps (at most)
-  add(ilu_group_bytes(n)); add(ilu_group_bytes(n));
+  if (ilu.llevel.empty()) {
+    // chunk offsets (at most one chunk per row), row descriptors
+    add((n + 1) * I); add(4 * n * I); add(4 * n * I); add((n + 1) * I);
+  } else {
+    // row groups of the two sweeps: rows and records
+    for (const auto* lev : {&ilu.llevel, &ilu.ulevel}) {
+      add(ilu_group_row_bytes(lev->size()));
+      add(ilu_group_bytes(lev->size()));
+    }
+  }
   // values and vectors
   add(36 * nk * D); add(36 * nm * D);
   for (int i = 0; i < 5; i++) add(N * D);

@@ -1823,8 +1823,8 @@ constexpr int kGroupNear = 16;  // blocks next to the diagonal, last pass
 // 2.44 ms, AMD ILU(0) (0.2) 0.41 / 0.60 ms, AMD ILU(3) (5.6) 0.75 / 0.58 ms,
 // RCM ILU(3) (5.0) 5.9 / 2.3 ms; RCM ILU(3) of a wingbox (1.6) 7.1 / 6.0 ms.
 constexpr double kGroupRatio = 1.5;
-// records of a sweep at most (a pattern that would need more is swept row by
-// row), for the accounting of device memory
+// records of a sweep at most, a bound of their memory (416 bytes each with its
+// rows): a pattern that would need more is swept row by row
 inline size_t group_records_max(size_t n) { return n / 4 + 64; }
 // kBatched: the groups of several systems, merged[q] = {system, group}; the
 // arrays of a system are in its slot.
@@ -2412,9 +2412,10 @@ size_t ilu_counter_bytes() {
   return sizeof(unsigned long long) * kCounterStride *
          (1 + kSweepThreads / 64);
 }
-size_t ilu_group_bytes(size_t n) {
-  return sizeof(int) * kGroupInts * group_records_max(n);
+size_t ilu_group_row_bytes(size_t nrec) {
+  return sizeof(int) * kGroupRows * nrec;
 }
+size_t ilu_group_bytes(size_t nrec) { return sizeof(int) * kGroupInts * nrec; }
 // Host analysis of a pattern: its levels, and how the sweeps run.
 int ilu_plan(int n, const int* rowp, const int* cols, IluPlan& pl,
              std::string* why) {
@@ -2616,8 +2617,10 @@ int ilu_create_planned(gf_context ctx, int n, const int* rowp,
       levels_into(h->uptr, um);
     }
   }
+  // (ProblemPlan::device_bytes mirrors the list; what is empty stays null)
   auto up = [&](int** dst, const int* src, size_t cnt) -> int {
-    GF_TRY(gf::dmalloc(ctx, (void**)dst, sizeof(int) * (cnt ? cnt : 1)));
+    if (!cnt) return GF_OK;
+    GF_TRY(gf::dmalloc(ctx, (void**)dst, sizeof(int) * cnt));
     GF_HIP(ctx, hipMemcpyAsync(*dst, src, sizeof(int) * cnt,
                                hipMemcpyHostToDevice, ctx->stream));
     return GF_OK;
@@ -2633,10 +2636,11 @@ int ilu_create_planned(gf_context ctx, int n, const int* rowp,
       (st = up((int**)&h->lmeta, (const int*)lm.data(), 4 * lm.size())) ||
       (st = up((int**)&h->umeta, (const int*)um.data(), 4 * um.size())) ||
       (st = up(&h->uchunk, uch.data(), uch.size())) ||
-      (st = gf::dmalloc(ctx, (void**)&h->lgroup,
-                        sizeof(int) * kGroupInts * (size_t)h->nlgroup)) ||
-      (st = gf::dmalloc(ctx, (void**)&h->ugroup,
-                        sizeof(int) * kGroupInts * (size_t)h->nugroup)) ||
+      (h->nlgroup &&
+       ((st = gf::dmalloc(ctx, (void**)&h->lgroup,
+                          ilu_group_bytes(h->nlgroup))) ||
+        (st = gf::dmalloc(ctx, (void**)&h->ugroup,
+                          ilu_group_bytes(h->nugroup))))) ||
       (st = gf::dmalloc(ctx, (void**)&h->pivot, sizeof(int))) ||
       (st = gf::dmalloc(ctx, (void**)&h->counter, gf::ilu_counter_bytes())) ||
       (st = gf::dmalloc(ctx, (void**)&h->err, 2 * sizeof(int))) ||

@@ -140,10 +140,11 @@ struct SweepItems {
 // tickets counters of a batched sweep pair (device, unsigned long long each)
 constexpr int kBatchCounters = 4;
 int ilu_view(gf_ilu h, IluView* v);
-// device memory of an analysis: ticket counters; row groups of one sweep (at
-// most) of a pattern of n rows
+// device memory of an analysis: ticket counters; rows and records of a sweep
+// with so many group records
 size_t ilu_counter_bytes();
-size_t ilu_group_bytes(size_t n);
+size_t ilu_group_row_bytes(size_t nrec);
+size_t ilu_group_bytes(size_t nrec);
 template <typename T>
 int launch_batch_sweeps(hipStream_t s, const SweepSlot<T>* slots,
                         const SweepItems& items, int grid, int ggrid,

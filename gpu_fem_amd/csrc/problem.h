@@ -41,6 +41,7 @@ struct ProblemPlan {
   std::vector<int> perm, iperm;     // perm[old] = new
   std::vector<int> krp, kcl;        // permuted K pattern
   std::vector<int> mrp, mcl;        // ILU(k) pattern
+  IluPlan ilu;                      // and its analysis
   std::vector<int> emap;            // elemIndMap, 16 per element
   std::vector<int> tr, tc, tm;      // transpose pattern and block map
   // bytes of device memory gf_problem_create allocates for this plan
