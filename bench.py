@@ -240,10 +240,13 @@ def live_pmc_traffic(args):
         units = max(1, len(f) // launches_per_unit)
         return (sum(f) * 1024 * ff + sum(w) * 1024 * wf) / units
 
-    # rows in groups, or row by row where the pattern has no chains
+    # rows in groups, row by row, or both sweeps of a small system in one
+    # launch (half of it each, then)
     def sweep_of(lower):
+        small = bytes_of("trsv_small_kernel<double")
         return (bytes_of(f"trsv_group_kernel<double, {lower}")
-                or bytes_of(f"trsv_syncfree_kernel<double, {lower}"))
+                or bytes_of(f"trsv_syncfree_kernel<double, {lower}")
+                or (small and small / 2))
 
     lo, up = sweep_of("true"), sweep_of("false")
     nasm = len(vals("jacobian_mfma_kernel<true>", "FETCH_SIZE"))
@@ -477,6 +480,9 @@ def main():
     sweep_bytes_launch = (lb + ub) / 2
     sweep_gbs = sweep_bytes_launch / sweep_launch_s / 1e9
     info_lv = ilu.info()
+    sweep_kernel = {"groups": "trsv_group_kernel", "small": "trsv_small_kernel",
+                    "levels": "trsv_level_kernel"}.get(
+                        ilu.sweep_info()["kind"], "trsv_syncfree_kernel")
     # the FP32 sweeps of the mixed paths, on the FP64 factors rounded to FP32
     # (a sweep's traffic and dependency latency do not depend on the values)
     mv32, b32 = mv.float(), b.float()
@@ -594,7 +600,7 @@ def main():
         "paths": {k: {kk: vv for kk, vv in v.items() if kk != "x_host"}
                   for k, v in results.items()},
         "roofline": {"bound": "hbm",
-                     "kernel": "trsv_group_kernel<double> (L and U)",
+                     "kernel": f"{sweep_kernel}<double> (L and U)",
                      "achieved": sweep_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": sweep_gbs / HBM_PEAK_GBS,
                      "traffic": (pmc["sweep_bytes_per_launch"] if pmc
@@ -610,7 +616,7 @@ def main():
         "residual_floor": floor,
         # the dominant kernel of the mixed paths (FP32 factors and vectors)
         "roofline_fp32_sweep": {
-            "bound": "hbm", "kernel": "trsv_group_kernel<float> (L and U)",
+            "bound": "hbm", "kernel": f"{sweep_kernel}<float> (L and U)",
             "achieved": sweep32_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": sweep32_gbs / HBM_PEAK_GBS,
             "bytes_per_launch": sweep32_bytes_launch,
