@@ -514,11 +514,14 @@ __global__ void __launch_bounds__(kIluThreads)
 // Dynamic LDS per position of row i: its column index, its place in the list
 // of the run's blocks, and per pivot of the window the index (+ 1) of the
 // position in the pivot's U part (0: not updated).
-// What bounds it: the rows' own time more than the chain of pivots.  400x400
-// plate, AMD + ILU(96), FP32: 9,266 such rows of 370 to 1,750 blocks take 2.5
-// ms each on 512 places; a run of 7.7 pivots took 42 us with the window of
-// one run, 9 of them preparing the next one after it, 6 forming L_ik, 5
-// loading the pivots' edges, 12 the update, 9 waiting.
+// What bounds it: memory.  400x400 plate, AMD + ILU(96), FP64: 352 GB read and
+// written (PMC) in 60.6 ms, 5.8 TB/s, more than a copy reaches (4.95): a block
+// update reads its U_kj from outside the L2, and rows share nothing.  FP32
+// moves 160 GB in 41.4 ms, 3.9 TB/s, and its rows' own time counts as well:
+// 9,266 rows of 370 to 1,750 blocks, 2.5 ms each on 512 places; a run of 7.7
+// pivots took 42 us with the window of one run, 9 of them preparing the next
+// one after it, 6 forming L_ik, 5 loading the pivots' edges, 12 the update, 9
+// waiting.
 #ifndef GPUFEM_ILU_BATCH
 #define GPUFEM_ILU_BATCH 8
 #endif
@@ -1991,8 +1994,8 @@ __global__ void __launch_bounds__(kGroupThreads, 4)
       T acc = T(0);
       const int nb = k1 - k0;
       // passes as in trsv_syncfree_kernel: the blocks next to the diagonal
-      // last (part 0), the others in passes of kPass dealt out over the parts,
-      // U rows taking theirs last to first
+      // last, the others in passes of kPass, all dealt out over the parts, U
+      // rows taking theirs last to first
       const bool split = nb > kPass;
       const int nfar = split ? nb - kGroupNear : nb;
       const int nfp = (nfar + kPass - 1) / kPass;

@@ -24,7 +24,7 @@ namespace {
 constexpr int kDotBlocks = 256;  // slices of the index range, at most
 constexpr int kDotThreads = 256;
 constexpr int kDotChunk = 8;
-// Slices of N entries: a thread has at least one entry.  (256 slices of 726
+// Slices of N entries: at most one for 256 entries.  (256 slices of 726
 // entries kept three threads of 256 busy: 16.6 us a product of a 10x10
 // plate's basis, 7.2 us so.)
 __host__ __device__ inline int dot_slices(size_t N) {
@@ -675,8 +675,12 @@ constexpr bool kDcgs2 = GPUFEM_GMRES_DCGS2;
 // each restart cycle runs until its residual estimate falls below this
 // fraction of rtol ||b|| (see the comment at its use)
 constexpr double kCycleTarget = GPUFEM_GMRES_CYCLE_TARGET;
-// sweep depth (L + U dependency levels) below which Arnoldi steps are issued
-// one ahead of the convergence test (see gmres_solve)
+// sweep depth (L + U dependency levels of rows, whatever the sweeps' items)
+// below which Arnoldi steps are issued one ahead of the convergence test (see
+// gmres_solve).  Deeper patterns, also those swept in a few dozen group
+// levels, are faster without: solve of a plate, FP64, without / with: 21x21
+// AMD ILU(3) (14 steps) 1.82 / 1.87 ms, 46x46 ILU(64) (1 step) 0.69 / 0.91,
+// 65x65 ILU(12) (20 steps) 5.12 / 5.40, 102x102 ILU(64) (4 steps) 2.31 / 3.29.
 constexpr int kLookaheadLevels = 128;
 // an estimate is formed ahead of step j when the rate so far predicts it at
 // or below this multiple of the cycle's target
@@ -696,9 +700,9 @@ int gmres_solve(KrylovWork& W, const Operator& op, const double* b, double* x,
   // Look-ahead: Arnoldi step j+1 is issued before the host reads step j's
   // residual estimate, hiding the host round trip (tens of microseconds)
   // between steps; a step issued past the stopping point is a wasted
-  // preconditioner application.  With deep sweeps (a step of milliseconds)
-  // the waste costs more than the round trips, so look-ahead is used only
-  // for shallow sweeps (GPUFEM_GMRES_LOOKAHEAD=0/1 overrides).
+  // preconditioner application.  With deep sweeps the waste costs more than
+  // the round trips, so look-ahead is used only for shallow sweeps
+  // (GPUFEM_GMRES_LOOKAHEAD=0/1 overrides).
   bool ahead = true;
   {
     int nl = 0, nu = 0;
