@@ -1807,8 +1807,8 @@ __device__ __forceinline__ bool finite(float v) {
 // its being seen, 0.5 us for the pass, 0.4 us to the solver, 0.7-1 us the
 // chain), and in the wide levels the 5-9 us latency of a record at two
 // workgroups a CU.  L+U pair, row by row -> groups: 400x400 plate AMD +
-// ILU(96) (1,372 row levels, 181 group levels) FP64 5.15 -> 2.15 ms, FP32
-// 4.88 -> 1.95 ms; 101x101 ILU(64) FP64 1.77 -> 0.50 ms; 45x45 ILU(64)
+// ILU(96) (1,372 row levels, 181 group levels) FP64 5.15 -> 2.17 ms, FP32
+// 4.88 -> 1.96 ms; 101x101 ILU(64) FP64 1.77 -> 0.50 ms; 45x45 ILU(64)
 // 0.79 -> 0.23 ms; complete LU of a 24,390-node wingbox (3,876 -> 489
 // levels) 10.5 -> 2.65 ms.
 //
